@@ -418,12 +418,16 @@ int mcint_schwarz(mcint_basis *b, int nshell, double *q);
  * component-chunk kernels: 0 never, 1 where measured faster (the tuned
  * table, mcint_tune_class_wave), 2 in every bucket of every class that has
  * one; read at launch.
+ * MCINT_TUNE_FILL_LANES: a class of a plan whose teams put fewer lanes than
+ * this to work has them widened (up to one wave per quartet); 0 keeps the
+ * tuned primitive quartets per lane, as for tuning them.
  * Applies to plans created afterwards; returns the previous value, or a
  * negative status. */
 #define MCINT_TUNE_PRIMS_PER_LANE 0
 #define MCINT_TUNE_GENERIC_ONLY 1
 #define MCINT_TUNE_GRAPH_BRANCHES 2
 #define MCINT_TUNE_WAVE_KERNELS 3
+#define MCINT_TUNE_FILL_LANES 4
 int mcint_tune(int key, int value);
 /* Per-class override of MCINT_TUNE_PRIMS_PER_LANE for one integral kind
  * (intor code) and canonical class (la >= lb, lc >= ld, (la,lb) >= (lc,ld)

@@ -160,6 +160,7 @@ TUNE_PRIMS_PER_LANE = 0
 TUNE_GENERIC_ONLY = 1
 TUNE_GRAPH_BRANCHES = 2
 TUNE_WAVE_KERNELS = 3
+TUNE_FILL_LANES = 4
 
 
 def tune(key: int, value: int) -> int:

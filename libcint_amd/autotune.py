@@ -34,7 +34,7 @@ import sys
 
 import numpy as np
 
-from . import (INTOR_CODES, TUNE_PRIMS_PER_LANE, TUNE_WAVE_KERNELS, DeviceBasis, Plan, tune,
+from . import (INTOR_CODES, TUNE_FILL_LANES, TUNE_PRIMS_PER_LANE, TUNE_WAVE_KERNELS, DeviceBasis, Plan, tune,
                tune_class, tune_class_wave, wave_kernel_exists)
 
 CANDIDATES = (8, 16, 32, 64, 128)
@@ -195,6 +195,7 @@ def main(argv):
     out_path = args[0] if args else DEFAULT_TABLE
     tables = load() if wave_only else {}
     tune(TUNE_WAVE_KERNELS, 1)
+    tune(TUNE_FILL_LANES, 0)  # the measured teams, not widened ones
     for name, db, q in _workloads():
         if name == "int2e_sph":
             if not wave_only:

@@ -401,7 +401,8 @@ void for_each_task(const std::vector<int>& vfirst, int dummy, int kind, const Qu
   }
 }
 
-// Set of bucket keys (open addressing; keys are < 2^27, ~0u marks empty).
+// Set of bucket keys (open addressing; ~0u marks empty and is no key: its
+// path field would be 3).
 struct KeySet {
   std::vector<uint32_t> slot = std::vector<uint32_t>(1024, ~0u);
   size_t n = 0;
@@ -455,6 +456,7 @@ struct KeyIndex {
 
 struct Bucket {
   int la, lb, lc, ld, team;
+  int tune_team;  // team size by the tuned primitive quartets per lane (team: widened to fill the chip)
   int mode;  // 0 generic, 1 fast (single chunk), 2 chunked
   int fp32;  // recurrences in FP32 (mode 1 only)
   int64_t t0, t1;
@@ -491,6 +493,9 @@ constexpr int64_t GEN_SCRATCH_DOUBLES = 512ll << 20;
 // copies of the gradient accumulators (spreads the digest's atomics)
 constexpr int GRAD_SLOTS = 64;
 
+// default of g_fill_lanes: 256 CUs x 4 SIMDs x 2 waves
+constexpr int FILL_LANES = 1 << 17;
+
 // Tuning state (mcint_tune): primitive quartets per lane that the team
 // size aims at.
 int g_prims_per_lane = 32;
@@ -503,10 +508,98 @@ constexpr int MAX_GRAPH_BRANCHES = 8;
 // integral kind and canonical class
 int16_t g_class_ppl[NKIND][NCLS] = {};
 
+// Lanes a class should put to work before a team takes the tuned number of
+// primitive quartets per lane (mcint_tune MCINT_TUNE_FILL_LANES).  The tuned
+// values come from lists that fill the chip; a class of a small molecule
+// fills a few of its 256 CUs, and its time is the chain of 32-128 primitive
+// quartets of one lane.  Two waves per SIMD of the whole chip: int2e of 28
+// shells 1.09 ms unwidened, 0.65 / 0.52 / 0.51 ms at 1/2, 1 and 2 of it; of
+// 84 shells 15.3 -> 13.8 ms; J/K of 98 shells 29.6 / 30.0 / 31.0 ms (wider
+// teams only cost there, hence no more than this).
+int g_fill_lanes = FILL_LANES;
+// Primitive quartets per lane below which teams are not widened further:
+// every lane of a team repeats the epilogue, so that short chains gain
+// nothing.  Measured at 4 / 8 / 16 / 32: int2e of 28 shells 0.55 / 0.52 /
+// 0.58 / 0.75 ms, of 84 shells 14.1 / 13.8 / 13.9 / 14.9 ms; three-centre
+// lists (whose quartets hold few primitives) of 0.9 M / 444 shells 2.5 / 2.5
+// / 2.1 / 2.1 ms, 2.3 ms without widening.
+constexpr int fill_ppl_min(int kind) { return kind_three(kind) ? 16 : 8; }
+
 int pick_team(int64_t nprim_quartets, int ppl) {
   int t = 1;
   while (t < fast_team_lanes_max() && (int64_t)t * ppl < nprim_quartets) t *= 2;
   return t;
+}
+
+// Team of a quartet of 2^lp primitive quartets widened by up to f: at most
+// one wave, and no fewer than fill_ppl_min primitive quartets per lane.
+int widen_team(int kind, int team, int64_t f, int lp) {
+  int t = team;
+  while (t < fast_team_lanes_max() && (int64_t)t * 2 <= (int64_t)team * f &&
+         (int64_t)t * 2 * fill_ppl_min(kind) <= ((int64_t)1 << lp))
+    t *= 2;
+  return t;
+}
+
+// The buckets' keys of a plan from its raw keys (class, log2 of the
+// primitive quartets, team by the tuned primitive quartets per lane, path,
+// precision) and their task counts; bucket_of[i]: the bucket of raw key i.
+// A class that puts fewer than g_fill_lanes lanes to work has its teams
+// widened, and keeps one bucket per team size and kernel: what bounds it is
+// the length of a lane's chain of primitive quartets and the number of its
+// launches.  The final key holds the tuned team size (which selects the
+// tuned kernel of a chunked class) where the raw key holds the primitives.
+std::vector<uint32_t> bucket_keys(const std::vector<uint32_t>& raw,
+                                  const std::vector<int64_t>& tasks, int kind, double omega,
+                                  std::vector<uint32_t>& bucket_of) {
+  constexpr uint32_t GROUP = ~((15u << 12) | (15u << 20));  // class, path, precision
+  const size_t n = raw.size();
+  std::vector<uint32_t> fin(n);
+  std::vector<uint32_t> groups(n);
+  for (size_t i = 0; i < n; ++i) groups[i] = raw[i] & GROUP;
+  std::sort(groups.begin(), groups.end());
+  groups.erase(std::unique(groups.begin(), groups.end()), groups.end());
+  std::vector<int64_t> lanes(groups.size(), 0);
+  auto group = [&](uint32_t k) {
+    return (size_t)(std::lower_bound(groups.begin(), groups.end(), k & GROUP) - groups.begin());
+  };
+  auto wave = [&](uint32_t k, int tl) {
+    return kind == KIND_2E && ((k >> 24) & 3) == 2 &&
+           chunk_class_on_wave(k & 7, (k >> 3) & 7, (k >> 6) & 7, (k >> 9) & 7, 1 << tl, omega,
+                               (k >> 26) & 1);
+  };
+  // smallest tuned team of each group on the chunk kernels / the wave kernel
+  std::vector<int> low(2 * groups.size(), 15);
+  for (size_t i = 0; i < n; ++i) {
+    const size_t g = group(raw[i]);
+    const int tl = (raw[i] >> 20) & 15;
+    lanes[g] += tasks[i] << tl;
+    int& l = low[2 * g + wave(raw[i], tl)];
+    l = std::min(l, tl);
+  }
+  for (size_t i = 0; i < n; ++i) {
+    const size_t g = group(raw[i]);
+    int tl = (raw[i] >> 20) & 15, tune = tl;
+    if (((raw[i] >> 24) & 3) != 0 && lanes[g] < g_fill_lanes) {
+      const bool w = wave(raw[i], tl);
+      tune = low[2 * g + w];
+      if (w) {
+        tl = tune;
+      } else {
+        const int t = widen_team(kind, 1 << tl, g_fill_lanes / std::max<int64_t>(1, lanes[g]),
+                                 (raw[i] >> 12) & 15);
+        while ((1 << tl) < t) ++tl;
+      }
+    }
+    fin[i] = (raw[i] & GROUP) | ((uint32_t)tune << 12) | ((uint32_t)tl << 20);
+  }
+  std::vector<uint32_t> keys = fin;
+  std::sort(keys.begin(), keys.end());
+  keys.erase(std::unique(keys.begin(), keys.end()), keys.end());
+  bucket_of.resize(n);
+  for (size_t i = 0; i < n; ++i)
+    bucket_of[i] = (uint32_t)(std::lower_bound(keys.begin(), keys.end(), fin[i]) - keys.begin());
+  return keys;
 }
 
 }  // namespace
@@ -644,6 +737,15 @@ extern "C" int mcint_tune(int key, int value) {
     g_generic_only = value;
     return old;
   }
+  if (key == MCINT_TUNE_FILL_LANES) {
+    if (value < 0) {
+      set_err("mcint_tune: lanes to fill must not be negative");
+      return MCINT_ERR_ARG;
+    }
+    const int old = g_fill_lanes;
+    g_fill_lanes = value;
+    return old;
+  }
   set_err("mcint_tune: unknown key");
   return MCINT_ERR_ARG;
 }
@@ -741,9 +843,11 @@ static int plan_create_impl(mcint_plan** out, mcint_basis* b, int intor, const F
                                 : 0u;
       int tl = 0;
       while ((1 << tl) < team) ++tl;
+      uint32_t lp = 0;  // log2 of the primitive quartets, rounded up
+      while (lp < 15 && ((int64_t)1 << lp) < nprimq) ++lp;
       // the axis map (perm) travels with each task, not in the key
       qkey[q] = (uint32_t)la | ((uint32_t)lb << 3) | ((uint32_t)lc << 6) | ((uint32_t)ld << 9) |
-                ((uint32_t)tl << 20) | ((uint32_t)mode << 24) | (lowp << 26);
+                (lp << 12) | ((uint32_t)tl << 20) | ((uint32_t)mode << 24) | (lowp << 26);
       uint32_t nt = 1;
       for (int a = 0; a < naxes; ++a) nt *= (uint32_t)Q.nc[a];
       qnt[q] = nt;
@@ -820,12 +924,12 @@ static int plan_create_impl(mcint_plan** out, mcint_basis* b, int intor, const F
   }
   timer.mark("offsets, distinct keys");
   const KeyIndex kindex(ukeys);
-  const size_t nkeys = ukeys.size();
-  std::vector<int64_t> tcount((size_t)nthr * nkeys, 0);
-  std::vector<int64_t> pcount((size_t)nthr * nkeys, 0);  // primitive quartets
+  const size_t nraw = ukeys.size();
+  std::vector<int64_t> raw_tasks((size_t)nthr * nraw, 0);
+  std::vector<int64_t> raw_prims((size_t)nthr * nraw, 0);  // primitive quartets
   parallel_for(nthr, nq, [&](int th, size_t q0, size_t q1) {
-    int64_t* c = tcount.data() + (size_t)th * nkeys;
-    int64_t* pc = pcount.data() + (size_t)th * nkeys;
+    int64_t* c = raw_tasks.data() + (size_t)th * nraw;
+    int64_t* pc = raw_prims.data() + (size_t)th * nraw;
     for (size_t q = q0; q < q1; ++q) {
       if (!qnt[q]) continue;
       const uint32_t id = kindex.find(qkey[q]);
@@ -836,6 +940,22 @@ static int plan_create_impl(mcint_plan** out, mcint_basis* b, int intor, const F
       pc[id] += np;
     }
   });
+  // team sizes of the buckets: distinct final keys and each raw key's bucket
+  std::vector<uint32_t> bucket_of;
+  {
+    std::vector<int64_t> tasks(nraw, 0);
+    for (int th = 0; th < nthr; ++th)
+      for (size_t i = 0; i < nraw; ++i) tasks[i] += raw_tasks[(size_t)th * nraw + i];
+    ukeys = bucket_keys(ukeys, tasks, kind, b->omega, bucket_of);
+  }
+  const size_t nkeys = ukeys.size();
+  std::vector<int64_t> tcount((size_t)nthr * nkeys, 0);
+  std::vector<int64_t> pcount((size_t)nthr * nkeys, 0);
+  for (int th = 0; th < nthr; ++th)
+    for (size_t i = 0; i < nraw; ++i) {
+      tcount[(size_t)th * nkeys + bucket_of[i]] += raw_tasks[(size_t)th * nraw + i];
+      pcount[(size_t)th * nkeys + bucket_of[i]] += raw_prims[(size_t)th * nraw + i];
+    }
   // bucket starts, and each thread's cursor inside every bucket
   std::vector<int64_t> cnt(nkeys + 1, 0);
   std::vector<int64_t> cursor((size_t)nthr * nkeys, 0);
@@ -863,7 +983,7 @@ static int plan_create_impl(mcint_plan** out, mcint_basis* b, int intor, const F
       int la, lb, lc, ld, perm;
       tuple_class(kind, Q, la, lb, lc, ld, perm);
       const FINT* s = shls + 4 * q;
-      int64_t& d = cur[qkey[q]];
+      int64_t& d = cur[bucket_of[qkey[q]]];
       // virtual expansion over contraction columns of the original axes
       for_each_task(b->vfirst, b->dummy, kind, Q, s, qoff[q], perm, [&](const Task& t) {
         sorted[d] = t;
@@ -924,6 +1044,7 @@ static int plan_create_impl(mcint_plan** out, mcint_basis* b, int intor, const F
     bk.lc = (k >> 6) & 7;
     bk.ld = (k >> 9) & 7;
     bk.team = 1 << ((k >> 20) & 15);
+    bk.tune_team = 1 << ((k >> 12) & 15);
     bk.mode = (k >> 24) & 3;
     bk.fp32 = (k >> 26) & 1;
     bk.t0 = cnt[i];
@@ -1084,6 +1205,7 @@ static BucketArgs bucket_args(const mcint_plan* p, const Bucket& bk, double* out
   A.kind = p->kind;
   A.sph = p->sph;
   A.team = bk.team;
+  A.tune_team = bk.tune_team;
   A.fp32 = bk.fp32;
   A.t0 = bk.t0;
   A.t1 = bk.t1;
@@ -2049,9 +2171,13 @@ int opt_tuple(OptDevice* d, int intor, const FINT* shls, double* blk_out) {
   const bool reg_ok = (b->omega >= 0 || kind != KIND_2E_IP1) && !g_generic_only;
   const int mode = reg_ok ? fast_kernel_mode(kind, sph, la, lb, lc, ld, b->omega) : 0;
   const int ppl_c = g_class_ppl[kind][class_index(la, lb, lc, ld)];
-  const int team = mode ? pick_team(nprimq, ppl_c ? ppl_c : g_prims_per_lane) : 1;
+  const int tune_team = mode ? pick_team(nprimq, ppl_c ? ppl_c : g_prims_per_lane) : 1;
   int nt = 1;
   for (int a = 0; a < naxes; ++a) nt *= Q.nc[a];
+  int lp = 0;
+  while (lp < 15 && ((int64_t)1 << lp) < nprimq) ++lp;
+  const int team = mode && g_fill_lanes > nt * tune_team
+                       ? widen_team(kind, tune_team, g_fill_lanes / (nt * tune_team), lp) : tune_team;
   const int64_t blk = Q.so[4] * ncomp;
   int64_t sstride = 0;
   if (mode == 2) {
@@ -2122,6 +2248,7 @@ int opt_tuple(OptDevice* d, int intor, const FINT* shls, double* blk_out) {
   A.kind = kind;
   A.sph = sph;
   A.team = team;
+  A.tune_team = tune_team;
   A.fp32 = 0;
   A.dm = nullptr;
   A.grad = nullptr;

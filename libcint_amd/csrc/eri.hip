@@ -815,5 +815,22 @@ int wave_kernel_exists(int la, int lb, int lc, int ld) {
   return 0;
 }
 #undef MC_WAVE_HAS
+#define MC_WAVE_DEFAULT(a, b, c, d) \
+  if (la == a && lb == b && lc == c && ld == d) return WaveCfg<a, b, c, d>::DEFAULT;
+static bool wave_kernel_default(int la, int lb, int lc, int ld) {
+  MCINT_CHUNK_CLASSES(MC_WAVE_DEFAULT)
+  return false;
+}
+#undef MC_WAVE_DEFAULT
+bool chunk_class_on_wave(int la, int lb, int lc, int ld, int tune_team, double omega, int fp32) {
+  if (omega < 0 || fp32 || g_wave_kernels == 0 || !wave_kernel_exists(la, lb, lc, ld)) return false;
+  if (g_wave_kernels == 2) return true;
+  // per class and team size: the tuned choice, else the built-in rule
+  // (team-of-one buckets, blocks of 480+ components)
+  int tl = 0;
+  while ((1 << tl) < tune_team && tl < 6) ++tl;
+  const int cw = g_class_wave[class_index(la, lb, lc, ld) * 7 + tl];
+  return cw ? cw == 2 : tune_team == 1 && wave_kernel_default(la, lb, lc, ld);
+}
 MCINT_FAST_DISPATCH
 }  // namespace mcint

@@ -1836,17 +1836,8 @@ hipError_t launch_chunks(const BasisView& B, const BucketArgs& A0, hipStream_t s
   hipError_t e = hipSuccess;
   BucketArgs A = A0;
   if constexpr (DER == 0 && WaveCfg<LA, LB, LC, LD>::OK) {
-    // team-of-one buckets (few primitive quartets per quartet), plain
-    // operator and long range, FP64
-    // per class and team size: the tuned choice, else the built-in rule
-    // (team-of-one buckets, blocks of 480+ components)
-    int tl = 0;
-    while ((1 << tl) < A.team && tl < 6) ++tl;
-    const int cw = g_class_wave[class_index(LA, LB, LC, LD) * 7 + tl];
-    const bool dflt = A.team == 1 && WaveCfg<LA, LB, LC, LD>::DEFAULT;
-    if (B.omega >= 0 && !A.fp32 &&
-        (g_wave_kernels == 2 ||
-         (g_wave_kernels == 1 && (cw ? cw == 2 : dflt)))) {
+    // few primitive quartets per quartet, plain operator and long range, FP64
+    if (chunk_class_on_wave(LA, LB, LC, LD, A.tune_team, B.omega, A.fp32)) {
       A.col_major = 1;
       constexpr int TPW = WaveCfg<LA, LB, LC, LD>::TPW;
       hipLaunchKernelGGL((eri_wave_kernel<LA, LB, LC, LD>), dim3((unsigned)((n + TPW - 1) / TPW)),

@@ -216,6 +216,9 @@ __host__ __device__ constexpr int class_index(int la, int lb, int lc, int ld) {
 extern int8_t g_class_wave[NCLS * 7];
 // 1 when the canonical plain class (la lb|lc ld) has a wave kernel
 int wave_kernel_exists(int la, int lb, int lc, int ld);
+// whether a bucket of the chunked plain class with teams of tune_team lanes
+// runs its wave kernel (the rule of launch_chunks)
+bool chunk_class_on_wave(int la, int lb, int lc, int ld, int tune_team, double omega, int fp32);
 int chunked_block_doubles(int kind, int la, int lb, int lc, int ld);
 int fast_team_lanes_max();
 hipError_t launch_fast(const BasisView& B, const BucketArgs& A, hipStream_t stream);

@@ -130,6 +130,8 @@ struct BucketArgs {
   int kind;
   int sph;
   int team;              // lanes per task (fast kernels)
+  int tune_team;         // team size that selects the tuned kernel of a chunked class
+                         // (= team unless the team was widened to fill the chip)
   int fp32;              // recurrences and contraction in FP32 (fast kernels)
   int col_major;         // chunked classes: per-task blocks stored [f][e] (wave
                          // kernel) instead of in the chunk order

@@ -1,0 +1,56 @@
+"""Launch shapes chosen by the size of a list, against the CPU oracle.
+
+Tolerance: the suite's |gpu - oracle| <= 1e-12 + 1e-10 |oracle| per element
+(sums over the same primitives in another order differ by rounding only).
+"""
+import numpy as np
+import pytest
+
+from libcint_amd.synthetic import make_molecule
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def mc():
+    import libcint_amd
+    libcint_amd.lib()
+    return libcint_amd
+
+
+@pytest.fixture(scope="module")
+def orc():
+    import oracle
+    oracle.build()
+    oracle.set_root_mode(oracle.ROOTS_TABLE)
+    yield oracle
+    oracle.set_root_mode(oracle.ROOTS_EXACT)
+
+
+def _close(got, ref, what):
+    err = np.abs(got - ref)
+    bad = err > 1e-12 + 1e-10 * np.abs(ref)
+    assert not bad.any(), f"{what}: {int(bad.sum())} elements, max |err| {err.max():.2e}"
+
+
+def _quartets(nbas, n, seed):
+    return np.random.default_rng(seed).integers(0, nbas, (n, 4)).astype(np.int32)
+
+
+@pytest.mark.parametrize("fill", [0, 1 << 11, 1 << 17, 1 << 30])
+@pytest.mark.parametrize("name", ["int2e_sph", "int2e_cart", "int3c2e_sph"])
+def test_widened_teams(mc, orc, name, fill):
+    """Teams as tuned (0), widened a little and widened to a whole wave give
+    the oracle's blocks and flags; contractions of 1 to 10 primitives."""
+    m = make_molecule("c4" if name == "int3c2e_sph" else "c1")
+    q = _quartets(m.nbas if m.aux_start < 0 else m.aux_start, 700, 5)
+    if m.aux_start >= 0:
+        q[:, 2] = np.random.default_rng(6).integers(m.aux_start, m.nbas, len(q))
+    old = mc.tune(mc.TUNE_FILL_LANES, fill)
+    try:
+        got, _, nz = mc.batch(name, q, mc.Basis(m.atm, m.bas, m.env))
+    finally:
+        mc.tune(mc.TUNE_FILL_LANES, old)
+    ref, _, nz_r = orc.batch(name, q, orc.Basis(m.atm, m.bas, m.env))
+    _close(got, ref, f"{name} fill {fill}")
+    np.testing.assert_array_equal(nz, nz_r)
