@@ -455,8 +455,9 @@ struct KeyIndex {
 };
 
 struct Bucket {
-  int la, lb, lc, ld, team;
-  int tune_team;  // team size by the tuned primitive quartets per lane (team: widened to fill the chip)
+  int la, lb, lc, ld;
+  int team;   // team size by the tuned primitive quartets per lane
+  int lanes;  // lanes per task at launch: team, or widened to fill the chip
   int mode;  // 0 generic, 1 fast (single chunk), 2 chunked
   int fp32;  // recurrences in FP32 (mode 1 only)
   int64_t t0, t1;
@@ -541,64 +542,54 @@ int widen_team(int kind, int team, int64_t f, int lp) {
   return t;
 }
 
-// The buckets' keys of a plan from its raw keys (class, log2 of the
-// primitive quartets, team by the tuned primitive quartets per lane, path,
-// precision) and their task counts; bucket_of[i]: the bucket of raw key i.
-// A class that puts fewer than g_fill_lanes lanes to work has its teams
-// widened, and keeps one bucket per team size and kernel: what bounds it is
-// the length of a lane's chain of primitive quartets and the number of its
-// launches.  The final key holds the tuned team size (which selects the
-// tuned kernel of a chunked class) where the raw key holds the primitives.
-std::vector<uint32_t> bucket_keys(const std::vector<uint32_t>& raw,
-                                  const std::vector<int64_t>& tasks, int kind, double omega,
-                                  std::vector<uint32_t>& bucket_of) {
-  constexpr uint32_t GROUP = ~((15u << 12) | (15u << 20));  // class, path, precision
+// Key fields of a group of tasks: class (bits 0-11), log2 of the primitive
+// quartets (12-15), log2 of the tuned team (20-23), path (24-25), FP32 (26).
+constexpr uint32_t KEY_PRIMS = 15u << 12, KEY_TEAM = 15u << 20;
+inline int key_prims(uint32_t k) { return (k >> 12) & 15; }
+inline int key_team(uint32_t k) { return (k >> 20) & 15; }
+inline int key_mode(uint32_t k) { return (k >> 24) & 3; }
+
+// Groups of a plan's tasks from their raw keys and task counts: group_of[i]
+// is the group of raw key i, lanes[g] the lanes per task of group g.  A
+// class that puts fewer than g_fill_lanes lanes to work has its teams
+// widened (what bounds it is one lane's chain of primitive quartets) and
+// keeps its groups by primitive quartets; other classes keep one group per
+// team.  Groups are ordered by path, precision and class, then by descending
+// team and primitives: a bucket (class, team) is a run of groups, and so is
+// a launch (class, lanes, kernel).
+std::vector<uint32_t> task_groups(const std::vector<uint32_t>& raw, const std::vector<int64_t>& tasks,
+                                  int kind, std::vector<uint32_t>& group_of, std::vector<int>& lanes) {
+  constexpr uint32_t CLASS = ~(KEY_PRIMS | KEY_TEAM);  // class, path, precision
   const size_t n = raw.size();
+  std::vector<uint32_t> classes(n);
+  for (size_t i = 0; i < n; ++i) classes[i] = raw[i] & CLASS;
+  std::sort(classes.begin(), classes.end());
+  classes.erase(std::unique(classes.begin(), classes.end()), classes.end());
+  auto class_of = [&](uint32_t k) {
+    return (size_t)(std::lower_bound(classes.begin(), classes.end(), k & CLASS) - classes.begin());
+  };
+  std::vector<int64_t> busy(classes.size(), 0);  // lanes at work
+  for (size_t i = 0; i < n; ++i) busy[class_of(raw[i])] += tasks[i] << key_team(raw[i]);
+  auto widened = [&](uint32_t k) { return key_mode(k) != 0 && busy[class_of(k)] < g_fill_lanes; };
   std::vector<uint32_t> fin(n);
-  std::vector<uint32_t> groups(n);
-  for (size_t i = 0; i < n; ++i) groups[i] = raw[i] & GROUP;
-  std::sort(groups.begin(), groups.end());
-  groups.erase(std::unique(groups.begin(), groups.end()), groups.end());
-  std::vector<int64_t> lanes(groups.size(), 0);
-  auto group = [&](uint32_t k) {
-    return (size_t)(std::lower_bound(groups.begin(), groups.end(), k & GROUP) - groups.begin());
-  };
-  auto wave = [&](uint32_t k, int tl) {
-    return kind == KIND_2E && ((k >> 24) & 3) == 2 &&
-           chunk_class_on_wave(k & 7, (k >> 3) & 7, (k >> 6) & 7, (k >> 9) & 7, 1 << tl, omega,
-                               (k >> 26) & 1);
-  };
-  // smallest tuned team of each group on the chunk kernels / the wave kernel
-  std::vector<int> low(2 * groups.size(), 15);
-  for (size_t i = 0; i < n; ++i) {
-    const size_t g = group(raw[i]);
-    const int tl = (raw[i] >> 20) & 15;
-    lanes[g] += tasks[i] << tl;
-    int& l = low[2 * g + wave(raw[i], tl)];
-    l = std::min(l, tl);
-  }
-  for (size_t i = 0; i < n; ++i) {
-    const size_t g = group(raw[i]);
-    int tl = (raw[i] >> 20) & 15, tune = tl;
-    if (((raw[i] >> 24) & 3) != 0 && lanes[g] < g_fill_lanes) {
-      const bool w = wave(raw[i], tl);
-      tune = low[2 * g + w];
-      if (w) {
-        tl = tune;
-      } else {
-        const int t = widen_team(kind, 1 << tl, g_fill_lanes / std::max<int64_t>(1, lanes[g]),
-                                 (raw[i] >> 12) & 15);
-        while ((1 << tl) < t) ++tl;
-      }
-    }
-    fin[i] = (raw[i] & GROUP) | ((uint32_t)tune << 12) | ((uint32_t)tl << 20);
-  }
+  for (size_t i = 0; i < n; ++i) fin[i] = widened(raw[i]) ? raw[i] : raw[i] & ~KEY_PRIMS;
   std::vector<uint32_t> keys = fin;
-  std::sort(keys.begin(), keys.end());
+  auto before = [&](uint32_t x, uint32_t y) {
+    if ((x ^ y) & CLASS) return (x & CLASS) < (y & CLASS);
+    return (x & ~CLASS) > (y & ~CLASS);
+  };
+  std::sort(keys.begin(), keys.end(), before);
   keys.erase(std::unique(keys.begin(), keys.end()), keys.end());
-  bucket_of.resize(n);
+  group_of.resize(n);
   for (size_t i = 0; i < n; ++i)
-    bucket_of[i] = (uint32_t)(std::lower_bound(keys.begin(), keys.end(), fin[i]) - keys.begin());
+    group_of[i] = (uint32_t)(std::lower_bound(keys.begin(), keys.end(), fin[i], before) - keys.begin());
+  lanes.resize(keys.size());
+  for (size_t g = 0; g < keys.size(); ++g) {
+    lanes[g] = 1 << key_team(keys[g]);
+    if (widened(keys[g]))
+      lanes[g] = widen_team(kind, lanes[g], g_fill_lanes / std::max<int64_t>(1, busy[class_of(keys[g])]),
+                            key_prims(keys[g]));
+  }
   return keys;
 }
 
@@ -608,7 +599,8 @@ struct mcint_plan {
   mcint_basis* b = nullptr;
   int intor = 0, kind = 0, sph = 1, ncomp = 1;
   int64_t nq = 0, ntasks = 0, out_size = 0;
-  std::vector<Bucket> buckets;
+  std::vector<Bucket> buckets;   // tasks of one class and tuned team
+  std::vector<Bucket> launches;  // tasks of one class, lanes per task and kernel
   Task* tasks_d = nullptr;
   int* task_id_d = nullptr;
   int64_t* pair_off_d = nullptr;
@@ -940,21 +932,22 @@ static int plan_create_impl(mcint_plan** out, mcint_basis* b, int intor, const F
       pc[id] += np;
     }
   });
-  // team sizes of the buckets: distinct final keys and each raw key's bucket
-  std::vector<uint32_t> bucket_of;
+  // groups of tasks with one team size, and each raw key's group
+  std::vector<uint32_t> group_of;
+  std::vector<int> lanes;
   {
     std::vector<int64_t> tasks(nraw, 0);
     for (int th = 0; th < nthr; ++th)
       for (size_t i = 0; i < nraw; ++i) tasks[i] += raw_tasks[(size_t)th * nraw + i];
-    ukeys = bucket_keys(ukeys, tasks, kind, b->omega, bucket_of);
+    ukeys = task_groups(ukeys, tasks, kind, group_of, lanes);
   }
   const size_t nkeys = ukeys.size();
   std::vector<int64_t> tcount((size_t)nthr * nkeys, 0);
   std::vector<int64_t> pcount((size_t)nthr * nkeys, 0);
   for (int th = 0; th < nthr; ++th)
     for (size_t i = 0; i < nraw; ++i) {
-      tcount[(size_t)th * nkeys + bucket_of[i]] += raw_tasks[(size_t)th * nraw + i];
-      pcount[(size_t)th * nkeys + bucket_of[i]] += raw_prims[(size_t)th * nraw + i];
+      tcount[(size_t)th * nkeys + group_of[i]] += raw_tasks[(size_t)th * nraw + i];
+      pcount[(size_t)th * nkeys + group_of[i]] += raw_prims[(size_t)th * nraw + i];
     }
   // bucket starts, and each thread's cursor inside every bucket
   std::vector<int64_t> cnt(nkeys + 1, 0);
@@ -983,7 +976,7 @@ static int plan_create_impl(mcint_plan** out, mcint_basis* b, int intor, const F
       int la, lb, lc, ld, perm;
       tuple_class(kind, Q, la, lb, lc, ld, perm);
       const FINT* s = shls + 4 * q;
-      int64_t& d = cur[bucket_of[qkey[q]]];
+      int64_t& d = cur[group_of[qkey[q]]];
       // virtual expansion over contraction columns of the original axes
       for_each_task(b->vfirst, b->dummy, kind, Q, s, qoff[q], perm, [&](const Task& t) {
         sorted[d] = t;
@@ -1002,7 +995,7 @@ static int plan_create_impl(mcint_plan** out, mcint_basis* b, int intor, const F
     const int naxes_s = kind_axes(kind);
     std::vector<size_t> small;
     for (size_t i = 0; i < nkeys; ++i)
-      if (((ukeys[i] >> 20) & 15) <= 1 && ((ukeys[i] >> 24) & 3) != 0 && cnt[i + 1] - cnt[i] > 1)
+      if (key_team(ukeys[i]) <= 1 && key_mode(ukeys[i]) != 0 && cnt[i + 1] - cnt[i] > 1)
         small.push_back(i);
     std::atomic<size_t> next{0};
     const int nw = std::min<int>(nthr, (int)small.size());
@@ -1043,9 +1036,9 @@ static int plan_create_impl(mcint_plan** out, mcint_basis* b, int intor, const F
     bk.lb = (k >> 3) & 7;
     bk.lc = (k >> 6) & 7;
     bk.ld = (k >> 9) & 7;
-    bk.team = 1 << ((k >> 20) & 15);
-    bk.tune_team = 1 << ((k >> 12) & 15);
-    bk.mode = (k >> 24) & 3;
+    bk.team = 1 << key_team(k);
+    bk.lanes = lanes[i];
+    bk.mode = key_mode(k);
     bk.fp32 = (k >> 26) & 1;
     bk.t0 = cnt[i];
     bk.t1 = cnt[i + 1];
@@ -1055,12 +1048,7 @@ static int plan_create_impl(mcint_plan** out, mcint_basis* b, int intor, const F
     if (bk.fp32) p->stats_fp32 += bk.t1 - bk.t0;
     bk.sstride = 0;
     if (bk.mode == 2) {
-      const int64_t nef = chunked_block_doubles(kind, bk.la, bk.lb, bk.lc, bk.ld);
-      bk.sstride = nef;
-      const int64_t chunk = std::max<int64_t>(1, std::min<int64_t>(bk.t1 - bk.t0, GEN_SCRATCH_DOUBLES / nef));
-      max_gen = std::max(max_gen, chunk * nef);
-      max_flags = std::max(max_flags, chunk);
-      p->stats[2] += bk.t1 - bk.t0;
+      bk.sstride = chunked_block_doubles(kind, bk.la, bk.lb, bk.lc, bk.ld);
     } else if (bk.mode == 0) {
       const GenLayout G = gen_layout(kind, sph, bk.la, bk.lb, bk.lc, bk.ld);
       const int nr = (bk.la + bk.lb + bk.lc + (kind_three(kind) ? 0 : bk.ld) +
@@ -1072,15 +1060,42 @@ static int plan_create_impl(mcint_plan** out, mcint_basis* b, int intor, const F
         return MCINT_ERR_UNSUPPORTED;
       }
       bk.sstride = G.total;
-      const int64_t chunk = std::max<int64_t>(1, std::min<int64_t>(bk.t1 - bk.t0,
-                                                   GEN_SCRATCH_DOUBLES / std::max<int64_t>(1, G.total)));
-      max_gen = std::max(max_gen, chunk * G.total);
-      p->stats[3] += bk.t1 - bk.t0;
-    } else {
-      p->stats[2] += bk.t1 - bk.t0;
     }
-    p->buckets.push_back(bk);
+    p->stats[bk.mode == 0 ? 3 : 2] += bk.t1 - bk.t0;
+    // runs of groups: the launch (same lanes and kernel) and the bucket
+    auto extend = [&](std::vector<Bucket>& v, bool join) {
+      if (join) {
+        v.back().t1 = bk.t1;
+        v.back().cost += bk.cost;
+      } else {
+        v.push_back(bk);
+      }
+    };
+    auto same_class = [&](const Bucket& o) {
+      return o.la == bk.la && o.lb == bk.lb && o.lc == bk.lc && o.ld == bk.ld && o.mode == bk.mode &&
+             o.fp32 == bk.fp32;
+    };
+    auto wave = [&](const Bucket& o) {
+      return o.mode == 2 && chunk_class_on_wave(o.la, o.lb, o.lc, o.ld, o.team, b->omega, o.fp32) &&
+             kind == KIND_2E;
+    };
+    const bool lj = !p->launches.empty() && same_class(p->launches.back()) &&
+                    wave(p->launches.back()) == wave(bk) &&
+                    (wave(bk) || p->launches.back().lanes == bk.lanes) &&
+                    (p->launches.back().team == bk.team || key_prims(k));
+    extend(p->launches, lj);
+    extend(p->buckets, !p->buckets.empty() && same_class(p->buckets.back()) &&
+                           p->buckets.back().team == bk.team);
+    p->buckets.back().lanes = bk.team;
   }
+  for (const auto* list : {&p->buckets, &p->launches})
+    for (const Bucket& bk : *list) {
+      if (bk.mode == 1) continue;
+      const int64_t n = std::max<int64_t>(1, std::min<int64_t>(bk.t1 - bk.t0,
+                                              GEN_SCRATCH_DOUBLES / std::max<int64_t>(1, bk.sstride)));
+      max_gen = std::max(max_gen, n * bk.sstride);
+      if (bk.mode == 2) max_flags = std::max(max_flags, n);
+    }
   p->stats[0] = p->ntasks;
   p->stats[1] = (int64_t)p->buckets.size();
 
@@ -1204,8 +1219,8 @@ static BucketArgs bucket_args(const mcint_plan* p, const Bucket& bk, double* out
   A.ld = bk.ld;
   A.kind = p->kind;
   A.sph = p->sph;
-  A.team = bk.team;
-  A.tune_team = bk.tune_team;
+  A.team = bk.lanes;
+  A.tune_team = bk.team;
   A.fp32 = bk.fp32;
   A.t0 = bk.t0;
   A.t1 = bk.t1;
@@ -1303,7 +1318,7 @@ static int bucket_launch(mcint_plan* p, const Bucket& bk, double* out, FINT* not
 
 static int plan_launch(mcint_plan* p, double* out, FINT* not0, hipStream_t stream,
                        const ScratchView& S) {
-  for (const Bucket& bk : p->buckets) {
+  for (const Bucket& bk : p->launches) {
     const int st = bucket_launch(p, bk, out, not0, stream, S);
     if (st) return st;
   }
@@ -1329,16 +1344,16 @@ static int launch_branched(mcint_plan* p, hipStream_t stream, int nbr, F&& launc
     HIPCHK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
     p->events.push_back(ev);
   }
-  std::vector<int> order(p->buckets.size());
+  std::vector<int> order(p->launches.size());
   for (size_t i = 0; i < order.size(); ++i) order[i] = (int)i;
   std::stable_sort(order.begin(), order.end(),
-                   [&](int a, int b) { return p->buckets[a].cost > p->buckets[b].cost; });
+                   [&](int a, int b) { return p->launches[a].cost > p->launches[b].cost; });
   std::vector<double> load(nbr, 0.0);
   std::vector<std::vector<int>> lists(nbr);
   for (int i : order) {
     const int k = (int)(std::min_element(load.begin(), load.end()) - load.begin());
     lists[k].push_back(i);
-    load[k] += p->buckets[i].cost;
+    load[k] += p->launches[i].cost;
   }
   HIPCHK(hipEventRecord(p->events[0], stream));
   int st = MCINT_OK;
@@ -1350,7 +1365,7 @@ static int launch_branched(mcint_plan* p, hipStream_t stream, int nbr, F&& launc
   if (e == hipSuccess) {
     for (int k = 0; k < nbr && st == MCINT_OK; ++k)
       for (int i : lists[k]) {
-        st = launch(p->buckets[i], p->side[k], plan_scratch(p, k));
+        st = launch(p->launches[i], p->side[k], plan_scratch(p, k));
         if (st) break;
       }
   }
@@ -1380,14 +1395,14 @@ extern "C" int mcint_plan_execute_grad(mcint_plan* p, const double* dm_dev, int 
     return MCINT_ERR_ARG;
   }
   hipStream_t stream = (hipStream_t)hip_stream;
-  for (const Bucket& bk : p->buckets)
+  for (const Bucket& bk : p->launches)
     if (bk.mode == 1) {
       set_err("mcint_plan_execute_grad: internal: derivative bucket on the single-kernel path");
       return MCINT_ERR_UNSUPPORTED;
     }
   // the buckets run over concurrent branches (as a captured plan does);
   // their digests add atomically into the shared accumulators
-  const int nbr = std::max(1, std::min<int>(g_graph_branches, (int)p->buckets.size()));
+  const int nbr = std::max(1, std::min<int>(g_graph_branches, (int)p->launches.size()));
   if (const int st = ensure_scratch(p, nbr)) return st;
   const BasisView B = plan_view(p);
   // per-block partial sums go to GRAD_SLOTS copies of the accumulators
@@ -1418,7 +1433,7 @@ extern "C" int mcint_plan_execute_grad(mcint_plan* p, const double* dm_dev, int 
   if (nbr > 1) {
     if (const int st = launch_branched(p, stream, nbr, launch)) return st;
   } else {
-    for (const Bucket& bk : p->buckets)
+    for (const Bucket& bk : p->launches)
       if (const int st = launch(bk, stream, plan_scratch(p))) return st;
   }
   HIPCHK(launch_grad_reduce(p->gslots_d, GRAD_SLOTS, n, grad_dev, stream));
@@ -1446,7 +1461,7 @@ extern "C" int mcint_plan_execute_jk(mcint_plan* p, const double* dm_dev, int na
     return MCINT_ERR_ARG;
   }
   hipStream_t stream = (hipStream_t)hip_stream;
-  const int nbr = std::max(1, std::min<int>(g_graph_branches, (int)p->buckets.size()));
+  const int nbr = std::max(1, std::min<int>(g_graph_branches, (int)p->launches.size()));
   if (const int st = ensure_scratch(p, nbr)) return st;
   const int64_t nn = (int64_t)nao * nao;
   if (p->jk_n < nn) {
@@ -1485,7 +1500,7 @@ extern "C" int mcint_plan_execute_jk(mcint_plan* p, const double* dm_dev, int na
   if (nbr > 1) {
     if (const int st = launch_branched(p, stream, nbr, launch)) return st;
   } else {
-    for (const Bucket& bk : p->buckets)
+    for (const Bucket& bk : p->launches)
       if (const int st = launch(bk, stream, plan_scratch(p))) return st;
   }
   if (vj_dev) HIPCHK(launch_symmetrize(Jp, vj_dev, nao, stream));
@@ -1756,7 +1771,7 @@ extern "C" int mcint_plan_execute(mcint_plan* p, double* out_dev, FINT* not0_dev
     if (const int st = ensure_scratch(p)) return st;
     return plan_launch(p, out_dev, not0_dev, stream, plan_scratch(p));
   }
-  const int nbr = std::max(1, std::min<int>(g_graph_branches, (int)p->buckets.size()));
+  const int nbr = std::max(1, std::min<int>(g_graph_branches, (int)p->launches.size()));
   if (const int st = ensure_scratch(p, nbr)) return st;
   if (!p->gexec || p->g_out != out_dev || p->g_not0 != not0_dev || p->g_stream != stream ||
       p->g_nbr != nbr) {
@@ -1798,7 +1813,7 @@ int mcint::plan_launch_scratch(mcint_plan* p, double* out, FINT* not0, hipStream
   S.nblocks = nblocks;
   S.flags = flags;
   S.nflags = nflags;
-  for (const Bucket& bk : p->buckets) {
+  for (const Bucket& bk : p->launches) {
     if (bk.mode != 1 && slice_tasks(bk, S) < 1) {
       char msg[200];
       snprintf(msg, sizeof msg,
