@@ -796,25 +796,26 @@ struct ChunkCfg {
   }
 };
 
-template <int LA, int LB, int LC, int LD, int CH, int DER = 0, typename R = double>
-__global__ void __launch_bounds__((ChunkCfg<LA, LB, LC, LD, DER>::THREADS))
-__attribute__((amdgpu_waves_per_eu(min_waves(LA, LB, LC, LD, DER, CH))))
-eri_chunk_kernel(BasisView Bv, BucketArgs A) {
+// Chunks of a class are independent (each evaluates the walk for its own
+// components), so a launch carries up to CHUNK_GROUP of them, one per grid
+// row: on short lists a class's time was the sum of its chunks' serial
+// chains, each on a few workgroups.  Rows are dispatched one after another,
+// so that long lists still run one chunk's code at a time per CU.  Eight:
+// a larger group only costs compile time (all its chunks are one kernel).
+constexpr int CHUNK_GROUP = 8;
+constexpr int chunk_groups(int nch) { return (nch + CHUNK_GROUP - 1) / CHUNK_GROUP; }
+
+// One chunk of one task: primitive sums of its components over the team,
+// stored to the task's block.
+template <int LA, int LB, int LC, int LD, int CH, int DER, typename R>
+__device__ __forceinline__ void chunk_body(const BasisView& Bv, const BucketArgs& A, int64_t t, int T,
+                                           int tl, const double* rtab, int* rows) {
   using G = ChunkCfg<LA, LB, LC, LD, DER>;
   constexpr int K0 = G::k0(CH), K1 = G::k1(CH);
-  __shared__ double s_rys[RysLds<G::C::NR>::N];
-  __shared__ int s_rows[DER == 2 || DER == 3 ? 1 : stair_lds_ints(G::THREADS)];
-  const double* rtab = rys_stage_table<G::C::NR>(s_rys);
-  const int T = A.team;
-  const int tid = threadIdx.x;
-  const int tl = tid & (T - 1);
-  const int64_t t = A.t0 + (int64_t)blockIdx.x * (G::THREADS / T) + tid / T;
-  if (t >= A.t1) return;
   const Task tk = A.tasks[t];
   R acc[K1 - K0];
   int any, live;
-  accumulate<LA, LB, LC, LD, K0, K1, R, DER, G::ORDW>(Bv, tk, T, tl, rtab, stair_rows(s_rows, T), acc,
-                                                      any, live);
+  accumulate<LA, LB, LC, LD, K0, K1, R, DER, G::ORDW>(Bv, tk, T, tl, rtab, rows, acc, any, live);
   for (int off = 1; off < T; off <<= 1) {
     sfor<K1 - K0>([&](auto I) {
       constexpr int i = decltype(I)::value;
@@ -834,6 +835,29 @@ eri_chunk_kernel(BasisView Bv, BucketArgs A) {
       if (A.not0) A.not0[A.task_id ? A.task_id[t] : t] = any && live;
     }
   }
+}
+
+// Chunks GRP * CHUNK_GROUP .. of a class, chunk blockIdx.y of the group.
+template <int LA, int LB, int LC, int LD, int GRP, int DER = 0, typename R = double>
+__global__ void __launch_bounds__((ChunkCfg<LA, LB, LC, LD, DER>::THREADS))
+__attribute__((amdgpu_waves_per_eu(min_waves(LA, LB, LC, LD, DER, GRP))))
+eri_chunk_kernel(BasisView Bv, BucketArgs A) {
+  using G = ChunkCfg<LA, LB, LC, LD, DER>;
+  constexpr int C0 = GRP * CHUNK_GROUP;
+  constexpr int N = G::NCH - C0 < CHUNK_GROUP ? G::NCH - C0 : CHUNK_GROUP;
+  __shared__ double s_rys[RysLds<G::C::NR>::N];
+  __shared__ int s_rows[DER == 2 || DER == 3 ? 1 : stair_lds_ints(G::THREADS)];
+  const double* rtab = rys_stage_table<G::C::NR>(s_rys);
+  const int T = A.team;
+  const int tid = threadIdx.x;
+  const int tl = tid & (T - 1);
+  const int64_t t = A.t0 + (int64_t)blockIdx.x * (G::THREADS / T) + tid / T;
+  if (t >= A.t1) return;
+  int* rows = stair_rows(s_rows, T);
+  sfor<N>([&](auto I) {
+    constexpr int c = decltype(I)::value;
+    if (blockIdx.y == c) chunk_body<LA, LB, LC, LD, C0 + c, DER, R>(Bv, A, t, T, tl, rtab, rows);
+  });
 }
 
 // (b, t) pairs of the transfer (a,b| = sum_t C(b,t) (A-B)^(b-t) [a+t| over
@@ -1812,27 +1836,29 @@ __global__ void __launch_bounds__(64) eri_wave_kernel(BasisView Bv, BucketArgs A
   }
 }
 
-template <int LA, int LB, int LC, int LD, int CH, int DER>
-hipError_t launch_one_chunk(const BasisView& B, const BucketArgs& A, hipStream_t stream, dim3 grid) {
-  constexpr int TH = ChunkCfg<LA, LB, LC, LD, DER>::THREADS;
+template <int LA, int LB, int LC, int LD, int GRP, int DER>
+hipError_t launch_chunk_group(const BasisView& B, const BucketArgs& A, hipStream_t stream, unsigned nblk) {
+  using G = ChunkCfg<LA, LB, LC, LD, DER>;
+  constexpr int N = G::NCH - GRP * CHUNK_GROUP < CHUNK_GROUP ? G::NCH - GRP * CHUNK_GROUP : CHUNK_GROUP;
+  const dim3 grid(nblk, N);
   // the FP32 tier exists for the derivative chunks (gradient digest)
   if constexpr (DER == 1) {
     if (A.fp32) {
-      hipLaunchKernelGGL((eri_chunk_kernel<LA, LB, LC, LD, CH, DER, float>), grid, dim3(TH), 0,
+      hipLaunchKernelGGL((eri_chunk_kernel<LA, LB, LC, LD, GRP, DER, float>), grid, dim3(G::THREADS), 0,
                          stream, B, A);
       return hipGetLastError();
     }
   }
-  hipLaunchKernelGGL((eri_chunk_kernel<LA, LB, LC, LD, CH, DER>), grid, dim3(TH), 0, stream, B, A);
+  hipLaunchKernelGGL((eri_chunk_kernel<LA, LB, LC, LD, GRP, DER>), grid, dim3(G::THREADS), 0, stream, B, A);
   return hipGetLastError();
 }
 
-template <int LA, int LB, int LC, int LD, int DER, int... CHs>
+template <int LA, int LB, int LC, int LD, int DER, int... GRPs>
 hipError_t launch_chunks(const BasisView& B, const BucketArgs& A0, hipStream_t stream,
-                         std::integer_sequence<int, CHs...>) {
+                         std::integer_sequence<int, GRPs...>) {
   const int64_t n = A0.t1 - A0.t0;
   const int64_t per = ChunkCfg<LA, LB, LC, LD, DER>::THREADS / A0.team;
-  const dim3 grid((unsigned)((n + per - 1) / per));
+  const unsigned nblk = (unsigned)((n + per - 1) / per);
   hipError_t e = hipSuccess;
   BucketArgs A = A0;
   if constexpr (DER == 0 && WaveCfg<LA, LB, LC, LD>::OK) {
@@ -1846,7 +1872,7 @@ hipError_t launch_chunks(const BasisView& B, const BucketArgs& A0, hipStream_t s
     }
   }
   if (!A.col_major)
-    ((e = (e == hipSuccess ? launch_one_chunk<LA, LB, LC, LD, CHs, DER>(B, A, stream, grid) : e)), ...);
+    ((e = (e == hipSuccess ? launch_chunk_group<LA, LB, LC, LD, GRPs, DER>(B, A, stream, nblk) : e)), ...);
   if (e != hipSuccess) return e;
   if constexpr (DER == 0 && WaveCfg<LA, LB, LC, LD>::OK) {
     // the wave kernel stored or digested the blocks itself
@@ -2036,9 +2062,9 @@ hipError_t launch_chunk3_class(const BasisView& B, const BucketArgs& A, hipStrea
                                               hipStream_t stream) {                        \
     if (B.omega < 0)                                                                       \
       return launch_chunks<a, b, c, d, 4>(                                                 \
-          B, A, stream, std::make_integer_sequence<int, ChunkCfg<a, b, c, d, 4>::NCH>{});  \
+          B, A, stream, std::make_integer_sequence<int, chunk_groups(ChunkCfg<a, b, c, d, 4>::NCH)>{});  \
     return launch_chunks<a, b, c, d, 0>(                                                   \
-        B, A, stream, std::make_integer_sequence<int, ChunkCfg<a, b, c, d>::NCH>{});       \
+        B, A, stream, std::make_integer_sequence<int, chunk_groups(ChunkCfg<a, b, c, d>::NCH)>{});       \
   }
 #define MCINT_FAST3_DEFINE(a, b, c, d)                                                     \
   template <>                                                                              \
@@ -2063,16 +2089,16 @@ hipError_t launch_chunk3_class(const BasisView& B, const BucketArgs& A, hipStrea
                                              hipStream_t stream) {                         \
     if (B.omega < 0)                                                                       \
       return launch_chunks<a, b, c, d, 3>(                                                 \
-          B, A, stream, std::make_integer_sequence<int, ChunkCfg<a, b, c, d, 3>::NCH>{});  \
+          B, A, stream, std::make_integer_sequence<int, chunk_groups(ChunkCfg<a, b, c, d, 3>::NCH)>{});  \
     return launch_chunks<a, b, c, d, 2>(                                                   \
-        B, A, stream, std::make_integer_sequence<int, ChunkCfg<a, b, c, d, 2>::NCH>{});    \
+        B, A, stream, std::make_integer_sequence<int, chunk_groups(ChunkCfg<a, b, c, d, 2>::NCH)>{});    \
   }
 #define MCINT_IP1_DEFINE(a, b, c, d)                                                       \
   template <>                                                                              \
   hipError_t launch_ip1_class<a, b, c, d>(const BasisView& B, const BucketArgs& A,         \
                                           hipStream_t stream) {                            \
     return launch_chunks<a, b, c, d, 1>(                                                   \
-        B, A, stream, std::make_integer_sequence<int, ChunkCfg<a, b, c, d, 1>::NCH>{});    \
+        B, A, stream, std::make_integer_sequence<int, chunk_groups(ChunkCfg<a, b, c, d, 1>::NCH)>{});    \
   }
 
 #define MCINT_FAST_DECLARE(a, b, c, d)                                                     \
