@@ -24,10 +24,10 @@ OBJ = os.path.join(HERE, "_obj")
 LIB = os.path.join(HERE, "libmcint.so")
 
 # longest compiles first
-SOURCES = ([f"ip1_{g}.hip" for g in (14, *range(14))]
+SOURCES = ([f"fast_{g}.hip" for g in (8, 7)] + [f"ip1_{g}.hip" for g in (14, *range(14))]
            + [f"chunk3_{g}.hip" for g in range(4)] + [f"fast3_{g}.hip" for g in range(4)]
            + [f"chunk_{g}.hip" for g in (17, 11, 18, 19, 20, 21, 12, 13, 14, 15, 16, 10, 9, 8, 7, 6, 5, 4, 3, 2, 1, 0)]
-           + [f"fast_{g}.hip" for g in (7, 3, 8, 5, 6, 4, 2, 1, 0)] + ["eri.hip", "jk.hip", "api.hip", "noalloc.hip", "sr_roots.hip"])
+           + [f"fast_{g}.hip" for g in (3, 5, 6, 4, 2, 1, 0)] + ["generic.hip", "eri.hip", "jk.hip", "api.hip", "noalloc.hip", "sr_roots.hip"])
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("MCINT_ARCH", "gfx950")

@@ -29,6 +29,7 @@
 
 #include "../../include/mcint.h"
 #include "eri_launch.h"
+#include "gen_layout.h"
 #include "host_internal.h"
 
 using namespace mcint;
@@ -461,7 +462,7 @@ struct Bucket {
   int mode;  // 0 generic, 1 fast (single chunk), 2 chunked
   int fp32;  // recurrences in FP32 (mode 1 only)
   int64_t t0, t1;
-  int64_t sstride;  // generic scratch doubles per task
+  int64_t sstride;  // scratch doubles per task (0: blocks in LDS)
   double cost;      // estimated work (balances the concurrent graph branches)
 };
 
@@ -1050,16 +1051,13 @@ static int plan_create_impl(mcint_plan** out, mcint_basis* b, int intor, const F
     if (bk.mode == 2) {
       bk.sstride = chunked_block_doubles(kind, bk.la, bk.lb, bk.lc, bk.ld);
     } else if (bk.mode == 0) {
-      const GenLayout G = gen_layout(kind, sph, bk.la, bk.lb, bk.lc, bk.ld);
-      const int nr = (bk.la + bk.lb + bk.lc + (kind_three(kind) ? 0 : bk.ld) +
-                      kind_bra_raise(kind) + kind_ket_raise(kind)) / 2 + 1;
-      const int nrt = b->omega < 0 ? 2 * nr : nr;
-      if (G.nE > GEN_ECAP || G.nF > GEN_FCAP || 3 * nrt * (G.E + 1) * (G.F + 1) > GEN_VCAP) {
+      const GenLayout G = gen_layout(kind, sph, bk.la, bk.lb, bk.lc, bk.ld, b->omega);
+      if (!gen_fits(G)) {
         plan_free(p);
         set_err("mcint_plan_create: angular momentum beyond the generic kernel's tables");
         return MCINT_ERR_UNSUPPORTED;
       }
-      bk.sstride = G.total;
+      bk.sstride = G.nblk;
     }
     p->stats[bk.mode == 0 ? 3 : 2] += bk.t1 - bk.t0;
     // runs of groups: the launch (same lanes and kernel) and the bucket
@@ -1281,7 +1279,8 @@ static int ensure_scratch(mcint_plan* p, int nbr = 1) {
 
 // tasks of one bucket that fit the scratch at once (0: not even one)
 static int64_t slice_tasks(const Bucket& bk, const ScratchView& S) {
-  int64_t n = S.nblocks / std::max<int64_t>(1, bk.sstride);
+  if (bk.sstride == 0) return bk.t1 - bk.t0;  // blocks in LDS
+  int64_t n = S.nblocks / bk.sstride;
   if (bk.mode == 2) n = std::min(n, S.nflags);
   return n;
 }
@@ -2198,15 +2197,12 @@ int opt_tuple(OptDevice* d, int intor, const FINT* shls, double* blk_out) {
   if (mode == 2) {
     sstride = chunked_block_doubles(kind, la, lb, lc, ld);
   } else if (mode == 0) {
-    const GenLayout G = gen_layout(kind, sph, la, lb, lc, ld);
-    const int nr = (la + lb + lc + (kind_three(kind) ? 0 : ld) + kind_bra_raise(kind) +
-                    kind_ket_raise(kind)) / 2 + 1;
-    const int nrt = b->omega < 0 ? 2 * nr : nr;
-    if (G.nE > GEN_ECAP || G.nF > GEN_FCAP || 3 * nrt * (G.E + 1) * (G.F + 1) > GEN_VCAP) {
+    const GenLayout G = gen_layout(kind, sph, la, lb, lc, ld, b->omega);
+    if (!gen_fits(G)) {
       set_err("angular momentum beyond the generic kernel's tables");
       return -1;
     }
-    sstride = G.total;
+    sstride = G.nblk;
   }
   CallCtx* c = nullptr;
   {

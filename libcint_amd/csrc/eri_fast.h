@@ -13,7 +13,7 @@
 #include <type_traits>
 #include <utility>
 
-#include "gen_walk.h"
+#include "device_common.h"
 
 namespace mcint {
 
@@ -1591,7 +1591,7 @@ __global__ void __launch_bounds__(64) eri_wave_kernel(BasisView Bv, BucketArgs A
     sfor<NF>([&](auto J) { acc[decltype(S)::value][decltype(J)::value] = 0.0; });
   });
 
-  // libcint's screening, as in gen_walk for plain four-centre integrals
+  // libcint's screening, as in the generic kernel for plain four-centre integrals
   // (src/cint2e.c:57-269 with the optimizer's cutoffs)
   const int nij = sa.nprim * sb.nprim, nkl = sc.nprim * sd.nprim;
   const int64_t pab = (int64_t)tk.sh[0] * Bv.nv + tk.sh[1];

@@ -1,0 +1,178 @@
+// Work layout of the generic (any class) kernel, computed on the host and
+// passed to the kernel by value.
+#pragma once
+#include "mcint_internal.h"
+
+namespace mcint {
+
+// Bounds of what the generic kernel takes: recurrence tables of one
+// primitive quartet (3 directions x roots, doubled for short range, x
+// (E+1)(F+1) doubles) and Cartesian components of the e-list and f-list (all
+// of l <= 14: ipip1 of (66|ss) reaches e = 14).
+constexpr int GEN_VCAP = 3 * 2 * NRYS_MAX * 90;
+constexpr int GEN_ECAP = 680;
+constexpr int GEN_FCAP = 680;
+constexpr int GEN_LANES = 64;  // lanes of a workgroup (one wave, one task at a time)
+
+// LDS per wave, in doubles: derivative components share a pass as long as
+// the whole stays below the first figure (20 KB: eight waves per CU);
+// classes that need more than the second for one component (64 KB) keep
+// their blocks in global scratch.
+constexpr int GEN_LDS_TARGET = 2560;
+constexpr int GEN_LDS_MAX = 8000;
+
+// Cartesian components of all shells below l
+__host__ __device__ constexpr int tet(int l) { return l * (l + 1) * (l + 2) / 6; }
+// terms of the horizontal transfers of all Cartesian components of shell l:
+// sum over (bx, by, bz) of (bx+1)(by+1)(bz+1) = C(l+5, 5)
+__host__ __device__ constexpr int xfer_count(int l) {
+  return (l + 5) * (l + 4) * (l + 3) * (l + 2) * (l + 1) / 120;
+}
+
+// Primitive sums are kept as row sets of the bra (shells blo..bhi on centre
+// A, weighted by the bw-th power of 2 a_i) by column sets of the ket (shells
+// klo..khi on C, weighted by the kw-th power of 2 a_k); derivatives are
+// formed from them after contraction.  With D_p|a> = a_p|a-1_p> - 2a|a+1_p>:
+//   plain    bra la..la+lb                               ket lc..lc+ld
+//   ip1      bra la-1.. (1), la+1.. (2a)                 ket as plain
+//   ip2 (3c) bra as plain                                ket lc-1, lc+1 (2a)
+//   ipip1    bra la-2.. (1), la.. (2a), la+2.. (4a^2)    ket as plain
+//   ip1ip2   bra as ip1                                  ket lc-1.. (1), lc+1.. (2a)
+// X holds set r's rows by all KF ket columns; H1/H2 the bra transferred and
+// transformed, H3 the ket transferred, nbg bra components at a time.
+struct GenLayout {
+  int nbs, blo[3], bhi[3], nes[3], bw[3], ox[3];
+  int nks, klo[2], khi[2], nfs[2], kw[2], cf[2];
+  int e_lo, E, f_lo, F, nE, nF, KF;
+  int nbc, nkc, ncomp;  // derivative components of the bra, the ket, in all
+  int nca, ncb, ncc, ncd, nAo, nBo, nCo, nDo;
+  int lij, lkl, nr, nrt;
+  int nX, nH1, nH2, nH3;  // doubles of X and of one bra component's passes
+  // LDS doubles: block regions (nbg components per pass), then the walk's
+  // tables in the same space as the passes, the transfer terms, the codes
+  int PB, nbg, oH1, oH2, oV, oP, ou, ow, oTb, oTk, oI;
+  int lds;          // doubles of LDS
+  int in_lds;       // blocks in LDS (else in global scratch, nblk per wave)
+  int64_t nblk;     // doubles of global scratch per wave
+};
+
+// Doubles per primitive quartet of a batch besides its recurrence tables
+constexpr int GEN_PRIM_D = 19;
+
+inline GenLayout gen_layout(int kind, int sph, int la, int lb, int lc, int ld, double omega) {
+  GenLayout g{};
+  const bool three = kind_three(kind);
+  if (three) ld = 0;
+  const bool ip1 = kind_bra_der(kind) || kind == KIND_2E_IP1IP2;
+  const bool ket = kind_ket_der(kind) || kind == KIND_2E_IP1IP2;
+  auto bset = [&](int shift, int w) {
+    if (la + shift < 0) return;
+    const int r = g.nbs++;
+    g.blo[r] = la + shift;
+    g.bhi[r] = la + lb + shift;
+    g.bw[r] = w;
+    g.nes[r] = tet(g.bhi[r] + 1) - tet(g.blo[r]);
+  };
+  if (kind == KIND_2E_IPIP1) {
+    bset(-2, 0);
+    bset(0, 1);
+    bset(2, 2);
+  } else if (ip1) {
+    bset(-1, 0);
+    bset(1, 1);
+  } else {
+    bset(0, 0);
+  }
+  auto kset = [&](int shift, int w) {
+    if (lc + shift < 0) return;
+    const int u = g.nks++;
+    g.klo[u] = lc + shift;
+    g.khi[u] = lc + ld + shift;
+    g.kw[u] = w;
+    g.nfs[u] = tet(g.khi[u] + 1) - tet(g.klo[u]);
+    g.cf[u] = g.KF;
+    g.KF += g.nfs[u];
+  };
+  if (ket) {
+    kset(-1, 0);
+    kset(1, 1);
+  } else {
+    kset(0, 0);
+  }
+  g.e_lo = g.blo[0];
+  g.E = g.bhi[g.nbs - 1];
+  g.f_lo = g.klo[0];
+  g.F = g.khi[g.nks - 1];
+  g.nE = tet(g.E + 1) - tet(g.e_lo);
+  g.nF = tet(g.F + 1) - tet(g.f_lo);
+  for (int r = 0; r < g.nbs; ++r) {
+    g.ox[r] = g.nX;
+    g.nX += g.nes[r] * g.KF;
+  }
+  g.nbc = kind == KIND_2E_IPIP1 ? 9 : (ip1 ? 3 : 1);
+  g.nkc = ket ? 3 : 1;
+  g.ncomp = g.nbc * g.nkc;
+  g.nca = ncart(la);
+  g.ncb = ncart(lb);
+  g.ncc = ncart(lc);
+  g.ncd = ncart(ld);
+  g.nAo = sph ? nsph(la) : g.nca;
+  g.nBo = sph ? nsph(lb) : g.ncb;
+  g.nCo = sph ? nsph(lc) : g.ncc;
+  g.nDo = sph ? nsph(ld) : g.ncd;
+  g.lij = la + lb + kind_bra_raise(kind);
+  g.lkl = lc + ld + kind_ket_raise(kind);
+  g.nr = (g.lij + g.lkl) / 2 + 1;
+  g.nrt = omega < 0 ? 2 * g.nr : g.nr;
+  // the bra transform is the identity for s and p and for Cartesian output;
+  // the ket needs no transfer with one plain shell
+  const bool bra_c2s = sph && (la > 1 || lb > 1);
+  const bool ket_x = !(three && g.nkc == 1);
+  g.nH1 = g.nca * g.ncb * g.KF;
+  g.nH2 = bra_c2s ? g.nAo * g.nBo * g.KF : 0;
+  g.nH3 = ket_x ? g.nkc * g.nAo * g.nBo * g.ncc * g.ncd : 0;
+  // H3 reuses H1's region unless H2 is H1
+  auto passes = [&](int n) {
+    const int a = bra_c2s ? (g.nH1 > g.nH3 ? g.nH1 : g.nH3) : g.nH1;
+    return n * (a + (bra_c2s ? g.nH2 : g.nH3));
+  };
+  const int PV = 3 * g.nrt * (g.E + 1) * (g.F + 1) + 2 * g.nrt + GEN_PRIM_D;
+  const int ncode = tet((g.E > g.F ? g.E : g.F) + 1);
+  // terms: weights (doubles), packed exponents (ints), starts per component
+  const int ntb = xfer_count(lb), ntk = three ? 1 : xfer_count(ld);
+  const int fixed = ntb + ntk + (ncode + ntb + ntk + g.ncb + g.ncd + 4 + 1) / 2;
+  // a batch of primitive quartets: enough (primitive, direction, root)
+  // recurrences for the lanes, at most 16 KB of tables
+  // (second derivatives of 20 shells: 29.4 ms; 8 KB 31.9 ms, 4 KB 46 ms)
+  g.PB = 1;
+  while (g.PB < 16 && g.PB * 3 * g.nrt < GEN_LANES && (g.PB + 1) * PV <= 2048) ++g.PB;
+  const int walk = g.PB * PV;
+  auto total = [&](int n) {
+    const int p = passes(n);
+    return g.nX + (p > walk ? p : walk) + fixed;
+  };
+  g.nbg = g.nbc;
+  while (g.nbg > 1 && total(g.nbg) > GEN_LDS_TARGET) g.nbg = (g.nbg + 1) / 2;
+  g.in_lds = total(g.nbg) <= GEN_LDS_MAX;
+  const int xl = g.in_lds ? g.nX : 0, pl = g.in_lds ? passes(g.nbg) : 0;
+  g.nblk = g.in_lds ? 0 : g.nX + passes(g.nbg);
+  // block offsets: in LDS or in the wave's global scratch
+  g.oH1 = g.nX;
+  g.oH2 = g.nX + g.nbg * (bra_c2s ? (g.nH1 > g.nH3 ? g.nH1 : g.nH3) : g.nH1);
+  g.oV = xl;
+  g.oP = g.oV + g.PB * 3 * g.nrt * (g.E + 1) * (g.F + 1);
+  g.ou = g.oP + g.PB * GEN_PRIM_D;
+  g.ow = g.ou + g.PB * g.nrt;
+  g.oTb = xl + (pl > walk ? pl : walk);
+  g.oTk = g.oTb + ntb;
+  g.oI = g.oTk + ntk;
+  g.lds = g.oTb + fixed;
+  return g;
+}
+
+// Whether the kernel's tables hold the class.
+inline bool gen_fits(const GenLayout& g) {
+  return g.nE <= GEN_ECAP && g.nF <= GEN_FCAP && 3 * g.nrt * (g.E + 1) * (g.F + 1) <= GEN_VCAP;
+}
+
+}  // namespace mcint

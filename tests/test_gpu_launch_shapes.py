@@ -54,3 +54,36 @@ def test_widened_teams(mc, orc, name, fill):
     ref, _, nz_r = orc.batch(name, q, orc.Basis(m.atm, m.bas, m.env))
     _close(got, ref, f"{name} fill {fill}")
     np.testing.assert_array_equal(nz, nz_r)
+
+
+@pytest.mark.parametrize("name,lmax,n", [("int3c2e_ip1_sph", 4, 40000), ("int3c2e_ip2_cart", 4, 34000),
+                                         ("int2e_ipip1_sph", 1, 33000), ("int2e_ip1ip2_sph", 3, 300)])
+def test_generic_kernel_lists(mc, orc, name, lmax, n):
+    """The generic kernel with one task per wave (short lists) and several
+    (long buckets), blocks in LDS and (f shells) in global scratch."""
+    m = make_molecule("c4" if "3c2e" in name else "c1")
+    rng = np.random.default_rng(8)
+    ls = m.bas[:, 1]
+    orb = np.flatnonzero((ls <= lmax) & (np.arange(m.nbas) < (m.aux_start if m.aux_start >= 0 else m.nbas)))
+    if "3c2e" in name:
+        # few shells: buckets of tens of thousands of tasks
+        orb = np.concatenate([orb[ls[orb] == l][:4] for l in range(4)])
+    elif lmax == 1:
+        orb = np.concatenate([orb[(ls[orb] == l) & (m.bas[orb, 2] == 1)][:6] for l in range(2)])
+    q = rng.choice(orb, (n, 4)).astype(np.int32)
+    if "3c2e" in name:
+        q[:, 2] = rng.integers(m.aux_start, m.nbas, n)
+        q[n // 2:, :2] = orb[:2]
+        q[n // 2:, 2] = m.aux_start + rng.integers(0, 12, n - n // 2)
+    elif lmax == 3:
+        q[:40] = rng.choice(np.flatnonzero(ls == 3), (40, 4))
+    B = mc.Basis(m.atm, m.bas, m.env)
+    got, off, nz = mc.batch(name, q, B)
+    ref, _, nz_r = orc.batch(name, q, orc.Basis(m.atm, m.bas, m.env))
+    # the reference transfers weighted sets per primitive; its own rounding
+    # on a block is relative to the block's largest intermediate
+    for i in range(n):
+        s = slice(off[i], off[i + 1])
+        scale = max(1.0, np.abs(ref[s]).max(initial=0.0))
+        assert np.abs(got[s] - ref[s]).max(initial=0.0) <= 1e-11 * scale + 1e-12, (name, q[i])
+    np.testing.assert_array_equal(nz, nz_r)
