@@ -355,6 +355,17 @@ int mcint_plan_count_primitives(mcint_plan *p, int64_t *per_bucket);
  * (row-major, symmetric).  Asynchronous on hip_stream. */
 int mcint_plan_execute_grad(mcint_plan *p, const double *dm_dev, int nao, double *grad_dev,
                             void *hip_stream);
+/* The same gradient from fewer quartets, by translational invariance: the
+ * four derivatives of a quartet sum to zero, so one atom of every unordered
+ * quartet (refs: the one whose derivatives would cost most) receives minus
+ * the others and no (i, j, k>=l) with i on it is listed.
+ * mcint_gradient_list fills shls (stride 4) and refs (host arrays of cap
+ * entries; cap = 0 only counts) and sets *n; mcint_plan_create_gradient
+ * plans any part of that list for mcint_plan_execute_grad, which then needs
+ * a symmetric density; such a plan stores no blocks (MCINT_ERR_ARG). */
+int mcint_gradient_list(const mcint_basis *b, FINT *shls, FINT *refs, size_t cap, size_t *n);
+int mcint_plan_create_gradient(mcint_plan **p, mcint_basis *b, const FINT *shls, const FINT *refs,
+                               size_t nq, const uint8_t *fp32_flags);
 
 /* Coulomb and exchange matrices fused into the integral kernels: executes
  * an int2e_sph plan over unique quartets (i>=j, k>=l, ij>=kl, each once)

@@ -82,6 +82,10 @@ def lib():
     L.mcint_plan_create_mixed.argtypes = [ctypes.POINTER(vp), vp, ctypes.c_int, ip, ctypes.c_size_t,
                                           ctypes.POINTER(ctypes.c_int64), ctypes.c_void_p,
                                           ctypes.POINTER(ctypes.c_int64)]
+    L.mcint_gradient_list.restype = ctypes.c_int
+    L.mcint_gradient_list.argtypes = [vp, ip, ip, ctypes.c_size_t, ctypes.POINTER(ctypes.c_size_t)]
+    L.mcint_plan_create_gradient.restype = ctypes.c_int
+    L.mcint_plan_create_gradient.argtypes = [ctypes.POINTER(vp), vp, ip, ip, ctypes.c_size_t, vp]
     L.mcint_plan_fp32_tasks.restype = ctypes.c_int64
     L.mcint_plan_fp32_tasks.argtypes = [vp]
     L.mcint_plan_execute.restype = ctypes.c_int
@@ -307,6 +311,18 @@ class DeviceBasis:
         _check(lib().mcint_schwarz(self.handle, nshell, _dp(q)), "mcint_schwarz")
         return q
 
+    def gradient_list(self):
+        """(quartets [n, 4], reference atoms [n]) of the two-electron gradient:
+        (i, j, k >= l) of every quartet except where i sits on the quartet's
+        reference atom, which receives minus the other derivatives."""
+        n = ctypes.c_size_t()
+        _check(lib().mcint_gradient_list(self.handle, None, None, 0, ctypes.byref(n)), "mcint_gradient_list")
+        shls, refs = np.empty((n.value, 4), np.int32), np.empty(n.value, np.int32)
+        if n.value:
+            _check(lib().mcint_gradient_list(self.handle, _ip(shls), _ip(refs), n.value, ctypes.byref(n)),
+                   "mcint_gradient_list")
+        return shls, refs
+
     def close(self):
         if self.handle:
             lib().mcint_basis_destroy(self.handle)
@@ -322,7 +338,8 @@ class DeviceBasis:
 class Plan:
     """mcint_plan over a host list of shell tuples; outputs live on the device."""
 
-    def __init__(self, dbasis: DeviceBasis, name: str, shls, out_offsets=None, fp32_flags=None):
+    def __init__(self, dbasis: DeviceBasis, name: str, shls, out_offsets=None, fp32_flags=None,
+                 grad_refs=None):
         self.dbasis = dbasis
         self.name = name
         shls = np.ascontiguousarray(shls, dtype=np.int32).reshape(-1, 4)
@@ -333,7 +350,18 @@ class Plan:
         if out_offsets is not None:
             self._off = np.ascontiguousarray(out_offsets, dtype=np.int64)
             offp = self._off.ctypes.data_as(ctypes.POINTER(ctypes.c_int64))
-        if fp32_flags is None:
+        if grad_refs is not None:  # part of a DeviceBasis.gradient_list()
+            assert name == "int2e_ip1_sph" and out_offsets is None
+            self._refs = np.ascontiguousarray(grad_refs, dtype=np.int32)
+            assert self._refs.size == self.nq
+            if fp32_flags is not None:
+                self._flags = np.ascontiguousarray(fp32_flags, dtype=np.uint8)
+                assert self._flags.size == self.nq
+            _check(lib().mcint_plan_create_gradient(
+                ctypes.byref(h), dbasis.handle, _ip(shls), _ip(self._refs), self.nq,
+                None if fp32_flags is None else self._flags.ctypes.data_as(ctypes.c_void_p)),
+                "mcint_plan_create_gradient")
+        elif fp32_flags is None:
             _check(lib().mcint_plan_create(ctypes.byref(h), dbasis.handle, INTOR_CODES[name],
                                            _ip(shls), self.nq, offp, ctypes.byref(osz)),
                    "mcint_plan_create")

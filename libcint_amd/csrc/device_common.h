@@ -36,14 +36,21 @@ __host__ __device__ inline double jk_degeneracy(int i, int j, int k, int l) {
          (((i == k && j == l) || (i == l && j == k)) ? 0.5 : 1.0);
 }
 
-// Gradient digest: adds the per-team partials g[k][x] (atom[k] < 0: none)
-// of one block to slot (block % nslot) of the accumulators, one atomic per
-// run of equal atoms and per component.  Call after a barrier that made g
-// and atom visible.
+// Atom that receives minus a task's gradient, -1: none (A.grad_refs).
+__device__ __forceinline__ int grad_ref(const BucketArgs& A, const Task& tk) {
+  return A.grad_refs ? (int)task_out(tk) - 1 : -1;
+}
+
+// Gradient digest: adds the per-team partials g[k][x] of one block to the
+// accumulators of atom[0][k] and subtracts them from those of atom[1][k]
+// (< 0: none), slot block % nslot, one atomic per run of equal atoms and per
+// component.  Call after a barrier that made g and atom visible.
 __device__ __forceinline__ void grad_block_flush(const BucketArgs& A, const double (*g)[3],
-                                                 const int* atom, int nteam) {
-  if (threadIdx.x < 3) {
-    const int c = threadIdx.x;
+                                                 const int* atom0, const int* atom1, int nteam) {
+  if (threadIdx.x < 6) {
+    const bool minus = threadIdx.x >= 3;
+    const int c = minus ? threadIdx.x - 3 : threadIdx.x;
+    const int* atom = minus ? atom1 : atom0;
     double* base = A.grad + (int64_t)(blockIdx.x % A.nslot) * A.grad_stride + c;
     int cur = -1;
     double s = 0.0;
@@ -55,7 +62,7 @@ __device__ __forceinline__ void grad_block_flush(const BucketArgs& A, const doub
         cur = at;
         s = 0.0;
       }
-      s += g[k][c];
+      s += minus ? -g[k][c] : g[k][c];
     }
     if (cur >= 0) atomicAdd(base + 3 * cur, s);
   }

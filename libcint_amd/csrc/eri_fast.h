@@ -1317,7 +1317,7 @@ __global__ void __launch_bounds__(256) eri_ip1_epi_kernel(BasisView Bv, BucketAr
   constexpr int NAo = nout(LA, SPH), NBo = nout(LB, SPH), NCo = nout(LC, SPH), NDo = nout(LD, SPH);
   __shared__ double sm[P::TPB * P::PER];
   __shared__ double s_g[P::TPB][3];
-  __shared__ int s_atom[P::TPB];
+  __shared__ int s_atom[2][P::TPB];
   const int team = threadIdx.x / TE;
   const int tl = threadIdx.x % TE;
   const int64_t t = A.t0 + (int64_t)blockIdx.x * P::TPB + team;
@@ -1483,10 +1483,11 @@ __global__ void __launch_bounds__(256) eri_ip1_epi_kernel(BasisView Bv, BucketAr
       s_g[team][0] = g0;
       s_g[team][1] = g1;
       s_g[team][2] = g2;
-      s_atom[team] = (valid && any) ? Bv.vsh[tk.sh[0]].atom : -1;
+      s_atom[0][team] = (valid && any) ? Bv.vsh[tk.sh[0]].atom : -1;
+      s_atom[1][team] = (valid && any) ? grad_ref(A, tk) : -1;
     }
     __syncthreads();
-    grad_block_flush(A, s_g, s_atom, P::TPB);
+    grad_block_flush(A, s_g, s_atom[0], s_atom[1], P::TPB);
   }
 }
 

@@ -653,11 +653,13 @@ __attribute__((amdgpu_waves_per_eu(3))) eri_generic_kernel(BasisView B, BucketAr
       __syncthreads();
     }
     if (digest) {
-      double* gs = A.grad + (int64_t)(blockIdx.x % A.nslot) * A.grad_stride + 3 * s0.atom;
+      double* gs = A.grad + (int64_t)(blockIdx.x % A.nslot) * A.grad_stride;
+      const int ref = grad_ref(A, tk);
       for (int c = 0; c < 3; ++c) {
         double g = gpart[c];
         for (int off = 1; off < GEN_LANES; off <<= 1) g += __shfl_xor(g, off);
-        if (lane == 0) atomicAdd(gs + c, g);
+        if (lane == 0) atomicAdd(gs + 3 * s0.atom + c, g);
+        if (lane == 0 && ref >= 0) atomicAdd(gs + 3 * ref + c, -g);
       }
     }
   }

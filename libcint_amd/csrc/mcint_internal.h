@@ -142,6 +142,9 @@ struct BucketArgs {
   int nao;
   int nslot;             // gradient accumulator copies (spreads the atomics)
   int grad_stride;
+  // translational invariance: the tasks' output field holds 1 + the atom
+  // that receives minus the sum (no entry differentiates a shell of it)
+  int grad_refs;
   // J/K digest (plain four-centre plans over unique quartets): instead of
   // storing the block, add its six block updates to the half matrices
   // J' (jk_j) and K' (jk_k), nao x nao row-major, density dm

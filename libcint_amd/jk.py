@@ -152,7 +152,7 @@ def energy(dm: torch.Tensor, vj: torch.Tensor, vk: torch.Tensor) -> torch.Tensor
 
 
 def gradient_quartets(nshell: int) -> np.ndarray:
-    """(i, j, k>=l) for all ordered i, j: the list the gradient digest needs."""
+    """(i, j, k>=l) for all ordered i, j: every derivative of the two-electron gradient."""
     ii, jj = np.meshgrid(np.arange(nshell), np.arange(nshell), indexing="ij")
     kk, ll = np.tril_indices(nshell)
     nij, nkl = ii.size, kk.size
@@ -165,8 +165,14 @@ def gradient_quartets(nshell: int) -> np.ndarray:
 
 
 class GradientPlan:
-    """Device plans of the ip1 list (i, j, k >= l) of a basis, reusable for
-    any density: ``run(dm)`` returns dE/dR (natm x 3) of E = 1/2 D J - 1/4 D K."""
+    """Device plans of the gradient's ip1 quartets of a basis, reusable for
+    any symmetric density: ``run(dm)`` returns dE/dR (natm x 3) of
+    E = 1/2 D J - 1/4 D K.
+
+    The four derivatives of a quartet sum to zero, so the plans hold (i, j,
+    k >= l) only where i is not on the quartet's costliest atom, which takes
+    minus the others (``DeviceBasis.gradient_list``): at most 3/4 of the
+    derivatives, fewer where shells of a quartet share atoms."""
 
     def __init__(self, basis: Basis, natm: int, chunk: int = 64_000_000, device="cuda",
                  fp32_threshold: float = 0.0, dmax: float = 1.0):
@@ -174,14 +180,14 @@ class GradientPlan:
         self.natm = natm
         self.nao = nao_sph(basis)
         self.db = DeviceBasis(basis)
-        q_all = gradient_quartets(basis.nbas)
+        q_all, refs = self.db.gradient_list()
         self.nquartets = q_all.shape[0]
         flags = None
         if fp32_threshold > 0:
             # the digest weighs each quartet by products of two density
             # elements: FP32 where sqrt((ij|ij)) sqrt((kl|kl)) dmax^2 is small
             flags = fp32_quartet_flags(self.db, q_all, np.array([dmax * dmax]), fp32_threshold)
-        self.plans = [Plan(self.db, "int2e_ip1_sph", q_all[c0:c0 + chunk],
+        self.plans = [Plan(self.db, "int2e_ip1_sph", q_all[c0:c0 + chunk], grad_refs=refs[c0:c0 + chunk],
                            fp32_flags=None if flags is None else flags[c0:c0 + chunk])
                       for c0 in range(0, q_all.shape[0], chunk)]
 

@@ -87,3 +87,55 @@ def test_generic_kernel_lists(mc, orc, name, lmax, n):
         scale = max(1.0, np.abs(ref[s]).max(initial=0.0))
         assert np.abs(got[s] - ref[s]).max(initial=0.0) <= 1e-11 * scale + 1e-12, (name, q[i])
     np.testing.assert_array_equal(nz, nz_r)
+
+
+def _grad_full(mc, B, m, dm):
+    """The gradient digest over every (i, j, k >= l)."""
+    import torch
+    from libcint_amd import jk
+    db = mc.DeviceBasis(B)
+    plan = mc.Plan(db, "int2e_ip1_sph", jk.gradient_quartets(m.nbas))
+    d = torch.tensor(dm, device="cuda")
+    g = torch.zeros((m.natm, 3), dtype=torch.float64, device="cuda")
+    plan.execute_grad(d.data_ptr(), dm.shape[0], g.data_ptr())
+    torch.cuda.synchronize()
+    plan.close()
+    db.close()
+    return g.cpu().numpy()
+
+
+def _gc_basis(m):
+    """m with its first s shell given a second contraction column."""
+    bas, env = m.bas.copy(), m.env
+    s = int(np.flatnonzero((bas[:, 1] == 0) & (bas[:, 2] > 1))[0])
+    n, pc = int(bas[s, 2]), int(bas[s, 6])
+    col = env[pc:pc + n]
+    bas[s, 3], bas[s, 6] = 2, len(env)
+    return bas, np.concatenate([env, col, col[::-1]])
+
+
+@pytest.mark.parametrize("case", ["atom", "pair", "mol", "general"])
+def test_gradient_list(mc, case):
+    """Translational invariance: the reduced list's gradient equals the full
+    list's (the same sums but for rounding, 1e-10 of the largest), holds no
+    derivative on a reference atom, and its plan stores no blocks."""
+    from libcint_amd import jk
+    from libcint_amd.synthetic import random_density, subset
+    m = subset(make_molecule("c3"), {"atom": 1, "pair": 2, "mol": 4, "general": 3}[case])
+    bas, env = _gc_basis(m) if case == "general" else (m.bas, m.env)
+    B = mc.Basis(m.atm, bas, env)
+    dm = random_density(jk.nao_sph(B), seed=4)
+    gp = jk.GradientPlan(B, m.natm)
+    got = gp.run(dm).cpu().numpy()
+    q, refs = gp.db.gradient_list()
+    assert gp.nquartets == len(q) == len(refs)
+    assert len(q) <= 3 * len(jk.gradient_quartets(m.nbas)) // 4
+    atom = bas[:, 0]
+    assert (atom[q[:, 0]] != refs).all() and (q[:, 2] >= q[:, 3]).all()
+    assert (atom[q] == refs[:, None]).any(axis=1).all()
+    for plan in gp.plans:
+        with pytest.raises(mc.McintError):
+            plan.execute(1 << 12, graph=False)
+    gp.close()
+    ref = _grad_full(mc, B, m, dm)
+    np.testing.assert_allclose(got, ref, rtol=0, atol=1e-10 * max(1.0, np.abs(ref).max()))
