@@ -461,6 +461,7 @@ struct Bucket {
   int lanes;  // lanes per task at launch: team, or widened to fill the chip
   int mode;  // 0 generic, 1 fast (single chunk), 2 chunked
   int fp32;  // recurrences in FP32 (mode 1 only)
+  int mm;    // generic path on the matrix kernel: waves per task (0: not)
   int64_t t0, t1;
   int64_t sstride;  // scratch doubles per task (0: blocks in LDS)
   double cost;      // estimated work (balances the concurrent graph branches)
@@ -492,6 +493,10 @@ double bucket_cost(int kind, int mode, int la, int lb, int lc, int ld, int64_t n
 // largest c1 bucket, 695,543 (fd|dp) quartets x 736 doubles, fits), 16 GiB
 // over four branches, allocated only up to what the plan needs.
 constexpr int64_t GEN_SCRATCH_DOUBLES = 512ll << 20;
+// Bound of a plan's transfer matrices (doubles, 2 GiB): 126 KB for a d pair's
+// second derivative, so 17 000 such pairs; beyond it the generic path forms
+// its transfers term by term.
+constexpr int64_t XFER_DOUBLES = 256ll << 20;
 // copies of the gradient accumulators (spreads the digest's atomics)
 constexpr int GRAD_SLOTS = 64;
 
@@ -616,6 +621,10 @@ struct mcint_plan {
   int64_t scratch_size = 0;
   int* flags_d = nullptr;
   int64_t flags_size = 0;
+  // generic path: transfer matrices of its pairs, and their offsets by
+  // ordered virtual pair (bra, then ket)
+  double* xfer_d = nullptr;
+  int64_t* xfer_off_d = nullptr;
   double* gslots_d = nullptr;  // gradient digest accumulators
   double* jk_d = nullptr;      // J', K' half matrices of the fused J/K digest
   int64_t jk_n = 0;            // nao * nao they hold
@@ -652,6 +661,8 @@ static void plan_free(mcint_plan* p) {
   dfree(p->flags_d);
   dfree(p->gslots_d);
   dfree(p->jk_d);
+  dfree(p->xfer_d);
+  dfree(p->xfer_off_d);
   delete p;
 }
 
@@ -1061,16 +1072,23 @@ static int plan_create_impl(mcint_plan** out, mcint_basis* b, int intor, const F
     bk.cost = bucket_cost(kind, bk.mode, bk.la, bk.lb, bk.lc, bk.ld, np, bk.t1 - bk.t0);
     if (bk.fp32) p->stats_fp32 += bk.t1 - bk.t0;
     bk.sstride = 0;
+    bk.mm = 0;
     if (bk.mode == 2) {
       bk.sstride = chunked_block_doubles(kind, bk.la, bk.lb, bk.lc, bk.ld);
     } else if (bk.mode == 0) {
       const GenLayout G = gen_layout(kind, sph, bk.la, bk.lb, bk.lc, bk.ld, b->omega);
+      // four waves per task where a task holds many primitive quartets or the
+      // bucket is too short to give every SIMD a wave
+      const int64_t n = bk.t1 - bk.t0;
+      const int waves = np >= MM_WAVES_PRIMS * n || n < 1024 ? 4 : 1;
+      for (int w = waves; w >= 1 && !bk.mm; w -= 3)
+        bk.mm = mm_layout(kind, sph, bk.la, bk.lb, bk.lc, bk.ld, b->omega, w).waves;
       if (!gen_fits(G)) {
         plan_free(p);
         set_err("mcint_plan_create: angular momentum beyond the generic kernel's tables");
         return MCINT_ERR_UNSUPPORTED;
       }
-      bk.sstride = G.nblk;
+      bk.sstride = bk.mm ? 0 : G.nblk;
     }
     p->stats[bk.mode == 0 ? 3 : 2] += bk.t1 - bk.t0;
     // runs of groups: the launch (same lanes and kernel) and the bucket
@@ -1099,6 +1117,38 @@ static int plan_create_impl(mcint_plan** out, mcint_basis* b, int intor, const F
                            p->buckets.back().team == bk.team);
     p->buckets.back().lanes = bk.team;
   }
+  // transfer matrices of the generic path's pairs: sizes, offsets
+  const int nv = b->nv;
+  std::vector<XferItem> xitems;
+  std::vector<int64_t> xoff;
+  int64_t xsize = 0;
+  for (const Bucket& bk : p->launches) {
+    if (!bk.mm) continue;
+    if (xoff.empty()) xoff.assign(2 * (size_t)nv * nv, -1);
+    const GenLayout G = mm_layout(kind, sph, bk.la, bk.lb, bk.lc, bk.ld, b->omega, bk.mm);
+    auto need = [&](int64_t at, int s, int s2, int ket, int rows, int ks) {
+      if (xoff[at] >= 0) return;
+      xoff[at] = xsize;
+      xitems.push_back(XferItem{s, s2, ket, rows, ks, xsize});
+      xsize += (int64_t)rows * ks * 64;
+    };
+    for (int64_t t = bk.t0; t < bk.t1; ++t) {
+      const int16_t* s = sorted[t].sh;
+      const int s3 = kind_three(kind) ? s[2] : s[3];
+      need((int64_t)s[0] * nv + s[1], s[0], s[1], 0, G.RT, G.KS);
+      need((int64_t)nv * nv + (int64_t)s[2] * nv + s3, s[2], s3, 1, G.CT2, G.KS2);
+    }
+  }
+  if (xsize > XFER_DOUBLES) {
+    xitems.clear();
+    for (auto* list : {&p->buckets, &p->launches})
+      for (Bucket& bk : *list) {
+        if (!bk.mm) continue;
+        bk.mm = 0;
+        bk.sstride = gen_layout(kind, sph, bk.la, bk.lb, bk.lc, bk.ld, b->omega).nblk;
+      }
+  }
+  timer.mark("transfer matrices");
   for (const auto* list : {&p->buckets, &p->launches})
     for (const Bucket& bk : *list) {
       if (bk.mode == 1) continue;
@@ -1111,7 +1161,6 @@ static int plan_create_impl(mcint_plan** out, mcint_basis* b, int intor, const F
   p->stats[1] = (int64_t)p->buckets.size();
 
   // ---- primitive-pair data of every pair the tasks touch ----------------
-  const int nv = b->nv;
   std::vector<uint8_t> used((size_t)nv * nv, 0);
   // read before writing: stores to lines other threads read would bounce
   // the lines between cores
@@ -1167,8 +1216,21 @@ static int plan_create_impl(mcint_plan** out, mcint_basis* b, int intor, const F
   if (e == hipSuccess)
     e = launch_pairdata(b->vsh_d, b->env_d, nv, pairs_d, (int)(pairs.size() / 2), p->pair_off_d,
                         p->pair_ld_d, pp_tmp, p->pp_d, p->pp_pos_d, nullptr);
+  XferItem* items_d = nullptr;
+  if (!xitems.empty()) {
+    if (e == hipSuccess) e = dalloc(&items_d, xitems.size());
+    if (e == hipSuccess) e = dalloc(&p->xfer_d, (size_t)xsize);
+    if (e == hipSuccess) e = dalloc(&p->xfer_off_d, xoff.size());
+    if (e == hipSuccess)
+      e = hipMemcpy(items_d, xitems.data(), xitems.size() * sizeof(XferItem), hipMemcpyHostToDevice);
+    if (e == hipSuccess)
+      e = hipMemcpy(p->xfer_off_d, xoff.data(), xoff.size() * sizeof(int64_t), hipMemcpyHostToDevice);
+    if (e == hipSuccess)
+      e = launch_xfer(b->vsh_d, kind, sph, items_d, (int)xitems.size(), p->xfer_d, nullptr);
+  }
   if (e == hipSuccess) e = hipDeviceSynchronize();
   timer.mark("device upload, pair data");
+  dfree(items_d);
   dfree(pairs_d);
   dfree(pp_tmp);
   if (e != hipSuccess) {
@@ -1415,6 +1477,14 @@ static int64_t slice_tasks(const Bucket& bk, const ScratchView& S) {
   return n;
 }
 
+static hipError_t generic_launch(const mcint_plan* p, const Bucket& bk, const BasisView& B,
+                                 const BucketArgs& A, hipStream_t stream) {
+  if (!bk.mm) return launch_generic(B, A, stream);
+  const int64_t nn = (int64_t)p->b->nv * p->b->nv;
+  return launch_matrix(B, A, XferView{p->xfer_d, p->xfer_off_d, p->xfer_off_d + nn, p->b->nv}, bk.mm,
+                       stream);
+}
+
 static int bucket_launch(mcint_plan* p, const Bucket& bk, double* out, FINT* not0,
                          hipStream_t stream, const ScratchView& S) {
   if (p->grad_refs) {
@@ -1444,7 +1514,7 @@ static int bucket_launch(mcint_plan* p, const Bucket& bk, double* out, FINT* not
     if (bk.mode == 2)
       HIPCHK(launch_chunked(B, A, stream));
     else
-      HIPCHK(launch_generic(B, A, stream));
+      HIPCHK(generic_launch(p, bk, B, A, stream));
   }
   return MCINT_OK;
 }
@@ -1560,7 +1630,7 @@ extern "C" int mcint_plan_execute_grad(mcint_plan* p, const double* dm_dev, int 
       if (bk.mode == 2)
         HIPCHK(launch_chunked(B, A, s));
       else
-        HIPCHK(launch_generic(B, A, s));
+        HIPCHK(generic_launch(p, bk, B, A, s));
     }
     return MCINT_OK;
   };
@@ -1627,7 +1697,7 @@ extern "C" int mcint_plan_execute_jk(mcint_plan* p, const double* dm_dev, int na
       if (bk.mode == 2)
         HIPCHK(launch_chunked(B, A, s));
       else
-        HIPCHK(launch_generic(B, A, s));
+        HIPCHK(generic_launch(p, bk, B, A, s));
     }
     return MCINT_OK;
   };

@@ -52,6 +52,15 @@ struct GenLayout {
   // tables in the same space as the passes, the transfer terms, the codes
   int PB, nbg, oH1, oH2, oV, oP, ou, ow, oTb, oTk, oI;
   int lds;          // doubles of LDS
+  // matrix kernel (mm_layout): Y = (bra matrix) X in tiles of 16 rows, then
+  // block = Y (ket matrix)^T; k steps of 4
+  int waves;            // waves per task, 0: the class does not fit
+  int nbu;              // distinct bra components (ipip1: p <= q)
+  int nrow, ncol;       // rows and columns of the block
+  int RT, KS, CT1;      // bra: row tiles, k steps, column tiles (of KF)
+  int CT2, KS2, YS;     // ket: column tiles, k steps, row stride of Y
+  int nXz;              // doubles of X with its rows padded to 4
+  int spread;           // lanes share a component's primitive quartets
   int in_lds;       // blocks in LDS (else in global scratch, nblk per wave)
   int64_t nblk;     // doubles of global scratch per wave
 };
@@ -169,6 +178,67 @@ inline GenLayout gen_layout(int kind, int sph, int la, int lb, int lc, int ld, d
   g.lds = g.oTb + fixed;
   return g;
 }
+
+// Primitive quartets per task from which the matrix kernel takes four waves
+// per task instead of one.
+constexpr int MM_WAVES_PRIMS = 24;
+
+// Layout of the matrix kernel: X, then the walk's tables, each wave's Y and
+// the partial sums of shared components in one space, then the codes.
+inline GenLayout mm_layout(int kind, int sph, int la, int lb, int lc, int ld, double omega, int waves) {
+  GenLayout g = gen_layout(kind, sph, la, lb, lc, ld, omega);
+  const bool three = kind_three(kind);
+  const int threads = 64 * waves;
+  int R = 0;
+  for (int r = 0; r < g.nbs; ++r) R += g.nes[r];
+  g.nbu = kind == KIND_2E_IPIP1 ? 6 : g.nbc;
+  g.nrow = g.nbu * g.nAo * g.nBo;
+  g.ncol = g.nkc * g.nCo * (three ? 1 : g.nDo);
+  g.RT = (g.nrow + 15) / 16;
+  g.KS = (R + 3) / 4;
+  g.CT1 = (g.KF + 15) / 16;
+  g.CT2 = (g.ncol + 15) / 16;
+  g.KS2 = (g.KF + 3) / 4;
+  g.YS = g.CT1 * 16 + 1;
+  g.nXz = g.KS * 4 * g.KF;
+  g.spread = 2 * g.nE * g.nF <= threads;
+  // a batch: enough (primitive, direction, root) recurrences for the lanes
+  const int VT = 3 * g.nrt * (g.E + 1) * (g.F + 1);
+  const int PV = VT + 2 * g.nrt + GEN_PRIM_D;
+  g.PB = 1;
+  while (g.PB < 16 * waves && g.PB * 3 * g.nrt < threads && (g.PB + 1) * PV <= (waves > 1 ? 4096 : 2048)) ++g.PB;
+  int space = g.PB * PV;
+  if (waves * 16 * g.YS > space) space = waves * 16 * g.YS;
+  if (g.spread && 5 * threads > space) space = 5 * threads;
+  const int ncode = tet((g.E > g.F ? g.E : g.F) + 1);
+  g.oV = g.nXz;
+  g.oP = g.oV + g.PB * VT;
+  g.ou = g.oP + g.PB * GEN_PRIM_D;
+  g.ow = g.ou + g.PB * g.nrt;
+  g.oI = g.nXz + space;
+  g.lds = g.oI + (ncode + g.nrow + g.ncol + 2 * waves + 1) / 2;
+  g.waves = g.lds <= GEN_LDS_MAX ? waves : 0;
+  return g;
+}
+
+// One matrix to lay out: the bra matrix of the virtual pair (a, b) or the
+// ket matrix of (a, b) (three-centre kinds: b = a, no transfer), at off.
+struct XferItem {
+  int a, b, ket, rows, ks;  // rows: tiles of 16; ks: k steps of 4
+  int64_t off;
+};
+// Matrices of a plan's pairs, by ordered virtual pair.
+struct XferView {
+  const double* m;
+  const int64_t* bra;
+  const int64_t* ket;
+  int nv;
+};
+hipError_t launch_xfer(const VShell* vsh, int kind, int sph, const XferItem* items, int n, double* m,
+                       hipStream_t stream);
+// The matrix kernel on waves per task (1 or 4; mm_layout(..., waves).waves != 0).
+hipError_t launch_matrix(const BasisView& B, const BucketArgs& A, const XferView& X, int waves,
+                         hipStream_t stream);
 
 // Whether the kernel's tables hold the class.
 inline bool gen_fits(const GenLayout& g) {

@@ -139,3 +139,44 @@ def test_gradient_list(mc, case):
     gp.close()
     ref = _grad_full(mc, B, m, dm)
     np.testing.assert_allclose(got, ref, rtol=0, atol=1e-10 * max(1.0, np.abs(ref).max()))
+
+
+@pytest.mark.parametrize("omega", [0.0, 0.4, -0.4])
+@pytest.mark.parametrize("name", ["int2e_ipip1_sph", "int2e_ipip1_cart", "int2e_ip1ip2_sph", "int2e_ip1ip2_cart",
+                                  "int3c2e_ip1_sph", "int3c2e_ip2_cart", "int2c2e_sph", "int2e_cart"])
+def test_matrix_kernel(mc, orc, name, omega):
+    """Plans on the matrix kernel: every order of s, p, d (and one f, one g)
+    shells, one and four waves per task (buckets below and above 1024 tasks),
+    1 to 4096 primitive quartets, all operators."""
+    if name == "int2e_cart" and omega >= 0:
+        pytest.skip("register kernels serve it")
+    m = make_molecule("c4" if "c2e" in name else "c1")
+    rng = np.random.default_rng(12)
+    ls, three = m.bas[:, 1], "c2e" in name
+    ns = m.aux_start if m.aux_start >= 0 else m.nbas
+    orb = np.arange(ns)
+    few = [orb[ls[:ns] == l][:5] for l in range(4)]
+    deep = [orb[(ls[:ns] == l) & (m.bas[:ns, 2] > 1)][:1] for l in range(2)]
+    pool = np.concatenate(few[:3] + deep)
+    q = rng.choice(pool, (260, 4)).astype(np.int32)
+    q[:4, 0] = few[3][0]
+    q[4:8, 2] = few[3][0]
+    short = rng.choice(np.concatenate([orb[(ls[:ns] == l) & (m.bas[:ns, 2] == 1)][:4] for l in range(2)]), (1, 4))
+    q = np.concatenate([q, np.repeat(short, 1100, axis=0)]).astype(np.int32)
+    if three:
+        aux = np.arange(m.aux_start, m.nbas)
+        q[:, 2] = rng.choice(aux, len(q))
+        q[260:, 2] = aux[ls[aux] == 0][0]
+        if name.startswith("int2c2e"):
+            q[:, 0], q[:, 1] = rng.choice(aux, len(q)), rng.choice(aux, len(q))
+        q[:, 3] = 0
+    env = m.env.copy()
+    env[8] = omega
+    got, off, nz = mc.batch(name, q, mc.Basis(m.atm, m.bas, env))
+    ref, _, nz_r = orc.batch(name, q, orc.Basis(m.atm, m.bas, env))
+    # as for the generic kernel: relative to the block's largest element
+    for i in range(len(q)):
+        s = slice(off[i], off[i + 1])
+        scale = max(1.0, np.abs(ref[s]).max(initial=0.0))
+        assert np.abs(got[s] - ref[s]).max(initial=0.0) <= 1e-11 * scale + 1e-12, (name, omega, q[i])
+    np.testing.assert_array_equal(nz, nz_r)
