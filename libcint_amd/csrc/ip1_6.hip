@@ -1,6 +1,6 @@
-// i-derivative chunked-path instantiations, group 6 (see eri_fast.h).
+// i-derivative chunked-path instantiations, group 6 (see ip1_wave.h).
 #include "device_common.h"
-#include "eri_fast.h"
+#include "ip1_wave.h"
 
 namespace mcint {
 MCINT_IP1_GROUP6(MCINT_IP1_DEFINE)

@@ -180,3 +180,48 @@ def test_matrix_kernel(mc, orc, name, omega):
         scale = max(1.0, np.abs(ref[s]).max(initial=0.0))
         assert np.abs(got[s] - ref[s]).max(initial=0.0) <= 1e-11 * scale + 1e-12, (name, omega, q[i])
     np.testing.assert_array_equal(nz, nz_r)
+
+
+@pytest.mark.parametrize("name", ["int2e_ip1_sph", "int2e_ip1_cart", "int2e_ip2_sph"])
+@pytest.mark.parametrize("omega", [0.0, 0.3])
+def test_derivative_wave_kernel(mc, name, omega):
+    """Derivative classes on the wave kernel (every class that has one, one to
+    1296 primitive quartets, odd counts per wave) against the chunk kernels:
+    the same sums in another order."""
+    m = make_molecule("c3")
+    ls, env = m.bas[:, 1], m.env.copy()
+    env[8] = omega
+    rng = np.random.default_rng(3)
+    pool = np.concatenate([np.flatnonzero(ls == l)[:6] for l in range(3)])
+    q = rng.choice(pool, (1501, 4)).astype(np.int32)
+    out = []
+    old = mc.tune(mc.TUNE_WAVE_KERNELS, 0)
+    try:
+        for mode in (0, 2):
+            mc.tune(mc.TUNE_WAVE_KERNELS, mode)
+            out.append(mc.batch(name, q, mc.Basis(m.atm, m.bas, env)))
+    finally:
+        mc.tune(mc.TUNE_WAVE_KERNELS, old)
+    (a, _, nza), (b, _, nzb) = out
+    scale = max(1.0, np.abs(a).max())
+    assert np.abs(a - b).max() <= 1e-12 * scale
+    np.testing.assert_array_equal(nza, nzb)
+
+
+def test_gradient_wave_kernel(mc):
+    """The gradient through wave and chunk kernels, waves taking many quartets."""
+    from libcint_amd import jk
+    from libcint_amd.synthetic import random_density, subset
+    m = subset(make_molecule("c3"), 4)
+    B = mc.Basis(m.atm, m.bas, m.env)
+    dm = random_density(m.nao_sph(), seed=9)
+    out = []
+    old = mc.tune(mc.TUNE_WAVE_KERNELS, 0)
+    try:
+        for mode in (0, 1, 2):
+            mc.tune(mc.TUNE_WAVE_KERNELS, mode)
+            out.append(jk.nuclear_gradient(B, dm, m.natm).cpu().numpy())
+    finally:
+        mc.tune(mc.TUNE_WAVE_KERNELS, old)
+    for g in out[1:]:
+        np.testing.assert_allclose(g, out[0], rtol=0, atol=1e-11 * max(1.0, np.abs(out[0]).max()))
