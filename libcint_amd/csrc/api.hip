@@ -499,6 +499,12 @@ constexpr int64_t GEN_SCRATCH_DOUBLES = 512ll << 20;
 constexpr int64_t XFER_DOUBLES = 256ll << 20;
 // copies of the gradient accumulators (spreads the digest's atomics)
 constexpr int GRAD_SLOTS = 64;
+// Copies of J', K' that the fused digest adds into, block b to copy b % 8, in
+// at most 256 MiB (1448 AOs; beyond, one).  Workgroups go to the eight XCDs in
+// turn, so a copy's lines stay in one XCD's L2 instead of moving between
+// eight: the atomics, not the sums, were the digest's cost.
+constexpr int JK_SLOTS = 8;
+constexpr int64_t JK_SLOT_DOUBLES = 32ll << 20;
 
 // default of g_fill_lanes: 256 CUs x 4 SIMDs x 2 waves
 constexpr int FILL_LANES = 1 << 17;
@@ -627,7 +633,7 @@ struct mcint_plan {
   int64_t* xfer_off_d = nullptr;
   double* gslots_d = nullptr;  // gradient digest accumulators
   double* jk_d = nullptr;      // J', K' half matrices of the fused J/K digest
-  int64_t jk_n = 0;            // nao * nao they hold
+  int64_t jk_n = 0;            // doubles they hold
   int64_t stats[6] = {0, 0, 0, 0, 0, 0};
   int64_t stats_fp32 = 0;
   // per-branch scratch: scratch_d / flags_d hold scratch_nbr regions of
@@ -1417,7 +1423,7 @@ static BucketArgs bucket_args(const mcint_plan* p, const Bucket& bk, double* out
   A.grad = nullptr;
   A.nao = 0;
   A.nslot = 1;
-  A.grad_stride = 0;
+  A.slot_stride = 0;
   A.grad_refs = 0;
   A.jk_j = nullptr;
   A.jk_k = nullptr;
@@ -1611,15 +1617,16 @@ extern "C" int mcint_plan_execute_grad(mcint_plan* p, const double* dm_dev, int 
   // per-block partial sums go to GRAD_SLOTS copies of the accumulators
   // (block % GRAD_SLOTS), reduced into grad_dev at the end
   const int n = 3 * p->b->natm;
-  if (!p->gslots_d) HIPCHK(dalloc(&p->gslots_d, (size_t)GRAD_SLOTS * n));
-  HIPCHK(hipMemsetAsync(p->gslots_d, 0, sizeof(double) * GRAD_SLOTS * n, stream));
+  const int64_t stride = (n + 15) & ~15;  // whole cache lines
+  if (!p->gslots_d) HIPCHK(dalloc(&p->gslots_d, (size_t)(GRAD_SLOTS * stride)));
+  HIPCHK(launch_zero(p->gslots_d, GRAD_SLOTS * stride, stream));
   auto launch = [&](const Bucket& bk, hipStream_t s, const ScratchView& S) -> int {
     BucketArgs A = bucket_args(p, bk, nullptr, nullptr);
     A.dm = dm_dev;
     A.grad = p->gslots_d;
     A.nao = nao;
     A.nslot = GRAD_SLOTS;
-    A.grad_stride = n;
+    A.slot_stride = stride;
     A.grad_refs = p->grad_refs;
     A.scratch = S.blocks;
     A.flags = S.flags;
@@ -1640,7 +1647,7 @@ extern "C" int mcint_plan_execute_grad(mcint_plan* p, const double* dm_dev, int 
     for (const Bucket& bk : p->launches)
       if (const int st = launch(bk, stream, plan_scratch(p))) return st;
   }
-  HIPCHK(launch_grad_reduce(p->gslots_d, GRAD_SLOTS, n, grad_dev, stream));
+  HIPCHK(launch_grad_reduce(p->gslots_d, GRAD_SLOTS, stride, n, grad_dev, stream));
   return MCINT_OK;
 }
 
@@ -1668,15 +1675,18 @@ extern "C" int mcint_plan_execute_jk(mcint_plan* p, const double* dm_dev, int na
   const int nbr = std::max(1, std::min<int>(g_graph_branches, (int)p->launches.size()));
   if (const int st = ensure_scratch(p, nbr)) return st;
   const int64_t nn = (int64_t)nao * nao;
-  if (p->jk_n < nn) {
+  const int64_t stride = (2 * nn + 15) & ~int64_t(15);  // whole cache lines
+  const int slots = JK_SLOTS * stride <= JK_SLOT_DOUBLES ? JK_SLOTS : 1;
+  if (p->jk_n < slots * stride) {
     if (p->jk_d) HIPCHK(hipDeviceSynchronize());
     dfree(p->jk_d);
-    HIPCHK(dalloc(&p->jk_d, (size_t)(2 * nn)));
-    p->jk_n = nn;
+    p->jk_n = 0;
+    HIPCHK(dalloc(&p->jk_d, (size_t)(slots * stride)));
+    p->jk_n = slots * stride;
   }
   double* Jp = vj_dev ? p->jk_d : nullptr;
   double* Kp = vk_dev ? p->jk_d + nn : nullptr;
-  HIPCHK(launch_zero(p->jk_d, 2 * nn, stream));
+  HIPCHK(launch_zero(p->jk_d, slots * stride, stream));
   const BasisView B = plan_view(p);
   auto launch = [&](const Bucket& bk, hipStream_t s, const ScratchView& S) -> int {
     BucketArgs A = bucket_args(p, bk, nullptr, nullptr);
@@ -1684,6 +1694,8 @@ extern "C" int mcint_plan_execute_jk(mcint_plan* p, const double* dm_dev, int na
     A.nao = nao;
     A.jk_j = Jp;
     A.jk_k = Kp;
+    A.nslot = slots;
+    A.slot_stride = stride;
     A.scratch = S.blocks;
     A.flags = S.flags;
     if (bk.mode == 1) {
@@ -1707,8 +1719,8 @@ extern "C" int mcint_plan_execute_jk(mcint_plan* p, const double* dm_dev, int na
     for (const Bucket& bk : p->launches)
       if (const int st = launch(bk, stream, plan_scratch(p))) return st;
   }
-  if (vj_dev) HIPCHK(launch_symmetrize(Jp, vj_dev, nao, stream));
-  if (vk_dev) HIPCHK(launch_symmetrize(Kp, vk_dev, nao, stream));
+  if (vj_dev) HIPCHK(launch_symmetrize(Jp, vj_dev, nao, slots, stride, stream));
+  if (vk_dev) HIPCHK(launch_symmetrize(Kp, vk_dev, nao, slots, stride, stream));
   return MCINT_OK;
 }
 
@@ -1884,8 +1896,8 @@ extern "C" int mcint_jk_plan_execute(mcint_jk_plan* j, const double* eri_dev, co
     HIPCHK(launch_jk_grouped(j->shls_d, j->off_d, j->rows_q_d, j->rows_ptr_d, j->nrows, j->rows_lds,
                              j->cols_q_d, j->cols_ptr_d, j->ncols, eri_dev, j->b->ao_loc_d, dm_dev,
                              j->nao, Jp, Kp, stream));
-  if (Jp) HIPCHK(launch_symmetrize(Jp, vj_dev, j->nao, stream));
-  if (Kp) HIPCHK(launch_symmetrize(Kp, vk_dev, j->nao, stream));
+  if (Jp) HIPCHK(launch_symmetrize(Jp, vj_dev, j->nao, 1, 0, stream));
+  if (Kp) HIPCHK(launch_symmetrize(Kp, vk_dev, j->nao, 1, 0, stream));
   return MCINT_OK;
 }
 

@@ -36,6 +36,11 @@ __host__ __device__ inline double jk_degeneracy(int i, int j, int k, int l) {
          (((i == k && j == l) || (i == l && j == k)) ? 0.5 : 1.0);
 }
 
+// This block's copy of the digest accumulators.
+__device__ __forceinline__ int64_t slot_offset(const BucketArgs& A) {
+  return (int64_t)(blockIdx.x % A.nslot) * A.slot_stride;
+}
+
 // Atom that receives minus a task's gradient, -1: none (A.grad_refs).
 __device__ __forceinline__ int grad_ref(const BucketArgs& A, const Task& tk) {
   return A.grad_refs ? (int)task_out(tk) - 1 : -1;
@@ -51,7 +56,7 @@ __device__ __forceinline__ void grad_block_flush(const BucketArgs& A, const doub
     const bool minus = threadIdx.x >= 3;
     const int c = minus ? threadIdx.x - 3 : threadIdx.x;
     const int* atom = minus ? atom1 : atom0;
-    double* base = A.grad + (int64_t)(blockIdx.x % A.nslot) * A.grad_stride + c;
+    double* base = A.grad + slot_offset(A) + c;
     int cur = -1;
     double s = 0.0;
     for (int k = 0; k < nteam; ++k) {

@@ -699,8 +699,8 @@ eri_fast_kernel(BasisView Bv, BucketArgs A) {
         }
       });
     }
-    double* __restrict__ Jp = A.jk_j;
-    double* __restrict__ Kp = A.jk_k;
+    double* __restrict__ Jp = A.jk_j ? A.jk_j + slot_offset(A) : nullptr;
+    double* __restrict__ Kp = A.jk_k ? A.jk_k + slot_offset(A) : nullptr;
     sfor<M>([&](auto I) {
       constexpr int m = decltype(I)::value;
       constexpr int r = m < O1 ? 0 : m < O2 ? 1 : m < O3 ? 2 : m < O4 ? 3 : m < O5 ? 4 : 5;
@@ -1242,7 +1242,7 @@ __global__ void __launch_bounds__(256) eri_epi_jk_kernel(BasisView Bv, BucketArg
     const int o0 = r == 0 ? 0 : r == 1 ? Q::O1 : r == 2 ? Q::O2 : r == 3 ? Q::O3 : r == 4 ? Q::O4 : Q::O5;
     const int ncol = r == 0 ? Q::NBo : (r == 1 || r == 3 || r == 5) ? Q::NDo : Q::NCo;
     const int i = (m - o0) / ncol, j = (m - o0) % ncol;
-    atomicAdd(dst + (rs[r] + i) * N + cs[r] + j, v);
+    atomicAdd(dst + slot_offset(A) + (rs[r] + i) * N + cs[r] + j, v);
   }
 }
 
@@ -1252,11 +1252,8 @@ __global__ void __launch_bounds__(256) eri_epi_jk_kernel(BasisView Bv, BucketArg
 //   (d/dA_x a b| = a_x (a-1_x, b| - (a+1_x, b|_2a_i        (bra transfers
 //     on the lowered and the 2 a_i-weighted raised sets, then spherical a,b)
 //   |c d) <- |f0] transfer, spherical c,d;
-// then either the store of the three component blocks (comp outermost,
-// libcint's layout) or, with A.dm set, the gradient digest
-//   g_x += (d/dA_x a b|c d) fkl [-2 D_ab D_cd + (D_ac D_bd + D_ad D_bc)/2]
-// summed per block over runs of equal atoms into slot (block % nslot) of
-// the gradient accumulators.
+// then the store of the three component blocks (comp outermost, libcint's
+// layout).  The gradient digest is ip1_wave.h's.
 // ---------------------------------------------------------------------
 template <int LA, int LB, int LC, int LD, bool SPH = true>
 struct Ip1EpiCfg {
@@ -1316,13 +1313,10 @@ __global__ void __launch_bounds__(256) eri_ip1_epi_kernel(BasisView Bv, BucketAr
   constexpr int NA = C::NA, NB = C::NB, NC = C::NC, ND = C::ND;
   constexpr int NAo = nout(LA, SPH), NBo = nout(LB, SPH), NCo = nout(LC, SPH), NDo = nout(LD, SPH);
   __shared__ double sm[P::TPB * P::PER];
-  __shared__ double s_g[P::TPB][3];
-  __shared__ int s_atom[2][P::TPB];
   const int team = threadIdx.x / TE;
   const int tl = threadIdx.x % TE;
   const int64_t t = A.t0 + (int64_t)blockIdx.x * P::TPB + team;
   const bool valid = t < A.t1;
-  const bool digest = A.dm != nullptr;
   double* X = sm + team * P::PER;
   double* Ys = X + NEF;
   int any = 0;
@@ -1386,7 +1380,6 @@ __global__ void __launch_bounds__(256) eri_ip1_epi_kernel(BasisView Bv, BucketAr
     }
   }
   __syncthreads();
-  double g0 = 0.0, g1 = 0.0, g2 = 0.0;
   if (valid) {
     const VShell& sa = Bv.vsh[tk.sh[0]];
     const VShell& sb = Bv.vsh[tk.sh[1]];
@@ -1398,12 +1391,11 @@ __global__ void __launch_bounds__(256) eri_ip1_epi_kernel(BasisView Bv, BucketAr
                             : (int64_t)sa.dcart * sb.dcart * sc.dcart * sd.dcart;
     double* __restrict__ out = A.out + task_out(tk);
     if (!any) {
-      if (!digest)
-        for (int k = tl; k < 3 * NAo * NBo * NCo * NDo; k += TE) {
-          const int ao = k % NAo, bo = (k / NAo) % NBo, co = (k / (NAo * NBo)) % NCo;
-          const int dd = (k / (NAo * NBo * NCo)) % NDo, x = k / (NAo * NBo * NCo * NDo);
-          out[x * stc + ao * st0 + bo * st1 + co * st2 + dd * st3] = 0.0;
-        }
+      for (int k = tl; k < 3 * NAo * NBo * NCo * NDo; k += TE) {
+        const int ao = k % NAo, bo = (k / NAo) % NBo, co = (k / (NAo * NBo)) % NCo;
+        const int dd = (k / (NAo * NBo * NCo)) % NDo, x = k / (NAo * NBo * NCo * NDo);
+        out[x * stc + ao * st0 + bo * st1 + co * st2 + dd * st3] = 0.0;
+      }
     } else {
       const double cd[3] = {sc.r[0] - sd.r[0], sc.r[1] - sd.r[1], sc.r[2] - sd.r[2]};
       double cdp[3][LD + 1];
@@ -1412,8 +1404,6 @@ __global__ void __launch_bounds__(256) eri_ip1_epi_kernel(BasisView Bv, BucketAr
         cdp[d][0] = 1.0;
         sfor<LD>([&](auto K) { cdp[d][decltype(K)::value + 1] = cdp[d][decltype(K)::value] * cd[d]; });
       });
-      const double fkl = sc.shell != sd.shell ? 2.0 : 1.0;
-      const int64_t N = A.nao;
       for (int row = tl; row < ROWS; row += TE) {
         const int x = row / (NAo * NBo);
         const int ao = (row / NBo) % NAo, bo = row % NBo;
@@ -1434,60 +1424,19 @@ __global__ void __launch_bounds__(256) eri_ip1_epi_kernel(BasisView Bv, BucketAr
           });
           Zc[c * ND + d] = s;
         });
-        if (digest) {
-          const double* __restrict__ D = A.dm;
-          const int64_t Pi = sa.ao + ao, Qi = sb.ao + bo;
-          const double* __restrict__ DP = D + Pi * N;
-          const double* __restrict__ DQ = D + Qi * N;
-          const double dpq = -2.0 * DP[Qi];
-          double acc = 0.0;
-          sfor<NCo * NDo>([&](auto OD) {
-            constexpr int co = decltype(OD)::value / NDo, dd = decltype(OD)::value % NDo;
-            double s = 0.0;
-            sfor<NC * ND>([&](auto CD) {
-              constexpr int c = decltype(CD)::value / ND, d = decltype(CD)::value % ND;
-              constexpr double cc = c2x(SPH, LC, co, c) * c2x(SPH, LD, dd, d);
-              if constexpr (cc != 0.0) s = fma(cc, Zc[c * ND + d], s);
-            });
-            const int64_t Ri = sc.ao + co, Si = sd.ao + dd;
-            const double w = fma(dpq, D[Ri * N + Si], 0.5 * (DP[Ri] * DQ[Si] + DP[Si] * DQ[Ri]));
-            acc = fma(s, w, acc);
+        double* orow = out + x * stc + ao * st0 + bo * st1;
+        sfor<NCo * NDo>([&](auto OD) {
+          constexpr int co = decltype(OD)::value / NDo, dd = decltype(OD)::value % NDo;
+          double s = 0.0;
+          sfor<NC * ND>([&](auto CD) {
+            constexpr int c = decltype(CD)::value / ND, d = decltype(CD)::value % ND;
+            constexpr double cc = c2x(SPH, LC, co, c) * c2x(SPH, LD, dd, d);
+            if constexpr (cc != 0.0) s = fma(cc, Zc[c * ND + d], s);
           });
-          acc *= fkl;
-          if (x == 0) g0 += acc;
-          else if (x == 1) g1 += acc;
-          else g2 += acc;
-        } else {
-          double* orow = out + x * stc + ao * st0 + bo * st1;
-          sfor<NCo * NDo>([&](auto OD) {
-            constexpr int co = decltype(OD)::value / NDo, dd = decltype(OD)::value % NDo;
-            double s = 0.0;
-            sfor<NC * ND>([&](auto CD) {
-              constexpr int c = decltype(CD)::value / ND, d = decltype(CD)::value % ND;
-              constexpr double cc = c2x(SPH, LC, co, c) * c2x(SPH, LD, dd, d);
-              if constexpr (cc != 0.0) s = fma(cc, Zc[c * ND + d], s);
-            });
-            orow[co * st2 + dd * st3] = s;
-          });
-        }
+          orow[co * st2 + dd * st3] = s;
+        });
       }
     }
-  }
-  if (digest) {
-    for (int off = 1; off < TE; off <<= 1) {
-      g0 += __shfl_xor(g0, off);
-      g1 += __shfl_xor(g1, off);
-      g2 += __shfl_xor(g2, off);
-    }
-    if (tl == 0) {
-      s_g[team][0] = g0;
-      s_g[team][1] = g1;
-      s_g[team][2] = g2;
-      s_atom[0][team] = (valid && any) ? Bv.vsh[tk.sh[0]].atom : -1;
-      s_atom[1][team] = (valid && any) ? grad_ref(A, tk) : -1;
-    }
-    __syncthreads();
-    grad_block_flush(A, s_g, s_atom[0], s_atom[1], P::TPB);
   }
 }
 
@@ -1782,7 +1731,7 @@ __global__ void __launch_bounds__(64) eri_wave_kernel(BasisView Bv, BucketArgs A
           const int64_t row0 = r == 0 ? P0 : r == 1 ? R0 : r <= 3 ? P0 : Q0;
           const int64_t col0 = r == 0 ? Q0 : r == 1 ? S0 : (r == 2 || r == 4) ? R0 : S0;
           const int i = (m - o0) / ncol, j = (m - o0) % ncol;
-          atomicAdd(dst + (row0 + i) * N + col0 + j, (r < 2 ? 2.0 * f : f) * v);
+          atomicAdd(dst + slot_offset(A) + (row0 + i) * N + col0 + j, (r < 2 ? 2.0 * f : f) * v);
         }
       }
       return;
@@ -1903,19 +1852,11 @@ hipError_t launch_chunks(const BasisView& B, const BucketArgs& A0, hipStream_t s
       hipLaunchKernelGGL((eri_epi_kernel<LA, LB, LC, LD, false, DER>), egrid, dim3(P::THREADS), 0,
                          stream, B, A);
     }
-  } else if constexpr (DER != 1) {
+  } else {
     using P = EpiCfg<LA, LB, LC, LD>;
     const dim3 egrid((unsigned)((n + P::TPB - 1) / P::TPB));
     hipLaunchKernelGGL((eri_epi_kernel<LA, LB, LC, LD, true, DER>), egrid, dim3(P::THREADS), 0,
                        stream, B, A);
-  } else if (A.sph) {
-    using P = Ip1EpiCfg<LA, LB, LC, LD>;
-    const dim3 egrid((unsigned)((n + P::TPB - 1) / P::TPB));
-    hipLaunchKernelGGL((eri_ip1_epi_kernel<LA, LB, LC, LD>), egrid, dim3(P::THREADS), 0, stream, B, A);
-  } else {
-    using P = Ip1EpiCfg<LA, LB, LC, LD, false>;
-    const dim3 egrid((unsigned)((n + P::TPB - 1) / P::TPB));
-    hipLaunchKernelGGL((eri_ip1_epi_kernel<LA, LB, LC, LD, false>), egrid, dim3(P::THREADS), 0, stream, B, A);
   }
   return hipGetLastError();
 }
@@ -2094,14 +2035,6 @@ hipError_t launch_chunk3_class(const BasisView& B, const BucketArgs& A, hipStrea
     return launch_chunks<a, b, c, d, 2>(                                                   \
         B, A, stream, std::make_integer_sequence<int, chunk_groups(ChunkCfg<a, b, c, d, 2>::NCH)>{});    \
   }
-#define MCINT_IP1_DEFINE(a, b, c, d)                                                       \
-  template <>                                                                              \
-  hipError_t launch_ip1_class<a, b, c, d>(const BasisView& B, const BucketArgs& A,         \
-                                          hipStream_t stream) {                            \
-    return launch_chunks<a, b, c, d, 1>(                                                   \
-        B, A, stream, std::make_integer_sequence<int, chunk_groups(ChunkCfg<a, b, c, d, 1>::NCH)>{});    \
-  }
-
 #define MCINT_FAST_DECLARE(a, b, c, d)                                                     \
   template <>                                                                              \
   hipError_t launch_fast_class<a, b, c, d>(const BasisView& B, const BucketArgs& A,        \

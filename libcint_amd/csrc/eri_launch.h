@@ -23,8 +23,9 @@ hipError_t launch_count_prims(const BasisView& B, const BucketArgs& A, unsigned 
 
 hipError_t launch_generic(const BasisView& B, const BucketArgs& A, hipStream_t stream);
 
-// grad[i] += sum over the nslot accumulator copies of acc[slot * n + i]
-hipError_t launch_grad_reduce(const double* acc, int nslot, int n, double* grad, hipStream_t stream);
+// grad[i] += sum over the nslot accumulator copies of acc[slot * stride + i], i < n
+hipError_t launch_grad_reduce(const double* acc, int nslot, int64_t stride, int n, double* grad,
+                              hipStream_t stream);
 
 // Grouped J/K digest: row pass (groups of quartets sharing (i,j), LDS of
 // rows_lds bytes) and column pass (groups sharing (k,l)) into the half
@@ -33,7 +34,9 @@ hipError_t launch_jk_grouped(const int* shls, const int64_t* off, const int* row
                              const int* rows_ptr, int nrows, size_t rows_lds, const int* cols_q,
                              const int* cols_ptr, int ncols, const double* eri, const int* ao_loc,
                              const double* D, int nao, double* Jp, double* Kp, hipStream_t stream);
-hipError_t launch_symmetrize(const double* X, double* out, int n, hipStream_t stream);
+// out = X + X^T of the sum of nslot copies of X, stride doubles apart
+hipError_t launch_symmetrize(const double* X, double* out, int n, int nslot, int64_t stride,
+                             hipStream_t stream);
 // x[0..n) = 0 (a kernel, so that captured graphs hold no memset node)
 hipError_t launch_zero(double* x, int64_t n, hipStream_t stream);
 

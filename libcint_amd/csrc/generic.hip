@@ -528,15 +528,16 @@ __attribute__((amdgpu_waves_per_eu(3))) eri_generic_kernel(BasisView B, BucketAr
             const int64_t N = A.nao;
             const int64_t P = s0.ao + ao, Q = s1.ao + bo, R = s2.ao + co, S = s3.ao + dd;
             const double* D = A.dm;
+            const int64_t slot = slot_offset(A);
             if (A.jk_j) {
-              atomicAdd(A.jk_j + P * N + Q, 2.0 * fjk * v * D[R * N + S]);
-              atomicAdd(A.jk_j + R * N + S, 2.0 * fjk * v * D[P * N + Q]);
+              atomicAdd(A.jk_j + slot + P * N + Q, 2.0 * fjk * v * D[R * N + S]);
+              atomicAdd(A.jk_j + slot + R * N + S, 2.0 * fjk * v * D[P * N + Q]);
             }
             if (A.jk_k) {
-              atomicAdd(A.jk_k + P * N + R, fjk * v * D[Q * N + S]);
-              atomicAdd(A.jk_k + P * N + S, fjk * v * D[Q * N + R]);
-              atomicAdd(A.jk_k + Q * N + R, fjk * v * D[P * N + S]);
-              atomicAdd(A.jk_k + Q * N + S, fjk * v * D[P * N + R]);
+              atomicAdd(A.jk_k + slot + P * N + R, fjk * v * D[Q * N + S]);
+              atomicAdd(A.jk_k + slot + P * N + S, fjk * v * D[Q * N + R]);
+              atomicAdd(A.jk_k + slot + Q * N + R, fjk * v * D[P * N + S]);
+              atomicAdd(A.jk_k + slot + Q * N + S, fjk * v * D[P * N + R]);
             }
           } else if (digest) {
             // dE/dA = sum (d/dr i j|kl) [-2 D_ij D_kl + (D_ik D_jl + D_il D_jk)/2],
@@ -557,7 +558,7 @@ __attribute__((amdgpu_waves_per_eu(3))) eri_generic_kernel(BasisView B, BucketAr
       __syncthreads();
     }
     if (digest) {
-      double* gs = A.grad + (int64_t)(blockIdx.x % A.nslot) * A.grad_stride;
+      double* gs = A.grad + slot_offset(A);
       const int ref = grad_ref(A, tk);
       for (int c = 0; c < 3; ++c) {
         double g = gpart[c];

@@ -326,7 +326,7 @@ __global__ void __launch_bounds__(64) eri_ip1_wave_kernel(BasisView Bv, BucketAr
   const bool digest = A.dm != nullptr;
   int cur = -1;      // lanes 0-2 of a quartet: x, y, z of its atom; 3-5: of the
   double cs = 0.0;   // reference atom, minus
-  double* const gbase = digest ? A.grad + (int64_t)(blockIdx.x % A.nslot) * A.grad_stride : nullptr;
+  double* const gbase = digest ? A.grad + slot_offset(A) : nullptr;
   const int64_t ngrp = (A.t1 - A.t0 + TPW - 1) / TPW;
   const int64_t g0 = ngrp * blockIdx.x / gridDim.x, g1 = ngrp * (blockIdx.x + 1) / gridDim.x;
   for (int64_t grp = g0; grp < g1; ++grp) {
@@ -563,7 +563,6 @@ hipError_t launch_ip1(const BasisView& B, const BucketArgs& A, hipStream_t strea
   return hipGetLastError();
 }
 
-#undef MCINT_IP1_DEFINE
 #define MCINT_IP1_DEFINE(a, b, c, d)                                                       \
   template <>                                                                              \
   hipError_t launch_ip1_class<a, b, c, d>(const BasisView& B, const BucketArgs& A,         \

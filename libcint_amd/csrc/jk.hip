@@ -194,11 +194,14 @@ hipError_t launch_zero(double* x, int64_t n, hipStream_t stream) {
   return hipGetLastError();
 }
 
-__global__ void symmetrize_kernel(const double* __restrict__ X, double* __restrict__ out, int n) {
+__global__ void symmetrize_kernel(const double* __restrict__ X, double* __restrict__ out, int n,
+                                  int nslot, int64_t stride) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= (int64_t)n * n) return;
   const int64_t i = t / n, j = t % n;
-  out[t] = X[i * n + j] + X[j * n + i];
+  double s = 0.0;
+  for (int k = 0; k < nslot; ++k, X += stride) s += X[i * n + j] + X[j * n + i];
+  out[t] = s;
 }
 
 hipError_t launch_jk_grouped(const int* shls, const int64_t* off, const int* rows_q,
@@ -219,27 +222,29 @@ hipError_t launch_jk_grouped(const int* shls, const int64_t* off, const int* row
   return hipSuccess;
 }
 
-hipError_t launch_symmetrize(const double* X, double* out, int n, hipStream_t stream) {
+hipError_t launch_symmetrize(const double* X, double* out, int n, int nslot, int64_t stride,
+                             hipStream_t stream) {
   const int64_t tot = (int64_t)n * n;
   if (tot <= 0) return hipSuccess;
   hipLaunchKernelGGL(symmetrize_kernel, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, stream,
-                     X, out, n);
+                     X, out, n, nslot, stride);
   return hipGetLastError();
 }
 
-__global__ void grad_reduce_kernel(const double* __restrict__ acc, int nslot, int n,
+__global__ void grad_reduce_kernel(const double* __restrict__ acc, int nslot, int64_t stride, int n,
                                    double* __restrict__ grad) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   double s = 0.0;
-  for (int k = 0; k < nslot; ++k) s += acc[(int64_t)k * n + i];
+  for (int k = 0; k < nslot; ++k) s += acc[k * stride + i];
   grad[i] += s;
 }
 
-hipError_t launch_grad_reduce(const double* acc, int nslot, int n, double* grad, hipStream_t stream) {
+hipError_t launch_grad_reduce(const double* acc, int nslot, int64_t stride, int n, double* grad,
+                              hipStream_t stream) {
   if (n <= 0) return hipSuccess;
   hipLaunchKernelGGL(grad_reduce_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream,
-                     acc, nslot, n, grad);
+                     acc, nslot, stride, n, grad);
   return hipGetLastError();
 }
 

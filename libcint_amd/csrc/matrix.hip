@@ -427,15 +427,16 @@ eri_matrix_kernel(BasisView B, BucketArgs A, GenLayout G, XferView XV) {
       const int64_t P = s0.ao + ao, Q = s1.ao + bo, R = s2.ao + co, Sd = s3.ao + dd;
       const double* D = A.dm;
       if (jk) {
+        const int64_t slot = slot_offset(A);
         if (A.jk_j) {
-          atomicAdd(A.jk_j + P * N + Q, 2.0 * fjk * v * D[R * N + Sd]);
-          atomicAdd(A.jk_j + R * N + Sd, 2.0 * fjk * v * D[P * N + Q]);
+          atomicAdd(A.jk_j + slot + P * N + Q, 2.0 * fjk * v * D[R * N + Sd]);
+          atomicAdd(A.jk_j + slot + R * N + Sd, 2.0 * fjk * v * D[P * N + Q]);
         }
         if (A.jk_k) {
-          atomicAdd(A.jk_k + P * N + R, fjk * v * D[Q * N + Sd]);
-          atomicAdd(A.jk_k + P * N + Sd, fjk * v * D[Q * N + R]);
-          atomicAdd(A.jk_k + Q * N + R, fjk * v * D[P * N + Sd]);
-          atomicAdd(A.jk_k + Q * N + Sd, fjk * v * D[P * N + R]);
+          atomicAdd(A.jk_k + slot + P * N + R, fjk * v * D[Q * N + Sd]);
+          atomicAdd(A.jk_k + slot + P * N + Sd, fjk * v * D[Q * N + R]);
+          atomicAdd(A.jk_k + slot + Q * N + R, fjk * v * D[P * N + Sd]);
+          atomicAdd(A.jk_k + slot + Q * N + Sd, fjk * v * D[P * N + R]);
         }
         return;
       }
@@ -531,7 +532,7 @@ eri_matrix_kernel(BasisView B, BucketArgs A, GenLayout G, XferView XV) {
       wave_sync();  // Y is rewritten
     }
     if (A.dm && !jk) {
-      double* gs = A.grad + (int64_t)(blockIdx.x % A.nslot) * A.grad_stride;
+      double* gs = A.grad + slot_offset(A);
       const int ref = grad_ref(A, tk);
       for (int c = 0; c < 3; ++c) {
         double g = gpart[c];

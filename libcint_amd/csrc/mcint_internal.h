@@ -140,14 +140,16 @@ struct BucketArgs {
   const double* dm;      // nao x nao density, row-major (nullable: store mode)
   double* grad;          // nslot blocks of grad_stride (= 3 natm) accumulators
   int nao;
-  int nslot;             // gradient accumulator copies (spreads the atomics)
-  int grad_stride;
+  // accumulator copies of the gradient and of J', K': block b adds to copy
+  // b % nslot, slot_stride doubles apart
+  int nslot;
+  int64_t slot_stride;
   // translational invariance: the tasks' output field holds 1 + the atom
   // that receives minus the sum (no entry differentiates a shell of it)
   int grad_refs;
   // J/K digest (plain four-centre plans over unique quartets): instead of
   // storing the block, add its six block updates to the half matrices
-  // J' (jk_j) and K' (jk_k), nao x nao row-major, density dm
+  // J' (jk_j) and K' (jk_k), nao x nao row-major, density dm (copies as above)
   double* jk_j;
   double* jk_k;
 };
