@@ -62,6 +62,161 @@ void dfree(T*& p) {
   p = nullptr;
 }
 
+// Things that are dear to make and serve any plan: kept between uses, at most
+// MAX of a kind, each with one owner at a time.
+template <typename T, int MAX>
+struct Kept {
+  std::mutex m;
+  std::vector<std::unique_ptr<T>> idle;
+  // one made on the current device, or nullptr
+  std::unique_ptr<T> take() {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return nullptr;
+    {
+      std::lock_guard<std::mutex> g(m);
+      for (size_t i = idle.size(); i-- > 0;)
+        if (idle[i]->device == dev) {
+          std::unique_ptr<T> t = std::move(idle[i]);
+          idle.erase(idle.begin() + i);
+          return t;
+        }
+    }
+    std::unique_ptr<T> t(new T);
+    t->device = dev;
+    return t->make() ? std::move(t) : nullptr;
+  }
+  void give(std::unique_ptr<T> t) {
+    if (!t) return;
+    std::lock_guard<std::mutex> g(m);
+    if (idle.size() < (size_t)MAX) idle.push_back(std::move(t));
+  }
+  // the list is not destroyed at exit (the runtime may be gone by then)
+  static Kept& get() {
+    static Kept* k = new Kept;
+    return *k;
+  }
+};
+
+// Pinned memory that pageable host data passes through.  A copy of more than
+// about a megabyte from or to pageable memory makes the runtime pin the
+// caller's pages: the 1.1 MB task list of a 72 000-quartet batch took 4 ms.
+struct Stage {
+  static constexpr size_t BYTES = 2 << 20;
+  int device = 0;
+  char* p = nullptr;
+  hipEvent_t ev = nullptr;
+  bool make() {
+    return hipHostMalloc((void**)&p, BYTES) == hipSuccess &&
+           hipEventCreateWithFlags(&ev, hipEventDisableTiming) == hipSuccess;
+  }
+  ~Stage() {
+    if (ev) (void)hipEventDestroy(ev);
+    if (p) (void)hipHostFree(p);
+  }
+};
+using Stages = Kept<Stage, 16>;
+constexpr size_t STAGE_MIN = 256 << 10;  // smaller copies go directly
+
+// dst (device) = n elements of src (pageable), on the null stream; returns
+// with src read and the copy done.
+template <typename T>
+hipError_t to_device(T* dst, const T* src, size_t n) {
+  const size_t bytes = n * sizeof(T);
+  std::unique_ptr<Stage> s[2];
+  if (bytes >= STAGE_MIN)
+    for (auto& x : s) x = Stages::get().take();
+  if (!s[0] || !s[1]) return hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice);
+  hipError_t e = hipSuccess;
+  size_t c = 0;
+  for (size_t o = 0; o < bytes && e == hipSuccess; o += Stage::BYTES, ++c) {
+    Stage& x = *s[c & 1];
+    const size_t k = std::min(Stage::BYTES, bytes - o);
+    if (c > 1) e = hipEventSynchronize(x.ev);
+    if (e != hipSuccess) break;
+    memcpy(x.p, (const char*)src + o, k);
+    e = hipMemcpyAsync((char*)dst + o, x.p, k, hipMemcpyHostToDevice, nullptr);
+    if (e == hipSuccess) e = hipEventRecord(x.ev, nullptr);
+  }
+  // the buffers are given back only when nothing reads them any more
+  const hipError_t d = hipStreamSynchronize(nullptr);
+  if (e == hipSuccess) e = d;
+  if (d == hipSuccess)
+    for (auto& x : s) Stages::get().give(std::move(x));
+  return e;
+}
+
+// Several device arrays in one allocation, the uploaded ones first: a short
+// list's uploads go as one copy (each costs about 10 us).
+struct Arena {
+  struct Part {
+    const void* src;
+    size_t off, bytes;
+  };
+  std::vector<Part> parts;
+  size_t bytes = 0, uploaded = 0;
+  // room for n elements; src: host data to upload, or nullptr
+  template <typename T>
+  size_t add(size_t n, const T* src) {
+    const size_t off = bytes;
+    parts.push_back(Part{src, off, src ? n * sizeof(T) : 0});
+    bytes = off + ((std::max<size_t>(n, 1) * sizeof(T) + 255) & ~size_t(255));
+    if (src) uploaded = bytes;
+    return off;
+  }
+  // allocates base and uploads
+  hipError_t make(char** base) {
+    hipError_t e = dalloc(base, bytes);
+    if (e != hipSuccess || !uploaded) return e;
+    if (uploaded < STAGE_MIN) {
+      std::vector<char> h(uploaded);
+      for (const Part& q : parts)
+        if (q.bytes) memcpy(h.data() + q.off, q.src, q.bytes);
+      return hipMemcpy(*base, h.data(), uploaded, hipMemcpyHostToDevice);
+    }
+    for (const Part& q : parts)
+      if (q.bytes && e == hipSuccess) e = to_device(*base + q.off, (const char*)q.src, q.bytes);
+    return e;
+  }
+};
+
+// dst (pageable) = bytes of src (device) after the work on stream; returns
+// when the copy is done.  Threads take the chunks in turn: the host's part
+// (page faults of a fresh array, the copy out) is the longer one.
+hipError_t to_host(void* dst, const void* src, size_t bytes, hipStream_t stream) {
+  const size_t chunks = (bytes + Stage::BYTES - 1) / Stage::BYTES;
+  int dev = 0;
+  if (chunks < 2 || hipGetDevice(&dev) != hipSuccess) {
+    const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream);
+    return e == hipSuccess ? hipStreamSynchronize(stream) : e;
+  }
+  std::atomic<size_t> next{0};
+  std::atomic<int> failed{(int)hipSuccess};
+  auto work = [&] {
+    hipError_t r = hipSetDevice(dev);
+    std::unique_ptr<Stage> x = r == hipSuccess ? Stages::get().take() : nullptr;
+    if (r == hipSuccess && !x) r = hipErrorOutOfMemory;
+    for (size_t c; r == hipSuccess && (c = next.fetch_add(1)) < chunks;) {
+      const size_t o = c * Stage::BYTES, k = std::min(Stage::BYTES, bytes - o);
+      r = hipMemcpyAsync(x->p, (const char*)src + o, k, hipMemcpyDeviceToHost, stream);
+      if (r == hipSuccess) r = hipEventRecord(x->ev, stream);
+      if (r == hipSuccess) r = hipEventSynchronize(x->ev);
+      if (r == hipSuccess) memcpy((char*)dst + o, x->p, k);
+    }
+    if (r != hipSuccess) failed = (int)r;
+    else Stages::get().give(std::move(x));
+  };
+  std::vector<std::thread> th;
+  th.reserve(8);
+  try {
+    while (th.size() + 1 < std::min<size_t>(8, chunks)) th.emplace_back(work);
+  } catch (...) {  // fewer threads, then
+  }
+  work();
+  for (auto& x : th) x.join();
+  const hipError_t e = hipStreamSynchronize(stream);
+  return e == hipSuccess ? (hipError_t)failed.load() : e;
+}
+
 int intor_kind(int intor) {
   switch (intor) {
     case MCINT_INT2E_SPH:
@@ -106,6 +261,7 @@ struct mcint_basis {
   std::vector<int> vfirst;  // first virtual shell of each real shell
   int dummy = 0;            // virtual shell of the exponent-0 s function (int2c2e's partner)
   size_t envlen = 0;        // doubles of the caller's env copied (env holds 2 more)
+  char* mem_d = nullptr;    // holds the device arrays below
   VShell* vsh_d = nullptr;
   double* env_d = nullptr;
   int* ao_loc_d = nullptr;  // spherical AO offsets of the real shells, nbas+1
@@ -209,20 +365,18 @@ static int basis_create_impl(mcint_basis** out, const FINT* atm, FINT natm, cons
     return MCINT_OK;
   }
   hipError_t e = hipGetDevice(&b->device);
-  if (e == hipSuccess) e = dalloc(&b->vsh_d, b->vsh.size());
-  if (e == hipSuccess) e = dalloc(&b->env_d, b->env.size());
-  if (e == hipSuccess) e = dalloc(&b->ao_loc_d, ao_loc.size());
-  if (e == hipSuccess)
-    e = hipMemcpy(b->ao_loc_d, ao_loc.data(), ao_loc.size() * sizeof(int), hipMemcpyHostToDevice);
-  if (e == hipSuccess)
-    e = hipMemcpy(b->vsh_d, b->vsh.data(), b->vsh.size() * sizeof(VShell), hipMemcpyHostToDevice);
-  if (e == hipSuccess)
-    e = hipMemcpy(b->env_d, b->env.data(), b->env.size() * sizeof(double), hipMemcpyHostToDevice);
+  if (e == hipSuccess) {
+    Arena m;
+    const size_t ov = m.add(b->vsh.size(), b->vsh.data()), oe = m.add(b->env.size(), b->env.data());
+    const size_t oa = m.add(ao_loc.size(), ao_loc.data());
+    e = m.make(&b->mem_d);
+    b->vsh_d = (VShell*)(b->mem_d + ov);
+    b->env_d = (double*)(b->mem_d + oe);
+    b->ao_loc_d = (int*)(b->mem_d + oa);
+  }
   if (e != hipSuccess) {
     set_err(std::string("mcint_basis_create: ") + hipGetErrorString(e));
-    dfree(b->vsh_d);
-    dfree(b->env_d);
-    dfree(b->ao_loc_d);
+    dfree(b->mem_d);
     delete b;
     return MCINT_ERR_HIP;
   }
@@ -237,9 +391,7 @@ extern "C" int mcint_basis_create(mcint_basis** out, const FINT* atm, FINT natm,
 
 extern "C" void mcint_basis_destroy(mcint_basis* b) {
   if (!b) return;
-  dfree(b->vsh_d);
-  dfree(b->env_d);
-  dfree(b->ao_loc_d);
+  dfree(b->mem_d);
   delete b;
 }
 
@@ -607,6 +759,30 @@ std::vector<uint32_t> task_groups(const std::vector<uint32_t>& raw, const std::v
 
 }  // namespace
 
+// Side streams of branched launches and their fork and join events; creating
+// four streams takes about 1.2 ms.
+struct Side {
+  int device = 0;
+  hipStream_t st[MAX_GRAPH_BRANCHES] = {};
+  hipEvent_t ev[MAX_GRAPH_BRANCHES + 1] = {};
+  int n = 0;
+  bool make() { return grow(1); }
+  bool grow(int nbr) {
+    for (; n < nbr; ++n)
+      if (hipStreamCreateWithFlags(&st[n], hipStreamNonBlocking) != hipSuccess) return false;
+    for (int i = 0; i <= nbr; ++i)
+      if (!ev[i] && hipEventCreateWithFlags(&ev[i], hipEventDisableTiming) != hipSuccess) return false;
+    return true;
+  }
+  ~Side() {
+    for (hipStream_t s : st)
+      if (s) (void)hipStreamDestroy(s);
+    for (hipEvent_t e : ev)
+      if (e) (void)hipEventDestroy(e);
+  }
+};
+using Sides = Kept<Side, 8>;
+
 struct mcint_plan {
   mcint_basis* b = nullptr;
   int intor = 0, kind = 0, sph = 1, ncomp = 1;
@@ -614,6 +790,7 @@ struct mcint_plan {
   bool grad_refs = false;  // gradient plan: tasks carry a reference atom, no output offset
   std::vector<Bucket> buckets;   // tasks of one class and tuned team
   std::vector<Bucket> launches;  // tasks of one class, lanes per task and kernel
+  char* mem_d = nullptr;  // holds the tasks, pair tables and pair data below
   Task* tasks_d = nullptr;
   int* task_id_d = nullptr;
   int64_t* pair_off_d = nullptr;
@@ -646,23 +823,15 @@ struct mcint_plan {
   FINT* g_not0 = nullptr;
   hipStream_t g_stream = nullptr;
   int g_nbr = 0;
-  // side streams and fork/join events of the branched capture
-  std::vector<hipStream_t> side;
-  std::vector<hipEvent_t> events;
+  std::unique_ptr<Side> side;  // of the branched launches
 };
 
 static void plan_free(mcint_plan* p) {
   if (!p) return;
   if (p->gexec) (void)hipGraphExecDestroy(p->gexec);
   if (p->graph) (void)hipGraphDestroy(p->graph);
-  for (hipStream_t st : p->side) (void)hipStreamDestroy(st);
-  for (hipEvent_t ev : p->events) (void)hipEventDestroy(ev);
-  dfree(p->tasks_d);
-  dfree(p->task_id_d);
-  dfree(p->pair_off_d);
-  dfree(p->pair_ld_d);
-  dfree(p->pp_d);
-  dfree(p->pp_pos_d);
+  Sides::get().give(std::move(p->side));  // work still on them comes first
+  dfree(p->mem_d);
   dfree(p->scratch_d);
   dfree(p->flags_d);
   dfree(p->gslots_d);
@@ -1198,27 +1367,25 @@ static int plan_create_impl(mcint_plan** out, mcint_basis* b, int intor, const F
     *out = p;
     return MCINT_OK;
   }
-  int* pairs_d = nullptr;
-  PairPrim* pp_tmp = nullptr;
-  hipError_t e = dalloc(&p->tasks_d, (size_t)std::max<int64_t>(ntasks, 1));
-  if (e == hipSuccess) e = dalloc(&p->task_id_d, (size_t)std::max<int64_t>(ntasks, 1));
-  if (e == hipSuccess) e = dalloc(&p->pair_off_d, pair_off.size());
-  if (e == hipSuccess) e = dalloc(&p->pair_ld_d, pair_off.size());
-  if (e == hipSuccess) e = dalloc(&p->pp_d, (size_t)std::max<int64_t>(npp, 1));
-  if (e == hipSuccess) e = dalloc(&p->pp_pos_d, (size_t)std::max<int64_t>(npp, 1));
-  if (e == hipSuccess) e = dalloc(&pp_tmp, (size_t)std::max<int64_t>(npp, 1));
-  if (e == hipSuccess) e = dalloc(&pairs_d, pairs.size());
+  char* tmp_d = nullptr;  // shell pairs and the pair kernel's staging records
+  Arena m, tmp;
+  const size_t ot = m.add((size_t)ntasks, sorted.get()), oi = m.add((size_t)ntasks, sorted_q.get());
+  const size_t oo = m.add(pair_off.size(), pair_off.data());
+  const size_t ol = m.add(pair_off.size(), (const double*)nullptr);
+  const size_t op = m.add((size_t)npp, (const PairPrim*)nullptr), os = m.add((size_t)npp, (const int*)nullptr);
+  const size_t xp = tmp.add(pairs.size(), pairs.data()), xt = tmp.add((size_t)npp, (const PairPrim*)nullptr);
+  hipError_t e = m.make(&p->mem_d);
+  if (e == hipSuccess) e = tmp.make(&tmp_d);
+  p->tasks_d = (Task*)(p->mem_d + ot);
+  p->task_id_d = (int*)(p->mem_d + oi);
+  p->pair_off_d = (int64_t*)(p->mem_d + oo);
+  p->pair_ld_d = (double*)(p->mem_d + ol);
+  p->pp_d = (PairPrim*)(p->mem_d + op);
+  p->pp_pos_d = (int*)(p->mem_d + os);
+  int* const pairs_d = (int*)(tmp_d + xp);
+  PairPrim* const pp_tmp = (PairPrim*)(tmp_d + xt);
   p->scratch_size = max_gen;
   p->flags_size = max_flags;
-  if (e == hipSuccess && ntasks > 0)
-    e = hipMemcpy(p->tasks_d, sorted.get(), (size_t)ntasks * sizeof(Task), hipMemcpyHostToDevice);
-  if (e == hipSuccess && ntasks > 0)
-    e = hipMemcpy(p->task_id_d, sorted_q.get(), (size_t)ntasks * sizeof(int), hipMemcpyHostToDevice);
-  if (e == hipSuccess)
-    e = hipMemcpy(p->pair_off_d, pair_off.data(), pair_off.size() * sizeof(int64_t),
-                  hipMemcpyHostToDevice);
-  if (e == hipSuccess && !pairs.empty())
-    e = hipMemcpy(pairs_d, pairs.data(), pairs.size() * sizeof(int), hipMemcpyHostToDevice);
   if (e == hipSuccess)
     e = launch_pairdata(b->vsh_d, b->env_d, nv, pairs_d, (int)(pairs.size() / 2), p->pair_off_d,
                         p->pair_ld_d, pp_tmp, p->pp_d, p->pp_pos_d, nullptr);
@@ -1228,17 +1395,15 @@ static int plan_create_impl(mcint_plan** out, mcint_basis* b, int intor, const F
     if (e == hipSuccess) e = dalloc(&p->xfer_d, (size_t)xsize);
     if (e == hipSuccess) e = dalloc(&p->xfer_off_d, xoff.size());
     if (e == hipSuccess)
-      e = hipMemcpy(items_d, xitems.data(), xitems.size() * sizeof(XferItem), hipMemcpyHostToDevice);
-    if (e == hipSuccess)
-      e = hipMemcpy(p->xfer_off_d, xoff.data(), xoff.size() * sizeof(int64_t), hipMemcpyHostToDevice);
+      e = to_device(items_d, xitems.data(), xitems.size());
+    if (e == hipSuccess) e = to_device(p->xfer_off_d, xoff.data(), xoff.size());
     if (e == hipSuccess)
       e = launch_xfer(b->vsh_d, kind, sph, items_d, (int)xitems.size(), p->xfer_d, nullptr);
   }
   if (e == hipSuccess) e = hipDeviceSynchronize();
   timer.mark("device upload, pair data");
   dfree(items_d);
-  dfree(pairs_d);
-  dfree(pp_tmp);
+  dfree(tmp_d);
   if (e != hipSuccess) {
     set_err(std::string("mcint_plan_create: ") + hipGetErrorString(e));
     plan_free(p);
@@ -1543,16 +1708,13 @@ static int plan_launch(mcint_plan* p, double* out, FINT* not0, hipStream_t strea
 // always end.
 template <class F>
 static int launch_branched(mcint_plan* p, hipStream_t stream, int nbr, F&& launch) {
-  while ((int)p->side.size() < nbr) {
-    hipStream_t st = nullptr;
-    HIPCHK(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
-    p->side.push_back(st);
+  if (!p->side) p->side = Sides::get().take();
+  if (!p->side || !p->side->grow(nbr)) {
+    set_err("side streams could not be created");
+    return MCINT_ERR_HIP;
   }
-  while ((int)p->events.size() < nbr + 1) {
-    hipEvent_t ev = nullptr;
-    HIPCHK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-    p->events.push_back(ev);
-  }
+  const hipStream_t* const side = p->side->st;
+  const hipEvent_t* const events = p->side->ev;
   std::vector<int> order(p->launches.size());
   for (size_t i = 0; i < order.size(); ++i) order[i] = (int)i;
   std::stable_sort(order.begin(), order.end(),
@@ -1564,23 +1726,23 @@ static int launch_branched(mcint_plan* p, hipStream_t stream, int nbr, F&& launc
     lists[k].push_back(i);
     load[k] += p->launches[i].cost;
   }
-  HIPCHK(hipEventRecord(p->events[0], stream));
+  HIPCHK(hipEventRecord(events[0], stream));
   int st = MCINT_OK;
   hipError_t e = hipSuccess;
   for (int k = 0; k < nbr; ++k) {
-    e = hipStreamWaitEvent(p->side[k], p->events[0], 0);
+    e = hipStreamWaitEvent(side[k], events[0], 0);
     if (e != hipSuccess) break;
   }
   if (e == hipSuccess) {
     for (int k = 0; k < nbr && st == MCINT_OK; ++k)
       for (int i : lists[k]) {
-        st = launch(p->launches[i], p->side[k], plan_scratch(p, k));
+        st = launch(p->launches[i], side[k], plan_scratch(p, k));
         if (st) break;
       }
   }
   for (int k = 0; k < nbr; ++k) {
-    const hipError_t a = hipEventRecord(p->events[k + 1], p->side[k]);
-    const hipError_t b = hipStreamWaitEvent(stream, p->events[k + 1], 0);
+    const hipError_t a = hipEventRecord(events[k + 1], side[k]);
+    const hipError_t b = hipStreamWaitEvent(stream, events[k + 1], 0);
     if (e == hipSuccess) e = a != hipSuccess ? a : b;
   }
   if (st != MCINT_OK) return st;
@@ -2074,6 +2236,18 @@ void mcint::set_error(const char* msg) { set_err(msg); }
 // ---------------------------------------------------------------------------
 // Host-pointer batches
 // ---------------------------------------------------------------------------
+// One run of a plan that will not run again: its launches on side streams,
+// unless a scratch region for each would be large.
+static int plan_run(mcint_plan* p, double* out, FINT* not0, hipStream_t stream) {
+  const int nbr = std::min<int>(g_graph_branches, (int)p->launches.size());
+  if (nbr <= 1 || p->scratch_size * nbr > GEN_SCRATCH_DOUBLES / 8)
+    return mcint_plan_execute_direct(p, out, not0, stream);
+  if (const int st = ensure_scratch(p, nbr)) return st;
+  return launch_branched(p, stream, nbr, [&](const Bucket& bk, hipStream_t s, const ScratchView& S) {
+    return bucket_launch(p, bk, out, not0, s, S);
+  });
+}
+
 static int host_batch(int intor, double* out, const size_t* out_offsets, const FINT* shls,
                       size_t nq, const FINT* atm, FINT natm, const FINT* bas, FINT nbas,
                       const double* env, FINT* not0, void* hip_stream) {
@@ -2104,12 +2278,10 @@ static int host_batch(int intor, double* out, const size_t* out_offsets, const F
     e = hipMemcpyAsync(od, out, (size_t)osz * sizeof(double), hipMemcpyHostToDevice, stream);
   }
   if (e == hipSuccess) {
-    st = mcint_plan_execute_direct(p, od, nd, stream);
+    st = plan_run(p, od, nd, stream);
     if (st == MCINT_OK) {
-      e = hipMemcpyAsync(out, od, (size_t)osz * sizeof(double), hipMemcpyDeviceToHost, stream);
-      if (e == hipSuccess && not0)
-        e = hipMemcpyAsync(not0, nd, nq * sizeof(FINT), hipMemcpyDeviceToHost, stream);
-      if (e == hipSuccess) e = hipStreamSynchronize(stream);
+      e = to_host(out, od, (size_t)osz * sizeof(double), stream);
+      if (e == hipSuccess && not0) e = to_host(not0, nd, nq * sizeof(FINT), stream);
     }
   }
   if (e != hipSuccess) {

@@ -225,3 +225,36 @@ def test_gradient_wave_kernel(mc):
         mc.tune(mc.TUNE_WAVE_KERNELS, old)
     for g in out[1:]:
         np.testing.assert_allclose(g, out[0], rtol=0, atol=1e-11 * max(1.0, np.abs(out[0]).max()))
+
+
+def test_large_host_batches(mc):
+    """Lists and outputs beyond the staging buffers' size: a host batch equals
+    the same plan's device buffer, from several threads at once as alone."""
+    import threading
+
+    import torch
+    from libcint_amd.synthetic import subset, unique_quartets
+    m = subset(make_molecule("c3"), 7)
+    B = mc.Basis(m.atm, m.bas, m.env)
+    q = unique_quartets(m.nbas)
+    assert q.nbytes > 4 << 20
+    db = mc.DeviceBasis(B)
+    plan = mc.Plan(db, "int2e_sph", q)
+    dev = torch.full((plan.out_size,), 7.0, dtype=torch.float64, device="cuda")
+    plan.execute(dev.data_ptr(), graph=False)
+    ref = dev.cpu().numpy()
+    plan.close()
+    db.close()
+    assert ref.nbytes > 3 * (2 << 20) + 8
+    got = [None] * 4
+
+    def work(i):
+        got[i] = mc.batch("int2e_sph", q[:len(q) - i], B)[0]
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for g in got:
+        np.testing.assert_allclose(g, ref[:len(g)], rtol=0, atol=1e-13)
