@@ -315,13 +315,16 @@ class DeviceBasis:
         """(quartets [n, 4], reference atoms [n]) of the two-electron gradient:
         (i, j, k >= l) of every quartet except where i sits on the quartet's
         reference atom, which receives minus the other derivatives."""
-        n = ctypes.c_size_t()
-        _check(lib().mcint_gradient_list(self.handle, None, None, 0, ctypes.byref(n)), "mcint_gradient_list")
-        shls, refs = np.empty((n.value, 4), np.int32), np.empty(n.value, np.int32)
-        if n.value:
-            _check(lib().mcint_gradient_list(self.handle, _ip(shls), _ip(refs), n.value, ctypes.byref(n)),
+        n, nb = ctypes.c_size_t(), self.basis.nbas
+        cap = nb ** 3 * (nb + 1) // 2  # the whole list; pages beyond the entries stay untouched
+        if cap > 1 << 24:
+            _check(lib().mcint_gradient_list(self.handle, None, None, 0, ctypes.byref(n)), "mcint_gradient_list")
+            cap = n.value
+        shls, refs = np.empty((cap, 4), np.int32), np.empty(cap, np.int32)
+        if cap:
+            _check(lib().mcint_gradient_list(self.handle, _ip(shls), _ip(refs), cap, ctypes.byref(n)),
                    "mcint_gradient_list")
-        return shls, refs
+        return shls[:n.value], refs[:n.value]
 
     def close(self):
         if self.handle:

@@ -419,10 +419,10 @@ struct PhaseTimer {
 #endif
 
 // Host threads for plan construction: at most 16 (one GPU's share of a
-// node), one per 200k quartets.
+// node), one per 16k quartets (a thread costs some 20 us, a quartet 50 ns).
 int host_threads(size_t n) {
   const unsigned hw = std::max(1u, std::thread::hardware_concurrency());
-  return (int)std::max<size_t>(1, std::min<size_t>({(size_t)16, (size_t)hw, n / 200000 + 1}));
+  return (int)std::max<size_t>(1, std::min<size_t>({(size_t)16, (size_t)hw, n / 16384 + 1}));
 }
 
 // f(thread, begin, end) over nthr contiguous ranges of [0, n)
