@@ -1252,11 +1252,7 @@ static int plan_create_impl(mcint_plan** out, mcint_basis* b, int intor, const F
       bk.sstride = chunked_block_doubles(kind, bk.la, bk.lb, bk.lc, bk.ld);
     } else if (bk.mode == 0) {
       const GenLayout G = gen_layout(kind, sph, bk.la, bk.lb, bk.lc, bk.ld, b->omega);
-      // four waves per task where a task holds many primitive quartets or the
-      // bucket is too short to give every SIMD a wave
-      const int64_t n = bk.t1 - bk.t0;
-      const int waves = np >= MM_WAVES_PRIMS * n || n < 1024 ? 4 : 1;
-      for (int w = waves; w >= 1 && !bk.mm; w -= 3)
+      for (int w = mm_waves(G, bk.t1 - bk.t0, np); w >= 1 && !bk.mm; w -= 3)
         bk.mm = mm_layout(kind, sph, bk.la, bk.lb, bk.lc, bk.ld, b->omega, w).waves;
       if (!gen_fits(G)) {
         plan_free(p);

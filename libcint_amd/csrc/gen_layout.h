@@ -179,10 +179,6 @@ inline GenLayout gen_layout(int kind, int sph, int la, int lb, int lc, int ld, d
   return g;
 }
 
-// Primitive quartets per task from which the matrix kernel takes four waves
-// per task instead of one.
-constexpr int MM_WAVES_PRIMS = 24;
-
 // Layout of the matrix kernel: X, then the walk's tables, each wave's Y and
 // the partial sums of shared components in one space, then the codes.
 inline GenLayout mm_layout(int kind, int sph, int la, int lb, int lc, int ld, double omega, int waves) {
@@ -219,6 +215,19 @@ inline GenLayout mm_layout(int kind, int sph, int la, int lb, int lc, int ld, do
   g.lds = g.oI + (ncode + g.nrow + g.ncol + 2 * waves + 1) / 2;
   g.waves = g.lds <= GEN_LDS_MAX ? waves : 0;
   return g;
+}
+
+// Waves per task of n tasks with np primitive quartets in all: four where a
+// task holds many, or the bucket is too short to give every SIMD a wave,
+// and the products of one task (components x roots x primitive quartets)
+// are enough to share.  Second derivatives of 20 shells / three-centre
+// derivatives of 186 shells: 11.4 / 5.1 ms; one wave everywhere below 64
+// primitive quartets 15.0 / 4.7, four from 8 primitive quartets and 1000
+// products 11.3 / 6.4, one and four by primitives and tasks alone 11.7 / 5.3.
+constexpr int64_t MM_PRIMS = 24, MM_TASKS = 1024, MM_WORK = 2000;
+inline int mm_waves(const GenLayout& g, int64_t n, int64_t np) {
+  const double work = (double)np * g.nE * g.nF * g.nrt;
+  return (np >= MM_PRIMS * n || n < MM_TASKS) && work >= (double)MM_WORK * n ? 4 : 1;
 }
 
 // One matrix to lay out: the bra matrix of the virtual pair (a, b) or the

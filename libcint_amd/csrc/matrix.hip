@@ -20,10 +20,10 @@
 // per batch) where tasks hold hundreds of primitive quartets, the set-up per
 // task where they hold one.  Measured against the generic kernel, whose
 // passes go term by term and whose tasks have one wave:
-//   int2e_ipip1 + int2e_ip1ip2 of 20 shells (168 000 quartets): 29.4 -> 12.6 ms
+//   int2e_ipip1 + int2e_ip1ip2 of 20 shells (168 000 quartets): 29.4 -> 11.4 ms
 //   ((pp|pp), 756 tasks of 330 primitive quartets: 4.2 -> 1.1 ms;
 //   (dd|dd), 160 tasks of one: 0.62 -> 0.05 ms)
-//   int3c2e_ip1 + int3c2e_ip2 of 186 shells: 5.53 -> 5.26 ms
+//   int3c2e_ip1 + int3c2e_ip2 of 186 shells: 5.53 -> 5.1 ms
 #include <algorithm>
 
 #include "gen_device.h"
@@ -39,12 +39,13 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Three waves per SIMD: at two (186 VGPRs, no spills) the second derivatives
-// of 20 shells take 16.9 ms instead of 12.6.
+// Waves per SIMD: one-wave workgroups at three (at two, 186 VGPRs and no
+// spills, second derivatives of 20 shells took 16.9 ms instead of 12.6),
+// four-wave workgroups at four (11.2 ms, 11.7 at three).
 // W waves per task; NRT roots (0: G.nrt, known at run time).
 template <int W, int NRT>
 __global__ void __launch_bounds__(64 * W)
-__attribute__((amdgpu_waves_per_eu(3)))
+__attribute__((amdgpu_waves_per_eu(W == 4 ? 4 : 3)))
 eri_matrix_kernel(BasisView B, BucketArgs A, GenLayout G, XferView XV) {
   constexpr int TH = 64 * W;
   extern __shared__ double sm[];
@@ -90,6 +91,8 @@ eri_matrix_kernel(BasisView B, BucketArgs A, GenLayout G, XferView XV) {
                       (three ? 1.0 : common_fac_sp(ld));
   const int nEF = G.nE * G.nF;
   const int te = tet_d(G.e_lo), tf = tet_d(G.f_lo);
+  // weights the row sets need: 2a_i, 4a_i^2 (bits 0, 1), 2a_k (bit 2)
+  const int wt = (G.nbc > 1 ? 1 : 0) | (G.nbc == 9 ? 2 : 0) | (G.nkc > 1 ? 4 : 0);
 
   for (int64_t t = A.t0 + blockIdx.x; t < A.t1; t += gridDim.x) {
     const Task tk = A.tasks[t];
@@ -145,36 +148,43 @@ eri_matrix_kernel(BasisView B, BucketArgs A, GenLayout G, XferView XV) {
     const int S = G.spread ? (int)((unsigned)TH / (unsigned)nEF) : 1;
     const int mys = G.spread ? (int)((unsigned)tid / (unsigned)nEF) : 0;
     double g0 = 0, g1 = 0, g2 = 0, h0 = 0, h1 = 0;
-    // products of component c over the batch's quartets q0, q0 + step, ...,
-    // with weights 1, 2a_i, 4a_i^2; the same times 2a_k
+    // products of one component over the batch's quartets q0, q0 + step, ...,
+    // with weights 1, 2a_i, 4a_i^2; the same times 2a_k: those that the row
+    // sets need (WT, uniform)
     auto products = [&](int ie, int jf, int q0, int step, int np) {
       const int ec = code[te + ie], fc = code[tf + jf];
-      const double* V = sV + q0 * VP;
       const int vx = ((ec & 15) * F1 + (fc & 15)) * nrt;
       const int vy = VD + (((ec >> 4) & 15) * F1 + ((fc >> 4) & 15)) * nrt;
       const int vz = 2 * VD + (((ec >> 8) & 15) * F1 + ((fc >> 8) & 15)) * nrt;
-      for (int q = q0; q < np; q += step) {
-        double g = 0;
-        if constexpr (NRT != 0) {
+      auto run = [&](auto WT) {
+        constexpr int wt = decltype(WT)::value;
+        const double* V = sV + q0 * VP;
+#pragma unroll 2
+        for (int q = q0; q < np; q += step) {
+          double g = 0;
+          if constexpr (NRT != 0) {
 #pragma unroll
-          for (int r = 0; r < NRT; ++r) g = fma(V[vx + r] * V[vy + r], V[vz + r], g);
-        } else {
-          for (int r = 0; r < nrt; ++r) g = fma(V[vx + r] * V[vy + r], V[vz + r], g);
+            for (int r = 0; r < NRT; ++r) g = fma(V[vx + r] * V[vy + r], V[vz + r], g);
+          } else {
+            for (int r = 0; r < nrt; ++r) g = fma(V[vx + r] * V[vy + r], V[vz + r], g);
+          }
+          g0 += g;
+          if constexpr (wt & 1) g1 = fma(g, sp[q].w[0], g1);
+          if constexpr (wt & 2) g2 = fma(g, sp[q].w[1], g2);
+          if constexpr (wt & 4) {
+            const double h = g * sp[q].w[2];
+            h0 += h;
+            if constexpr (wt & 1) h1 = fma(h, sp[q].w[0], h1);
+          }
+          V += step * VP;
         }
-        g0 += g;
-        if (G.nbs > 1) {
-          g1 = fma(g, sp[q].w[0], g1);
-          if (G.nbc == 9) g2 = fma(g, sp[q].w[1], g2);
-        } else if (G.nbc > 1) {  // a lone raised set (no lowered shell)
-          g1 = fma(g, sp[q].w[0], g1);
-          g2 = fma(g, sp[q].w[1], g2);
-        }
-        if (G.nkc > 1) {
-          const double h = g * sp[q].w[2];
-          h0 += h;
-          h1 = fma(h, sp[q].w[0], h1);
-        }
-        V += step * VP;
+      };
+      switch (wt) {
+        case 0: run(std::integral_constant<int, 0>{}); break;
+        case 1: run(std::integral_constant<int, 1>{}); break;
+        case 3: run(std::integral_constant<int, 3>{}); break;
+        case 4: run(std::integral_constant<int, 4>{}); break;
+        default: run(std::integral_constant<int, 5>{}); break;
       }
     };
     // adds a component's sums to the sets it belongs to
