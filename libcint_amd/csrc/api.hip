@@ -1588,6 +1588,7 @@ static BucketArgs bucket_args(const mcint_plan* p, const Bucket& bk, double* out
   A.grad_refs = 0;
   A.jk_j = nullptr;
   A.jk_k = nullptr;
+  A.jk_rows = 0;
   A.col_major = 0;
   return A;
 }
@@ -2651,6 +2652,7 @@ int opt_tuple(OptDevice* d, int intor, const FINT* shls, double* blk_out) {
   A.nslot = 1;
   A.jk_j = nullptr;
   A.jk_k = nullptr;
+  A.jk_rows = 0;
   A.col_major = 0;
   e = hipMemcpyAsync(c->task_d, c->task_h, sizeof(Task) * nt, hipMemcpyHostToDevice, c->stream);
   if (e == hipSuccess)

@@ -152,6 +152,7 @@ struct BucketArgs {
   // J' (jk_j) and K' (jk_k), nao x nao row-major, density dm (copies as above)
   double* jk_j;
   double* jk_k;
+  int jk_rows;           // single-chunk kernels: rows of K' in LDS (JkRows)
 };
 
 __host__ __device__ constexpr int ncart(int l) { return (l + 1) * (l + 2) / 2; }
