@@ -104,7 +104,7 @@ def cpu_baseline(basis_np, quartets, target_s=12.0, max_threads=16):
 def sampled_check(db, B, plan, quart, out, per_bucket=2, seed=7) -> dict:
     """Blocks of per_bucket tasks at random positions of every bucket, read
     from the timed run's output, against the same quartets recomputed by the
-    generic kernel (a separate implementation: runtime class, recurrences in
+    matrix kernel (a separate implementation: runtime class, recurrences in
     LDS; the parity tests pin both to the oracle)."""
     import torch
     import libcint_amd as mc
@@ -131,7 +131,7 @@ def sampled_check(db, B, plan, quart, out, per_bucket=2, seed=7) -> dict:
     gp.close()
     err = np.abs(got - ref)
     return {"quartets": int(idx.size), "buckets": len(plan.buckets()),
-            "reference": "generic kernel on the same quartets",
+            "reference": "matrix kernel on the same quartets",
             "max_abs_err": float(err.max()),
             "max_rel_err": float((err / np.maximum(np.abs(ref), 1e-300)).max()),
             "within_1e-12_abs_1e-10_rel": bool(np.all(err <= 1e-12 + 1e-10 * np.abs(ref)))}
@@ -207,7 +207,7 @@ def gradient_section(reps: int = 3) -> dict:
     g32_err = float((g32 - g).abs().max())
     gp32.close()
     # the plain FP64 GPU path for the same work: every quartet on the
-    # generic kernel (one workgroup per quartet, runtime class, no register
+    # matrix kernel (one workgroup per quartet, runtime class, no register
     # kernels, no FP32 tier); one run each
     old = mc.tune(mc.TUNE_GENERIC_ONLY, 1)
     try:
@@ -261,7 +261,7 @@ def gradient_section(reps: int = 3) -> dict:
                                                    / (t_plain + t_jk32 + t_grad32),
             "speedup_mixed_vs_fp64_batched": (t_plain + t_jk + t_grad) / (t_plain + t_jk32 + t_grad32),
             "plain_fp64_generic_max_abs_diff_jk_grad": gen_err,
-            "definition": "plain FP64 GPU path = every quartet on the generic kernel (one "
+            "definition": "plain FP64 GPU path = every quartet on the matrix kernel (one "
                           "workgroup per quartet, runtime class, FP64); batched mixed = class "
                           "buckets on the register kernels in concurrent graph branches with "
                           "the FP32 tier for Schwarz x max|D|^2 < 1e-7",
@@ -290,7 +290,8 @@ def fused_jk_section(plan, m, reps: int, t_step: float) -> dict:
     return {"workload": f"{m.name}: J and K for a random density D = A A^T / N, {nao} AOs",
             "ms": dt * 1e3, "eri_step_ms": t_step * 1e3, "vs_eri_step": dt / t_step,
             "eri_buffer_bytes": 0, "energy": e,
-            "device_memory_beyond_plan_bytes": 2 * nao * nao * 8}
+            # eight copies of the half matrices J', K'
+            "device_memory_beyond_plan_bytes": 8 * 2 * nao * nao * 8}
 
 
 def c2_section(reps: int = 2) -> dict:

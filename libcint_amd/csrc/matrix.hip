@@ -63,7 +63,7 @@ eri_matrix_kernel(BasisView B, BucketArgs A, GenLayout G, XferView XV) {
   int* const code = reinterpret_cast<int*>(sm + G.oI);  // exponents of the components
   int* const rt = code + ncode;    // output functions and component of each block row
   int* const ct = rt + G.nrow;     // ... and column, a | b << 8 | component << 16
-  int* const scnt = ct + G.ncol;   // survivors of each wave, two rounds
+  int* const scnt = ct + G.ncol;   // survivors of each wave, twice
   for (int i = tid; i < ncode; i += TH) {
     int l = 0, k = i;
     while (k >= ncart(l)) { k -= ncart(l); ++l; }
@@ -231,7 +231,7 @@ eri_matrix_kernel(BasisView B, BucketArgs A, GenLayout G, XferView XV) {
       int nsurv = __popcll(mask);
       int slot = __popcll(mask & ((1ull << ln) - 1));
       if constexpr (W > 1) {
-        // counts of this round; the next round's go beside them, since a wave
+        // counts of these candidates; the next ones go beside them, since a wave
         // may be one barrier ahead of another's reads
         int* const cnt = scnt + odd;
         if (ln == 0) cnt[wave] = nsurv;

@@ -141,15 +141,13 @@ def test_gradient_list(mc, case):
     np.testing.assert_allclose(got, ref, rtol=0, atol=1e-10 * max(1.0, np.abs(ref).max()))
 
 
-@pytest.mark.parametrize("omega", [0.0, 0.4, -0.4])
-@pytest.mark.parametrize("name", ["int2e_ipip1_sph", "int2e_ipip1_cart", "int2e_ip1ip2_sph", "int2e_ip1ip2_cart",
-                                  "int3c2e_ip1_sph", "int3c2e_ip2_cart", "int2c2e_sph", "int2e_cart"])
+@pytest.mark.parametrize("name,omega", [(n, w) for n in (
+    "int2e_ipip1_sph", "int2e_ipip1_cart", "int2e_ip1ip2_sph", "int2e_ip1ip2_cart", "int3c2e_ip1_sph",
+    "int3c2e_ip2_cart", "int2c2e_sph") for w in (0.0, 0.4, -0.4)] + [("int2e_cart", -0.4)])
 def test_matrix_kernel(mc, orc, name, omega):
     """Plans on the matrix kernel: every order of s, p, d (and one f, one g)
     shells, one and four waves per task (buckets below and above 1024 tasks),
     1 to 4096 primitive quartets, all operators."""
-    if name == "int2e_cart" and omega >= 0:
-        pytest.skip("register kernels serve it")
     m = make_molecule("c4" if "c2e" in name else "c1")
     rng = np.random.default_rng(12)
     ls, three = m.bas[:, 1], "c2e" in name
