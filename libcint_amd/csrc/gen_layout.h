@@ -198,11 +198,16 @@ inline GenLayout mm_layout(int kind, int sph, int la, int lb, int lc, int ld, do
   g.YS = g.CT1 * 16 + 1;
   g.nXz = g.KS * 4 * g.KF;
   g.spread = 2 * g.nE * g.nF <= threads;
-  // a batch: enough (primitive, direction, root) recurrences for the lanes
+  // A batch: two (primitive, direction, root) recurrences per lane, so that
+  // its barriers are shared by more primitive quartets, in tables that leave
+  // the LDS to several workgroups.  Second derivatives of 20 shells / three-
+  // centre derivatives of 186 shells: 10.9 / 4.95 ms; one recurrence per lane
+  // 11.3 / 5.1; four 10.8 / 5.2; tables of 24 and 16 KB (four waves, one)
+  // 11.2 / 4.9, of 32 and 16 KB 10.8 / 5.1.
   const int VT = 3 * g.nrt * (g.E + 1) * (g.F + 1);
   const int PV = VT + 2 * g.nrt + GEN_PRIM_D;
   g.PB = 1;
-  while (g.PB < 16 * waves && g.PB * 3 * g.nrt < threads && (g.PB + 1) * PV <= (waves > 1 ? 4096 : 2048)) ++g.PB;
+  while (g.PB < 16 * waves && g.PB * 3 * g.nrt < 2 * threads && (g.PB + 1) * PV <= (waves > 1 ? 3584 : 1536)) ++g.PB;
   int space = g.PB * PV;
   if (waves * 16 * g.YS > space) space = waves * 16 * g.YS;
   if (g.spread && 5 * threads > space) space = 5 * threads;
