@@ -181,7 +181,9 @@ struct Arena {
 
 // dst (pageable) = bytes of src (device) after the work on stream; returns
 // when the copy is done.  Threads take the chunks in turn: the host's part
-// (page faults of a fresh array, the copy out) is the longer one.
+// (page faults of a fresh array, the copy out) is the longer one.  This thread
+// waits for the work first: hipStreamPerThread is another stream in each of
+// them, so that the handle alone would not order their copies after it.
 hipError_t to_host(void* dst, const void* src, size_t bytes, hipStream_t stream) {
   const size_t chunks = (bytes + Stage::BYTES - 1) / Stage::BYTES;
   int dev = 0;
@@ -189,6 +191,8 @@ hipError_t to_host(void* dst, const void* src, size_t bytes, hipStream_t stream)
     const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream);
     return e == hipSuccess ? hipStreamSynchronize(stream) : e;
   }
+  const hipError_t done = hipStreamSynchronize(stream);
+  if (done != hipSuccess) return done;
   std::atomic<size_t> next{0};
   std::atomic<int> failed{(int)hipSuccess};
   auto work = [&] {
@@ -213,8 +217,7 @@ hipError_t to_host(void* dst, const void* src, size_t bytes, hipStream_t stream)
   }
   work();
   for (auto& x : th) x.join();
-  const hipError_t e = hipStreamSynchronize(stream);
-  return e == hipSuccess ? (hipError_t)failed.load() : e;
+  return (hipError_t)failed.load();
 }
 
 int intor_kind(int intor) {
