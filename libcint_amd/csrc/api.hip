@@ -23,6 +23,7 @@
 #include <chrono>
 #include <memory>
 #include <mutex>
+#include <new>
 #include <string>
 #include <thread>
 #include <vector>
@@ -68,10 +69,12 @@ template <typename T, int MAX>
 struct Kept {
   std::mutex m;
   std::vector<std::unique_ptr<T>> idle;
+  Kept() { idle.reserve(MAX); }  // so that giving back never throws
   // one made on the current device, or nullptr
   std::unique_ptr<T> take() {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return nullptr;
+    std::unique_ptr<T> other;  // makes room; destroyed outside the lock
     {
       std::lock_guard<std::mutex> g(m);
       for (size_t i = idle.size(); i-- > 0;)
@@ -80,10 +83,18 @@ struct Kept {
           idle.erase(idle.begin() + i);
           return t;
         }
+      if (idle.size() == (size_t)MAX) {
+        other = std::move(idle.front());
+        idle.erase(idle.begin());
+      }
     }
-    std::unique_ptr<T> t(new T);
+    other.reset();
+    std::unique_ptr<T> t(new (std::nothrow) T);
+    if (!t) return nullptr;
     t->device = dev;
-    return t->make() ? std::move(t) : nullptr;
+    if (t->make()) return t;
+    (void)hipGetLastError();  // the caller goes on without one
+    return nullptr;
   }
   void give(std::unique_ptr<T> t) {
     if (!t) return;
@@ -100,21 +111,28 @@ struct Kept {
 // Pinned memory that pageable host data passes through.  A copy of more than
 // about a megabyte from or to pageable memory makes the runtime pin the
 // caller's pages: the 1.1 MB task list of a 72 000-quartet batch took 4 ms.
+// At most STAGES exist, in use or kept; who gets none copies without.
+constexpr int STAGES = 16;
+std::atomic<int> g_stage_limit{STAGES};
 struct Stage {
   static constexpr size_t BYTES = 2 << 20;
+  static std::atomic<int> live;
   int device = 0;
   char* p = nullptr;
   hipEvent_t ev = nullptr;
+  Stage() { ++live; }
   bool make() {
-    return hipHostMalloc((void**)&p, BYTES) == hipSuccess &&
+    return live <= g_stage_limit && hipHostMalloc((void**)&p, BYTES) == hipSuccess &&
            hipEventCreateWithFlags(&ev, hipEventDisableTiming) == hipSuccess;
   }
   ~Stage() {
     if (ev) (void)hipEventDestroy(ev);
     if (p) (void)hipHostFree(p);
+    --live;
   }
 };
-using Stages = Kept<Stage, 16>;
+std::atomic<int> Stage::live{0};
+using Stages = Kept<Stage, STAGES>;
 constexpr size_t STAGE_MIN = 256 << 10;  // smaller copies go directly
 
 // dst (device) = n elements of src (pageable), on the null stream; returns
@@ -184,40 +202,41 @@ struct Arena {
 // (page faults of a fresh array, the copy out) is the longer one.  This thread
 // waits for the work first: hipStreamPerThread is another stream in each of
 // them, so that the handle alone would not order their copies after it.
+// A thread without a staging buffer leaves its chunks to the others.
 hipError_t to_host(void* dst, const void* src, size_t bytes, hipStream_t stream) {
   const size_t chunks = (bytes + Stage::BYTES - 1) / Stage::BYTES;
   int dev = 0;
-  if (chunks < 2 || hipGetDevice(&dev) != hipSuccess) {
-    const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream);
-    return e == hipSuccess ? hipStreamSynchronize(stream) : e;
-  }
-  const hipError_t done = hipStreamSynchronize(stream);
-  if (done != hipSuccess) return done;
-  std::atomic<size_t> next{0};
-  std::atomic<int> failed{(int)hipSuccess};
-  auto work = [&] {
-    hipError_t r = hipSetDevice(dev);
-    std::unique_ptr<Stage> x = r == hipSuccess ? Stages::get().take() : nullptr;
-    if (r == hipSuccess && !x) r = hipErrorOutOfMemory;
-    for (size_t c; r == hipSuccess && (c = next.fetch_add(1)) < chunks;) {
-      const size_t o = c * Stage::BYTES, k = std::min(Stage::BYTES, bytes - o);
-      r = hipMemcpyAsync(x->p, (const char*)src + o, k, hipMemcpyDeviceToHost, stream);
-      if (r == hipSuccess) r = hipEventRecord(x->ev, stream);
-      if (r == hipSuccess) r = hipEventSynchronize(x->ev);
-      if (r == hipSuccess) memcpy((char*)dst + o, x->p, k);
+  if (chunks > 1 && hipGetDevice(&dev) == hipSuccess) {
+    const hipError_t done = hipStreamSynchronize(stream);
+    if (done != hipSuccess) return done;
+    std::atomic<size_t> next{0};
+    std::atomic<int> failed{(int)hipSuccess};
+    auto work = [&] {
+      std::unique_ptr<Stage> x = hipSetDevice(dev) == hipSuccess ? Stages::get().take() : nullptr;
+      if (!x) return;
+      hipError_t r = hipSuccess;
+      for (size_t c; r == hipSuccess && (c = next.fetch_add(1)) < chunks;) {
+        const size_t o = c * Stage::BYTES, k = std::min(Stage::BYTES, bytes - o);
+        r = hipMemcpyAsync(x->p, (const char*)src + o, k, hipMemcpyDeviceToHost, stream);
+        if (r == hipSuccess) r = hipEventRecord(x->ev, stream);
+        if (r == hipSuccess) r = hipEventSynchronize(x->ev);
+        if (r == hipSuccess) memcpy((char*)dst + o, x->p, k);
+      }
+      if (r != hipSuccess) failed = (int)r;
+      else Stages::get().give(std::move(x));
+    };
+    std::vector<std::thread> th;
+    try {
+      th.reserve(8);
+      while (th.size() + 1 < std::min<size_t>(8, chunks)) th.emplace_back(work);
+    } catch (...) {  // fewer threads, then
     }
-    if (r != hipSuccess) failed = (int)r;
-    else Stages::get().give(std::move(x));
-  };
-  std::vector<std::thread> th;
-  th.reserve(8);
-  try {
-    while (th.size() + 1 < std::min<size_t>(8, chunks)) th.emplace_back(work);
-  } catch (...) {  // fewer threads, then
+    work();
+    for (auto& x : th) x.join();
+    if (next > 0) return (hipError_t)failed.load();
   }
-  work();
-  for (auto& x : th) x.join();
-  return (hipError_t)failed.load();
+  const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream);
+  return e == hipSuccess ? hipStreamSynchronize(stream) : e;
 }
 
 int intor_kind(int intor) {
@@ -2241,6 +2260,16 @@ int mcint::plan_build_host_only(const FINT* atm, FINT natm, const FINT* bas, FIN
 }
 
 void mcint::set_error(const char* msg) { set_err(msg); }
+
+int mcint::stage_limit(int n) {
+  Stages& k = Stages::get();
+  std::lock_guard<std::mutex> g(k.m);
+  const int old = g_stage_limit.exchange(n);
+  k.idle.clear();
+  return old;
+}
+
+int mcint::stages_live() { return Stage::live; }
 
 // ---------------------------------------------------------------------------
 // Host-pointer batches

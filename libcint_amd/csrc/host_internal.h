@@ -35,4 +35,10 @@ int plan_build_host_only(const FINT* atm, FINT natm, const FINT* bas, FINT nbas,
 // Sets the calling thread's mcint_last_error() text.
 void set_error(const char* msg);
 
+// Pinned staging buffers of host transfers: sets how many may exist (default
+// 16; 0: every transfer goes without), gives up the idle ones and returns the
+// previous bound; the buffers that exist.  For tests.
+int stage_limit(int n);
+int stages_live();
+
 }  // namespace mcint

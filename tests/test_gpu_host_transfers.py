@@ -66,3 +66,30 @@ def test_batch_on_the_per_thread_stream(mc, case, callers):
         t.join()
     for g in got:
         _same(g, case)
+
+
+@pytest.mark.parametrize("limit", [0, 1, 3, 16])
+def test_batch_without_staging_buffers(mc, case, limit):
+    """Threads that get no pinned buffer leave their part to the others, and a
+    transfer that gets none goes without; no more exist than the bound."""
+    B, q, out, _ = case
+    L = mc.lib()
+    set_limit, live = L._ZN5mcint11stage_limitEi, L._ZN5mcint11stages_liveEv
+    old = set_limit(limit)
+    try:
+        assert live() == 0
+        got = [None] * 3
+
+        def work(i):
+            got[i] = _batch(mc, B, q, out.size, None)
+
+        threads = [threading.Thread(target=work, args=(i,)) for i in range(3)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert live() <= limit
+    finally:
+        set_limit(old)
+    for g in got:
+        _same(g, case)
