@@ -25,6 +25,7 @@
 #include <mutex>
 #include <new>
 #include <string>
+#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -447,19 +448,25 @@ int host_threads(size_t n) {
   return (int)std::max<size_t>(1, std::min<size_t>({(size_t)16, (size_t)hw, n / 16384 + 1}));
 }
 
-// f(thread, begin, end) over nthr contiguous ranges of [0, n)
+// f(thread, begin, end) over nthr contiguous ranges of [0, n); ranges whose
+// thread cannot be started run on this one
 template <typename F>
 void parallel_for(int nthr, size_t n, F&& f) {
+  auto range = [&](int t) {
+    f(t, n * (size_t)t / (size_t)nthr, n * (size_t)(t + 1) / (size_t)nthr);
+  };
   if (nthr <= 1) {
     f(0, (size_t)0, n);
     return;
   }
   std::vector<std::thread> th;
   th.reserve(nthr);
-  for (int t = 0; t < nthr; ++t) {
-    const size_t a = n * (size_t)t / (size_t)nthr, e = n * (size_t)(t + 1) / (size_t)nthr;
-    th.emplace_back([&f, t, a, e] { f(t, a, e); });
+  int t = 0;
+  try {
+    for (; t < nthr; ++t) th.emplace_back([&range, t] { range(t); });
+  } catch (const std::system_error&) {
   }
+  for (; t < nthr; ++t) range(t);
   for (auto& x : th) x.join();
 }
 
