@@ -432,6 +432,10 @@ int mcint_schwarz(mcint_basis *b, int nshell, double *q);
  * MCINT_TUNE_FILL_LANES: a class of a plan whose teams put fewer lanes than
  * this to work has them widened (up to one wave per quartet); 0 keeps the
  * tuned primitive quartets per lane, as for tuning them.
+ * MCINT_TUNE_MATRIX_KIB (default 2097152, 2 GiB): bound of the transfer
+ * matrices that a plan lays out for its runtime classes; the costliest
+ * classes have theirs first, and classes whose matrices no longer fit (all
+ * with 0) run on the generic kernel, which forms the transfers term by term.
  * Applies to plans created afterwards; returns the previous value, or a
  * negative status. */
 #define MCINT_TUNE_PRIMS_PER_LANE 0
@@ -439,6 +443,7 @@ int mcint_schwarz(mcint_basis *b, int nshell, double *q);
 #define MCINT_TUNE_GRAPH_BRANCHES 2
 #define MCINT_TUNE_WAVE_KERNELS 3
 #define MCINT_TUNE_FILL_LANES 4
+#define MCINT_TUNE_MATRIX_KIB 5
 int mcint_tune(int key, int value);
 /* Per-class override of MCINT_TUNE_PRIMS_PER_LANE for one integral kind
  * (intor code) and canonical class (la >= lb, lc >= ld, (la,lb) >= (lc,ld)

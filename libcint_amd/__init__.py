@@ -165,6 +165,7 @@ TUNE_GENERIC_ONLY = 1
 TUNE_GRAPH_BRANCHES = 2
 TUNE_WAVE_KERNELS = 3
 TUNE_FILL_LANES = 4
+TUNE_MATRIX_KIB = 5
 
 
 def tune(key: int, value: int) -> int:

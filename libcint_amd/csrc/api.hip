@@ -674,10 +674,10 @@ double bucket_cost(int kind, int mode, int la, int lb, int lc, int ld, int64_t n
 // largest c1 bucket, 695,543 (fd|dp) quartets x 736 doubles, fits), 16 GiB
 // over four branches, allocated only up to what the plan needs.
 constexpr int64_t GEN_SCRATCH_DOUBLES = 512ll << 20;
-// Bound of a plan's transfer matrices (doubles, 2 GiB): 126 KB for a d pair's
-// second derivative, so 17 000 such pairs; beyond it the generic path forms
-// its transfers term by term.
-constexpr int64_t XFER_DOUBLES = 256ll << 20;
+// Bound of a plan's transfer matrices (KiB, mcint_tune MCINT_TUNE_MATRIX_KIB):
+// 2 GiB hold the bra matrices of 15 500 spherical d pairs' second derivatives
+// (int2e_ipip1: 10 x 27 tiles of 64 doubles, 138 KB) without any ket matrix.
+int g_matrix_kib = 2 << 20;
 // copies of the gradient accumulators (spreads the digest's atomics)
 constexpr int GRAD_SLOTS = 64;
 // Copies of J', K' that the fused digest adds into, block b to copy b % 8, in
@@ -846,6 +846,7 @@ struct mcint_plan {
   // ordered virtual pair (bra, then ket)
   double* xfer_d = nullptr;
   int64_t* xfer_off_d = nullptr;
+  int64_t xfer_size = 0;  // doubles
   double* gslots_d = nullptr;  // gradient digest accumulators
   double* jk_d = nullptr;      // J', K' half matrices of the fused J/K digest
   int64_t jk_n = 0;            // doubles they hold
@@ -964,8 +965,84 @@ extern "C" int mcint_tune(int key, int value) {
     g_fill_lanes = value;
     return old;
   }
+  if (key == MCINT_TUNE_MATRIX_KIB) {
+    if (value < 0) {
+      set_err("mcint_tune: MCINT_TUNE_MATRIX_KIB must not be negative");
+      return MCINT_ERR_ARG;
+    }
+    const int old = g_matrix_kib;
+    g_matrix_kib = value;
+    return old;
+  }
   set_err("mcint_tune: unknown key");
   return MCINT_ERR_ARG;
+}
+
+// Moves a runtime-class launch from the matrix kernel to the generic one.
+static void off_matrix(const mcint_plan* p, Bucket& bk) {
+  if (!bk.mm) return;
+  bk.mm = 0;
+  bk.sstride = gen_layout(p->kind, p->sph, bk.la, bk.lb, bk.lc, bk.ld, p->b->omega).nblk;
+}
+
+// Transfer matrices of a plan: what to lay out, and the offsets by ordered
+// virtual pair (bra, then ket; -1: none).
+struct Matrices {
+  std::vector<XferItem> items;
+  std::vector<int64_t> off;
+  int64_t size = 0;  // doubles
+};
+
+// The matrices of the plan's matrix launches, the costliest launch first;
+// one whose pairs no longer fit the bound goes to the generic kernel (2.7
+// times slower: 29.4 against 10.9 ms for the second derivatives of 20
+// shells), and only it.
+static void admit_matrices(mcint_plan* p, const Task* tasks, Matrices& X) {
+  const int kind = p->kind, nv = p->b->nv;
+  const int64_t nn = (int64_t)nv * nv, bound = (int64_t)g_matrix_kib * 128;
+  std::vector<Bucket*> order;
+  for (Bucket& bk : p->launches)
+    if (bk.mm) order.push_back(&bk);
+  if (order.empty()) return;
+  std::stable_sort(order.begin(), order.end(), [](const Bucket* x, const Bucket* y) { return x->cost > y->cost; });
+  X.off.assign(2 * (size_t)nn, -1);
+  std::vector<uint8_t> seen(2 * (size_t)nn, 0);
+  for (Bucket* bk : order) {
+    const GenLayout G = mm_layout(kind, p->sph, bk->la, bk->lb, bk->lc, bk->ld, p->b->omega, bk->mm);
+    const int nthr = host_threads((size_t)(bk->t1 - bk->t0));
+    std::vector<std::vector<int64_t>> found(nthr);  // pairs without a matrix so far
+    parallel_for(nthr, (size_t)(bk->t1 - bk->t0), [&](int th, size_t t0, size_t t1) {
+      auto need = [&](int64_t at) {
+        if (!__atomic_load_n(&seen[at], __ATOMIC_RELAXED) && !__atomic_exchange_n(&seen[at], (uint8_t)1, __ATOMIC_RELAXED))
+          found[th].push_back(at);
+      };
+      for (size_t t = t0; t < t1; ++t) {
+        const int16_t* s = tasks[bk->t0 + t].sh;
+        need((int64_t)s[0] * nv + s[1]);
+        need(nn + (int64_t)s[2] * nv + (kind_three(kind) ? s[2] : s[3]));
+      }
+    });
+    std::vector<int64_t> pairs;
+    for (const auto& f : found) pairs.insert(pairs.end(), f.begin(), f.end());
+    const int64_t bra = (int64_t)G.RT * G.KS * 64, ket = (int64_t)G.CT2 * G.KS2 * 64;
+    int64_t more = 0;
+    for (int64_t at : pairs) more += at < nn ? bra : ket;
+    if (X.size + more > bound) {
+      for (int64_t at : pairs) seen[at] = 0;
+      for (Bucket& o : p->buckets)  // a runtime class is one bucket and one launch
+        if (o.mode == 0 && o.t0 == bk->t0) off_matrix(p, o);
+      off_matrix(p, *bk);
+      continue;
+    }
+    std::sort(pairs.begin(), pairs.end());
+    for (int64_t at : pairs) {
+      const bool k = at >= nn;
+      const int s = (int)((at - (k ? nn : 0)) / nv), s2 = (int)((at - (k ? nn : 0)) % nv);
+      X.off[at] = X.size;
+      X.items.push_back(XferItem{s, s2, k, k ? G.CT2 : G.RT, k ? G.KS2 : G.KS, X.size});
+      X.size += k ? ket : bra;
+    }
+  }
 }
 
 // upload = false returns the plan after its host stage (buckets, task list,
@@ -1266,7 +1343,6 @@ static int plan_create_impl(mcint_plan** out, mcint_basis* b, int intor, const F
     });
   }
   timer.mark("order small-team buckets by primitive count");
-  int64_t max_gen = 0, max_flags = 0;
   for (size_t i = 0; i < nkeys; ++i) {
     const uint32_t k = ukeys[i];
     Bucket bk;
@@ -1326,46 +1402,23 @@ static int plan_create_impl(mcint_plan** out, mcint_basis* b, int intor, const F
                            p->buckets.back().team == bk.team);
     p->buckets.back().lanes = bk.team;
   }
-  // transfer matrices of the generic path's pairs: sizes, offsets
   const int nv = b->nv;
-  std::vector<XferItem> xitems;
-  std::vector<int64_t> xoff;
-  int64_t xsize = 0;
-  for (const Bucket& bk : p->launches) {
-    if (!bk.mm) continue;
-    if (xoff.empty()) xoff.assign(2 * (size_t)nv * nv, -1);
-    const GenLayout G = mm_layout(kind, sph, bk.la, bk.lb, bk.lc, bk.ld, b->omega, bk.mm);
-    auto need = [&](int64_t at, int s, int s2, int ket, int rows, int ks) {
-      if (xoff[at] >= 0) return;
-      xoff[at] = xsize;
-      xitems.push_back(XferItem{s, s2, ket, rows, ks, xsize});
-      xsize += (int64_t)rows * ks * 64;
-    };
-    for (int64_t t = bk.t0; t < bk.t1; ++t) {
-      const int16_t* s = sorted[t].sh;
-      const int s3 = kind_three(kind) ? s[2] : s[3];
-      need((int64_t)s[0] * nv + s[1], s[0], s[1], 0, G.RT, G.KS);
-      need((int64_t)nv * nv + (int64_t)s[2] * nv + s3, s[2], s3, 1, G.CT2, G.KS2);
-    }
-  }
-  if (xsize > XFER_DOUBLES) {
-    xitems.clear();
-    for (auto* list : {&p->buckets, &p->launches})
-      for (Bucket& bk : *list) {
-        if (!bk.mm) continue;
-        bk.mm = 0;
-        bk.sstride = gen_layout(kind, sph, bk.la, bk.lb, bk.lc, bk.ld, b->omega).nblk;
-      }
-  }
+  Matrices X;
+  admit_matrices(p, sorted.get(), X);
+  p->xfer_size = X.size;
   timer.mark("transfer matrices");
-  for (const auto* list : {&p->buckets, &p->launches})
-    for (const Bucket& bk : *list) {
-      if (bk.mode == 1) continue;
-      const int64_t n = std::max<int64_t>(1, std::min<int64_t>(bk.t1 - bk.t0,
-                                              GEN_SCRATCH_DOUBLES / std::max<int64_t>(1, bk.sstride)));
-      max_gen = std::max(max_gen, n * bk.sstride);
-      if (bk.mode == 2) max_flags = std::max(max_flags, n);
-    }
+  auto size_scratch = [&] {
+    p->scratch_size = p->flags_size = 0;
+    for (const auto* list : {&p->buckets, &p->launches})
+      for (const Bucket& bk : *list) {
+        if (bk.mode == 1) continue;
+        const int64_t n = std::max<int64_t>(1, std::min<int64_t>(bk.t1 - bk.t0,
+                                                GEN_SCRATCH_DOUBLES / std::max<int64_t>(1, bk.sstride)));
+        p->scratch_size = std::max(p->scratch_size, n * bk.sstride);
+        if (bk.mode == 2) p->flags_size = std::max(p->flags_size, n);
+      }
+  };
+  size_scratch();
   p->stats[0] = p->ntasks;
   p->stats[1] = (int64_t)p->buckets.size();
 
@@ -1396,8 +1449,6 @@ static int plan_create_impl(mcint_plan** out, mcint_basis* b, int intor, const F
       pairs.push_back(c);
     }
   if (!upload) {
-    p->scratch_size = max_gen;
-    p->flags_size = max_flags;
     *out = p;
     return MCINT_OK;
   }
@@ -1418,21 +1469,27 @@ static int plan_create_impl(mcint_plan** out, mcint_basis* b, int intor, const F
   p->pp_pos_d = (int*)(p->mem_d + os);
   int* const pairs_d = (int*)(tmp_d + xp);
   PairPrim* const pp_tmp = (PairPrim*)(tmp_d + xt);
-  p->scratch_size = max_gen;
-  p->flags_size = max_flags;
   if (e == hipSuccess)
     e = launch_pairdata(b->vsh_d, b->env_d, nv, pairs_d, (int)(pairs.size() / 2), p->pair_off_d,
                         p->pair_ld_d, pp_tmp, p->pp_d, p->pp_pos_d, nullptr);
   XferItem* items_d = nullptr;
-  if (!xitems.empty()) {
-    if (e == hipSuccess) e = dalloc(&items_d, xitems.size());
-    if (e == hipSuccess) e = dalloc(&p->xfer_d, (size_t)xsize);
-    if (e == hipSuccess) e = dalloc(&p->xfer_off_d, xoff.size());
-    if (e == hipSuccess)
-      e = to_device(items_d, xitems.data(), xitems.size());
-    if (e == hipSuccess) e = to_device(p->xfer_off_d, xoff.data(), xoff.size());
-    if (e == hipSuccess)
-      e = launch_xfer(b->vsh_d, kind, sph, items_d, (int)xitems.size(), p->xfer_d, nullptr);
+  if (e == hipSuccess && !X.items.empty()) {
+    if (dalloc(&items_d, X.items.size()) != hipSuccess || dalloc(&p->xfer_d, (size_t)X.size) != hipSuccess ||
+        dalloc(&p->xfer_off_d, X.off.size()) != hipSuccess) {
+      // no room for the matrices: the generic kernel does without
+      (void)hipGetLastError();
+      dfree(p->xfer_d);
+      dfree(p->xfer_off_d);
+      p->xfer_size = 0;
+      for (auto* list : {&p->buckets, &p->launches})
+        for (Bucket& bk : *list) off_matrix(p, bk);
+      size_scratch();
+    } else {
+      e = to_device(items_d, X.items.data(), X.items.size());
+      if (e == hipSuccess) e = to_device(p->xfer_off_d, X.off.data(), X.off.size());
+      if (e == hipSuccess)
+        e = launch_xfer(b->vsh_d, kind, sph, items_d, (int)X.items.size(), p->xfer_d, nullptr);
+    }
   }
   if (e == hipSuccess) e = hipDeviceSynchronize();
   timer.mark("device upload, pair data");
@@ -2260,6 +2317,25 @@ int mcint::plan_build_host_only(const FINT* atm, FINT natm, const FINT* bas, FIN
         bucket_info->insert(bucket_info->end(), info, info + 8);
       }
     }
+    plan_free(p);
+  }
+  mcint_basis_destroy(b);
+  return st;
+}
+
+int mcint::plan_matrices_host_only(const FINT* atm, FINT natm, const FINT* bas, FINT nbas, const double* env,
+                                   int intor, const FINT* shls, size_t nq, int64_t* n) {
+  mcint_basis* b = nullptr;
+  int st = basis_create_impl(&b, atm, natm, bas, nbas, env, false);
+  if (st != MCINT_OK) return st;
+  mcint_plan* p = nullptr;
+  st = plan_create_impl(&p, b, intor, shls, nq, nullptr, nullptr, nullptr, false);
+  if (st == MCINT_OK) {
+    n[0] = n[1] = 0;
+    for (const Bucket& bk : p->launches)
+      if (bk.mode == 0) n[bk.mm ? 0 : 1] += bk.t1 - bk.t0;
+    n[2] = p->xfer_size;
+    n[3] = p->scratch_size;
     plan_free(p);
   }
   mcint_basis_destroy(b);

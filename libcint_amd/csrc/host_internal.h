@@ -32,6 +32,12 @@ int plan_build_host_only(const FINT* atm, FINT natm, const FINT* bas, FINT nbas,
                          const uint8_t* fp32_flags, int64_t* stats,
                          std::vector<int64_t>* bucket_info);
 
+// The host stage of plan construction alone (no HIP call): n[0], n[1] tasks
+// of runtime classes on the matrix and on the generic kernel, n[2] doubles of
+// transfer matrices, n[3] scratch doubles per branch.  For tests.
+int plan_matrices_host_only(const FINT* atm, FINT natm, const FINT* bas, FINT nbas, const double* env,
+                            int intor, const FINT* shls, size_t nq, int64_t* n);
+
 // Sets the calling thread's mcint_last_error() text.
 void set_error(const char* msg);
 
