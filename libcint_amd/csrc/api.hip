@@ -1366,7 +1366,8 @@ static int plan_create_impl(mcint_plan** out, mcint_basis* b, int intor, const F
       bk.sstride = chunked_block_doubles(kind, bk.la, bk.lb, bk.lc, bk.ld);
     } else if (bk.mode == 0) {
       const GenLayout G = gen_layout(kind, sph, bk.la, bk.lb, bk.lc, bk.ld, b->omega);
-      for (int w = mm_waves(G, bk.t1 - bk.t0, np); w >= 1 && !bk.mm; w -= 3)
+      // one wave where a block must not depend on its list (mm_waves looks at it)
+      for (int w = g_fill_lanes ? mm_waves(G, bk.t1 - bk.t0, np) : 1; w >= 1 && !bk.mm; w -= 3)
         bk.mm = mm_layout(kind, sph, bk.la, bk.lb, bk.lc, bk.ld, b->omega, w).waves;
       if (!gen_fits(G)) {
         plan_free(p);
