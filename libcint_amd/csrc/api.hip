@@ -200,16 +200,18 @@ struct Arena {
 
 // dst (pageable) = bytes of src (device) after the work on stream; returns
 // when the copy is done.  Threads take the chunks in turn: the host's part
-// (page faults of a fresh array, the copy out) is the longer one.  This thread
-// waits for the work first: hipStreamPerThread is another stream in each of
-// them, so that the handle alone would not order their copies after it.
+// (page faults of a fresh array, the copy out) is the longer one.
+// hipStreamPerThread is another stream in each of them: only there the handle
+// does not order their copies after the work, and this thread waits for it.
 // A thread without a staging buffer leaves its chunks to the others.
 hipError_t to_host(void* dst, const void* src, size_t bytes, hipStream_t stream) {
   const size_t chunks = (bytes + Stage::BYTES - 1) / Stage::BYTES;
   int dev = 0;
   if (chunks > 1 && hipGetDevice(&dev) == hipSuccess) {
-    const hipError_t done = hipStreamSynchronize(stream);
-    if (done != hipSuccess) return done;
+    if (stream == hipStreamPerThread) {
+      const hipError_t done = hipStreamSynchronize(stream);
+      if (done != hipSuccess) return done;
+    }
     std::atomic<size_t> next{0};
     std::atomic<int> failed{(int)hipSuccess};
     auto work = [&] {
