@@ -99,4 +99,41 @@ struct GenPrim {
 };
 static_assert(sizeof(GenPrim) == GEN_PRIM_D * sizeof(double), "GEN_PRIM_D");
 
+// The sets of X in LDS, three row sets and two column sets: first e (f) among
+// the list | number << 16, offset | weight << 28.  Absent ones are empty.
+constexpr int GEN_SETS = 5;
+__device__ __forceinline__ void put_sets(const GenLayout& G, int2* sets) {
+#pragma unroll
+  for (int r = 0; r < 3; ++r)
+    sets[r] = r < G.nbs ? make_int2(G.be[r] | (G.nes[r] << 16), G.ox[r] | (G.bw[r] << 28)) : make_int2(0, 0);
+#pragma unroll
+  for (int u = 0; u < 2; ++u)
+    sets[3 + u] = u < G.nks ? make_int2(G.kf[u] | (G.nfs[u] << 16), G.cf[u] | (G.kw[u] << 28)) : make_int2(0, 0);
+}
+// Adds a component's sums (e-list position ie, f-list position jf; g0, g1, g2
+// weighted 1, 2a_i, 4a_i^2, h0, h1 the first two times 2a_k) to the sets of X
+// it belongs to.  The sets come from LDS: indexed by a loop variable the
+// layout's arrays are read from memory one by one for every component, and
+// with constant indices they take scalar registers that the rest spills.
+// i-derivatives (dd|dg) of 256 primitives: 29.1 -> 25.2 ms on the generic kernel.
+__device__ __forceinline__ void add_to_sets(const int2* sets, int KF, double* X, int ie, int jf, double g0, double g1,
+                                            double g2, double h0, double h1) {
+  const int2 c[2] = {sets[3], sets[4]};
+  constexpr int OFF = (1 << 28) - 1;
+#pragma unroll
+  for (int r = 0; r < 3; ++r) {
+    const int2 q = sets[r];
+    const int er = ie - (q.x & 0xffff);
+    if ((unsigned)er >= ((unsigned)q.x >> 16)) continue;
+    double* const row = X + (q.y & OFF) + er * KF;
+    const int w = q.y >> 28;
+    const double g = w == 0 ? g0 : (w == 1 ? g1 : g2), h = w ? h1 : h0;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int fu = jf - (c[u].x & 0xffff);
+      if ((unsigned)fu < ((unsigned)c[u].x >> 16)) row[(c[u].y & OFF) + fu] += c[u].y >> 28 ? h : g;
+    }
+  }
+}
+
 }  // namespace mcint

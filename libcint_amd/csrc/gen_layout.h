@@ -43,6 +43,7 @@ __host__ __device__ constexpr int xfer_count(int l) {
 struct GenLayout {
   int nbs, blo[3], bhi[3], nes[3], bw[3], ox[3];
   int nks, klo[2], khi[2], nfs[2], kw[2], cf[2];
+  int be[3], kf[2];       // first e (f) of a set among the e-list (f-list)
   int e_lo, E, f_lo, F, nE, nF, KF;
   int nbc, nkc, ncomp;  // derivative components of the bra, the ket, in all
   int nca, ncb, ncc, ncd, nAo, nBo, nCo, nDo;
@@ -116,8 +117,10 @@ inline GenLayout gen_layout(int kind, int sph, int la, int lb, int lc, int ld, d
   g.nF = tet(g.F + 1) - tet(g.f_lo);
   for (int r = 0; r < g.nbs; ++r) {
     g.ox[r] = g.nX;
+    g.be[r] = tet(g.blo[r]) - tet(g.e_lo);
     g.nX += g.nes[r] * g.KF;
   }
+  for (int u = 0; u < g.nks; ++u) g.kf[u] = tet(g.klo[u]) - tet(g.f_lo);
   g.nbc = kind == KIND_2E_IPIP1 ? 9 : (ip1 ? 3 : 1);
   g.nkc = ket ? 3 : 1;
   g.ncomp = g.nbc * g.nkc;
@@ -149,7 +152,7 @@ inline GenLayout gen_layout(int kind, int sph, int la, int lb, int lc, int ld, d
   const int ncode = tet((g.E > g.F ? g.E : g.F) + 1);
   // terms: weights (doubles), packed exponents (ints), starts per component
   const int ntb = xfer_count(lb), ntk = three ? 1 : xfer_count(ld);
-  const int fixed = ntb + ntk + (ncode + ntb + ntk + g.ncb + g.ncd + 4 + 1) / 2;
+  const int fixed = ntb + ntk + (10 + ncode + ntb + ntk + g.ncb + g.ncd + 4 + 1) / 2;
   // a batch of primitive quartets: enough (primitive, direction, root)
   // recurrences for the lanes, at most 16 KB of tables
   // (second derivatives of 20 shells: 29.4 ms; 8 KB 31.9 ms, 4 KB 46 ms)
@@ -217,7 +220,7 @@ inline GenLayout mm_layout(int kind, int sph, int la, int lb, int lc, int ld, do
   g.ou = g.oP + g.PB * GEN_PRIM_D;
   g.ow = g.ou + g.PB * g.nrt;
   g.oI = g.nXz + space;
-  g.lds = g.oI + (ncode + g.nrow + g.ncol + 2 * waves + 1) / 2;
+  g.lds = g.oI + (10 + g.nrow + g.ncol + 2 * waves + (ncode + 1) / 2 + 1) / 2;
   g.waves = g.lds <= GEN_LDS_MAX ? waves : 0;
   return g;
 }

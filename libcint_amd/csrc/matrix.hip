@@ -60,10 +60,12 @@ eri_matrix_kernel(BasisView B, BucketArgs A, GenLayout G, XferView XV) {
   double* const su = sm + G.ou;
   double* const sw = sm + G.ow;
   const int ncode = tet((G.E > G.F ? G.E : G.F) + 1);
-  int* const code = reinterpret_cast<int*>(sm + G.oI);  // exponents of the components
-  int* const rt = code + ncode;    // output functions and component of each block row
+  int2* const sets = reinterpret_cast<int2*>(sm + G.oI);  // put_sets
+  int* const rt = reinterpret_cast<int*>(sets + GEN_SETS);  // output functions and component of each block row
   int* const ct = rt + G.nrow;     // ... and column, a | b << 8 | component << 16
   int* const scnt = ct + G.ncol;   // survivors of each wave, twice
+  uint16_t* const code = reinterpret_cast<uint16_t*>(scnt + 2 * W);  // exponents of the components
+  if (tid == 0) put_sets(G, sets);
   for (int i = tid; i < ncode; i += TH) {
     int l = 0, k = i;
     while (k >= ncart(l)) { k -= ncart(l); ++l; }
@@ -166,7 +168,15 @@ eri_matrix_kernel(BasisView B, BucketArgs A, GenLayout G, XferView XV) {
 #pragma unroll
             for (int r = 0; r < NRT; ++r) g = fma(V[vx + r] * V[vy + r], V[vz + r], g);
           } else {
-            for (int r = 0; r < nrt; ++r) g = fma(V[vx + r] * V[vy + r], V[vz + r], g);
+            double x = V[vx], y = V[vy], z = V[vz];
+            for (int r = 1; r < nrt; ++r) {
+              const double nx = V[vx + r], ny = V[vy + r], nz_ = V[vz + r];
+              g = fma(x * y, z, g);
+              x = nx;
+              y = ny;
+              z = nz_;
+            }
+            g = fma(x * y, z, g);
           }
           g0 += g;
           if constexpr (wt & 1) g1 = fma(g, sp[q].w[0], g1);
@@ -187,19 +197,7 @@ eri_matrix_kernel(BasisView B, BucketArgs A, GenLayout G, XferView XV) {
         default: run(std::integral_constant<int, 5>{}); break;
       }
     };
-    // adds a component's sums to the sets it belongs to
-    auto scatter = [&](int ie, int jf) {
-      for (int r = 0; r < G.nbs; ++r) {
-        const int er = ie + te - tet_d(G.blo[r]);
-        if (er < 0 || er >= G.nes[r]) continue;
-        for (int u = 0; u < G.nks; ++u) {
-          const int fu = jf + tf - tet_d(G.klo[u]);
-          if (fu < 0 || fu >= G.nfs[u]) continue;
-          const double v = G.kw[u] ? (G.bw[r] ? h1 : h0) : (G.bw[r] == 0 ? g0 : (G.bw[r] == 1 ? g1 : g2));
-          X[G.ox[r] + er * G.KF + G.cf[u] + fu] += v;
-        }
-      }
-    };
+    auto scatter = [&](int ie, int jf) { add_to_sets(sets, G.KF, X, ie, jf, g0, g1, g2, h0, h1); };
     for (int base = 0, odd = 0; base < npq; base += TH, odd ^= W) {
       // one candidate per lane, libcint's tests
       const int p = base + tid;
