@@ -1369,8 +1369,8 @@ static int plan_create_impl(mcint_plan** out, mcint_basis* b, int intor, const F
     } else if (bk.mode == 0) {
       const GenLayout G = gen_layout(kind, sph, bk.la, bk.lb, bk.lc, bk.ld, b->omega);
       // one wave where a block must not depend on its list (mm_waves looks at it)
-      for (int w = g_fill_lanes ? mm_waves(G, bk.t1 - bk.t0, np) : 1; w >= 1 && !bk.mm; w -= 3)
-        bk.mm = mm_layout(kind, sph, bk.la, bk.lb, bk.lc, bk.ld, b->omega, w).waves;
+      bk.mm = g_fill_lanes ? mm_waves(kind, sph, bk.la, bk.lb, bk.lc, bk.ld, b->omega, bk.t1 - bk.t0, np)
+                           : mm_layout(kind, sph, bk.la, bk.lb, bk.lc, bk.ld, b->omega, 1).waves;
       if (!gen_fits(G)) {
         plan_free(p);
         set_err("mcint_plan_create: angular momentum beyond the generic kernel's tables");

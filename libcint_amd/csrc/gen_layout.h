@@ -1,6 +1,8 @@
 // Work layout of the generic (any class) kernel, computed on the host and
 // passed to the kernel by value.
 #pragma once
+#include <algorithm>
+
 #include "mcint_internal.h"
 
 namespace mcint {
@@ -182,6 +184,11 @@ inline GenLayout gen_layout(int kind, int sph, int la, int lb, int lc, int ld, d
   return g;
 }
 
+// LDS doubles of the matrix kernel's four-wave workgroup: two of them per CU.
+constexpr int MM_LDS4 = 10200;
+// The matrix kernel's instances: up to this many roots, and one for more.
+constexpr int MM_NRT = 6;
+
 // Layout of the matrix kernel: X, then the walk's tables, each wave's Y and
 // the partial sums of shared components in one space, then the codes.
 inline GenLayout mm_layout(int kind, int sph, int la, int lb, int lc, int ld, double omega, int waves) {
@@ -221,21 +228,46 @@ inline GenLayout mm_layout(int kind, int sph, int la, int lb, int lc, int ld, do
   g.ow = g.ou + g.PB * g.nrt;
   g.oI = g.nXz + space;
   g.lds = g.oI + (10 + g.nrow + g.ncol + 2 * waves + (ncode + 1) / 2 + 1) / 2;
-  g.waves = g.lds <= GEN_LDS_MAX ? waves : 0;
+  g.waves = g.lds <= (waves > 1 ? MM_LDS4 : GEN_LDS_MAX) ? waves : 0;
   return g;
 }
 
-// Waves per task of n tasks with np primitive quartets in all: four where a
-// task holds many, or the bucket is too short to give every SIMD a wave,
-// and the products of one task (components x roots x primitive quartets)
-// are enough to share.  Second derivatives of 20 shells / three-centre
-// derivatives of 186 shells: 11.4 / 5.1 ms; one wave everywhere below 64
-// primitive quartets 15.0 / 4.7, four from 8 primitive quartets and 1000
-// products 11.3 / 6.4, one and four by primitives and tasks alone 11.7 / 5.3.
-constexpr int64_t MM_PRIMS = 24, MM_TASKS = 1024, MM_WORK = 2000;
-inline int mm_waves(const GenLayout& g, int64_t n, int64_t np) {
-  const double work = (double)np * g.nE * g.nF * g.nrt;
-  return (np >= MM_PRIMS * n || n < MM_TASKS) && work >= (double)MM_WORK * n ? 4 : 1;
+// Waves per task of a launch of n tasks with np primitive quartets in all: four
+// or one on the matrix kernel, 0 on the generic one.  Work is a task's products
+// (components x roots x primitive quartets).
+//   Four: with 2000 products or more to share, where the list is short, tasks
+//   hold many primitives (or many products of more roots than are compiled
+//   in), or the LDS then leaves a CU twice the waves (i-derivatives (dd|dg) of
+//   256 primitives, 3000 tasks: 44 KB for one wave, 69 for four; 52 and 11 ms).
+//   None: where the bra matrix outweighs the walk and at most four columns use
+//   it, of the matrix instruction's 16 (3000 Cartesian (gg|ss) of one
+//   primitive: 364 us, 54 on the generic kernel), where one-wave
+//   workgroups fill the LDS and tasks hold primitives for more than two to
+//   four waves (int2e_ip1ip2 (fp|df) of 256: 97 and 34 ms), and for (s|s) and
+//   (p|s), which are set-up alone (30 000 (s|s) of one primitive: 215 and 170 us).
+// Over 2716 lists (280 classes of every kind, s to i shells, 1 to 256 primitive
+// quartets, 300 to 30 000 tasks) this takes 1.04 times the fastest of the three
+// on geometric average; by tasks and primitives alone 1.14.
+constexpr int64_t MM_TASKS = 1024;
+constexpr double MM_PRIMS = 24, MM_WORK = 2000, MM_WORK4 = 50000;
+inline int mm_waves(int kind, int sph, int la, int lb, int lc, int ld, double omega, int64_t n, int64_t np) {
+  const GenLayout g1 = mm_layout(kind, sph, la, lb, lc, ld, omega, 1);
+  const GenLayout g4 = mm_layout(kind, sph, la, lb, lc, ld, omega, 4);
+  const double prims = (double)np / (double)n, work = prims * g1.nE * g1.nF * g1.nrt;
+  const bool four = g4.waves && work >= MM_WORK;
+  if (four && n < MM_TASKS) return 4;
+  const int bra = g1.RT * g1.KS;
+  if (g1.KS2 == 1 && bra >= 240 && work < 32.0 * bra) return 0;
+  if (kind == KIND_2C2E && work < 4) return 0;
+  // waves of a CU (160 KB of LDS, 256 CUs): by the LDS, and with this list
+  const int lds = 160 * 1024 / 8;
+  const int cu1 = std::min(12, lds / g1.lds), cu4 = 4 * std::min(4, lds / g4.lds);
+  const double tasks = n / 256.0;
+  if (four && (prims >= MM_PRIMS || (g1.nrt > MM_NRT && work >= MM_WORK4) ||
+               (prims >= 12 && std::min<double>(cu4, 4 * tasks) >= 2 * std::min<double>(cu1, tasks))))
+    return 4;
+  if (!g1.waves || (n >= MM_TASKS / 2 && ((cu1 <= 4 && prims >= MM_PRIMS) || (cu1 <= 2 && prims >= 8)))) return 0;
+  return 1;
 }
 
 // One matrix to lay out: the bra matrix of the virtual pair (a, b) or the

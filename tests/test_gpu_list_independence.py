@@ -22,7 +22,7 @@ def test_bits_of_a_block(name, omega):
         aux = rng.choice(np.arange(m.aux_start, m.nbas), 12, replace=False)
         q[:, 2] = rng.choice(aux, len(q))
         if name.startswith("int2c2e"):
-            q[:, 0] = rng.choice(aux, len(q))
+            q[:, 0], q[:, 1] = rng.choice(aux, len(q)), rng.choice(aux, len(q))
     env = m.env.copy()
     env[8] = omega
     B = mc.Basis(m.atm, m.bas, env)

@@ -15,6 +15,7 @@ import numpy as np
 import pytest
 
 from libcint_amd.synthetic import make_molecule, random_density, subset, unique_quartets
+from test_matrix_bound import CLASSES, _one_class
 
 pytestmark = pytest.mark.gpu
 
@@ -94,9 +95,9 @@ def _list(m, name, seed):
         q[:, 2] = rng.choice(aux, len(q))
         q[250:, 2] = rng.choice(aux[ls[aux] == 1], len(long))
         if name.startswith("int2c2e"):
-            q[:, 0] = rng.choice(aux, len(q))
+            q[:, 0], q[:, 1] = rng.choice(aux, len(q)), rng.choice(aux, len(q))
             q[250:, 0] = rng.choice(aux[ls[aux] == 0], len(long))
-            q[:, 1] = 0
+            q[250:, 1] = rng.choice(aux[ls[aux] == 1], len(long))
         q[:, 3] = 0
     return q
 
@@ -119,6 +120,21 @@ def test_blocks(mc, orc, name, omega, kernel):
     bad = np.flatnonzero(err > 1e-12 + 1e-10 * size)
     assert not len(bad), (f"{len(bad)} blocks, the first {q[bad[0]]} (l {m.bas[q[bad[0]], 1]}): "
                           f"{err[bad[0]]:.2e} of {size[bad[0]]:.2e}, largest {err.max():.2e}")
+    np.testing.assert_array_equal(nz, nz_r)
+
+
+@pytest.mark.parametrize("name,ls,nprim,n,omega", [c[:4] + (0.0,) for c in CLASSES]
+                         + [("int2e_cart", (4, 2, 3, 0), 2, 1100, -0.4)])
+def test_choice_of_kernel(mc, orc, name, ls, nprim, n, omega):
+    """One class on the kernel and waves its size, list and primitives choose;
+    the exponents are at most 6."""
+    m, q = _one_class(ls, nprim, n)
+    m.env[8] = omega
+    got, off, nz = mc.batch(name, q, mc.Basis(m.atm, m.bas, m.env))
+    ref, _, nz_r = orc.batch(name, q, orc.Basis(m.atm, m.bas, m.env))
+    size = np.maximum.reduceat(np.abs(ref), off[:-1])
+    err = np.maximum.reduceat(np.abs(got - ref), off[:-1])
+    assert (err <= 1e-12 + 1e-10 * size).all(), f"{err.max():.2e}"
     np.testing.assert_array_equal(nz, nz_r)
 
 
