@@ -244,7 +244,7 @@ inline GenLayout mm_layout(int kind, int sph, int la, int lb, int lc, int ld, do
 //   primitive: 364 us, 54 on the generic kernel), where one-wave
 //   workgroups fill the LDS and tasks hold primitives for more than two to
 //   four waves (int2e_ip1ip2 (fp|df) of 256: 97 and 34 ms), and for (s|s) and
-//   (p|s), which are set-up alone (30 000 (s|s) of one primitive: 215 and 170 us).
+//   (p|s), which are set-up alone (30 000 (s|s) of one primitive: 206 and 146 us).
 // Over 2716 lists (280 classes of every kind, s to i shells, 1 to 256 primitive
 // quartets, 300 to 30 000 tasks) this takes 1.04 times the fastest of the three
 // on geometric average; by tasks and primitives alone 1.14.
@@ -288,6 +288,12 @@ hipError_t launch_xfer(const VShell* vsh, int kind, int sph, const XferItem* ite
 // The matrix kernel on waves per task (1 or 4; mm_layout(..., waves).waves != 0).
 hipError_t launch_matrix(const BasisView& B, const BucketArgs& A, const XferView& X, int waves,
                          hipStream_t stream);
+
+// Waves from which on a workgroup takes several tasks, one after another: where
+// a primitive quartet's products are few, the set-up of a workgroup weighs more
+// than an even load (30 000 (s|s): 170 -> 146 us on the generic kernel; 30 000
+// (pf|dg) second derivatives 29.0 -> 30.8 ms).
+inline int64_t gen_share(const GenLayout& g) { return g.nE * g.nF * g.nrt <= 2000 ? 8192 : 16384; }
 
 // Whether the kernel's tables hold the class.
 inline bool gen_fits(const GenLayout& g) {

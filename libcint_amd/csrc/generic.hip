@@ -578,7 +578,7 @@ hipError_t launch_generic(const BasisView& B, const BucketArgs& A, hipStream_t s
   if (!gen_fits(G)) return hipErrorInvalidValue;
   if (A.scratch_stride < G.nblk) return hipErrorInvalidValue;
   // several tasks per wave share its tables once the chip is full
-  const int64_t per = std::min<int64_t>(8, std::max<int64_t>(1, n / 16384));
+  const int64_t per = std::min<int64_t>(8, std::max<int64_t>(1, n / gen_share(G)));
   const dim3 grid((unsigned)((n + per - 1) / per));
   const size_t lds = sizeof(double) * G.lds;
   if (G.in_lds)

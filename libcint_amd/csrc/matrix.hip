@@ -559,7 +559,7 @@ hipError_t launch_matrix(const BasisView& B, const BucketArgs& A, const XferView
   const GenLayout G = mm_layout(A.kind, A.sph, A.la, A.lb, A.lc, A.ld, B.omega, waves);
   if (!gen_fits(G) || !G.waves || !XV.m) return hipErrorInvalidValue;
   // several tasks per workgroup share its tables once the chip is full
-  const int64_t per = std::min<int64_t>(8, std::max<int64_t>(1, n * waves / 16384));
+  const int64_t per = std::min<int64_t>(8, std::max<int64_t>(1, n * waves / gen_share(G)));
   const dim3 grid((unsigned)((n + per - 1) / per));
   const size_t lds = sizeof(double) * G.lds;
   auto go = [&](auto W, auto N) {
