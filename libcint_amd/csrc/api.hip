@@ -830,7 +830,7 @@ struct mcint_plan {
   bool grad_refs = false;  // gradient plan: tasks carry a reference atom, no output offset
   std::vector<Bucket> buckets;   // tasks of one class and tuned team
   std::vector<Bucket> launches;  // tasks of one class, lanes per task and kernel
-  char* mem_d = nullptr;  // holds the tasks, pair tables and pair data below
+  char* mem_d = nullptr;  // holds the tasks, pair tables, pair data and matrices below
   Task* tasks_d = nullptr;
   int* task_id_d = nullptr;
   int64_t* pair_off_d = nullptr;
@@ -877,8 +877,6 @@ static void plan_free(mcint_plan* p) {
   dfree(p->flags_d);
   dfree(p->gslots_d);
   dfree(p->jk_d);
-  dfree(p->xfer_d);
-  dfree(p->xfer_off_d);
   delete p;
 }
 
@@ -993,6 +991,7 @@ struct Matrices {
   std::vector<XferItem> items;
   std::vector<int64_t> off;
   int64_t size = 0;  // doubles
+  int max_rows = 0, max_ks = 0;
 };
 
 // The matrices of the plan's matrix launches, the costliest launch first;
@@ -1043,6 +1042,8 @@ static void admit_matrices(mcint_plan* p, const Task* tasks, Matrices& X) {
       X.off[at] = X.size;
       X.items.push_back(XferItem{s, s2, k, k ? G.CT2 : G.RT, k ? G.KS2 : G.KS, X.size});
       X.size += k ? ket : bra;
+      X.max_rows = std::max(X.max_rows, X.items.back().rows);
+      X.max_ks = std::max(X.max_ks, X.items.back().ks);
     }
   }
 }
@@ -1455,48 +1456,52 @@ static int plan_create_impl(mcint_plan** out, mcint_basis* b, int intor, const F
     *out = p;
     return MCINT_OK;
   }
-  char* tmp_d = nullptr;  // shell pairs and the pair kernel's staging records
-  Arena m, tmp;
-  const size_t ot = m.add((size_t)ntasks, sorted.get()), oi = m.add((size_t)ntasks, sorted_q.get());
-  const size_t oo = m.add(pair_off.size(), pair_off.data());
-  const size_t ol = m.add(pair_off.size(), (const double*)nullptr);
-  const size_t op = m.add((size_t)npp, (const PairPrim*)nullptr), os = m.add((size_t)npp, (const int*)nullptr);
-  const size_t xp = tmp.add(pairs.size(), pairs.data()), xt = tmp.add((size_t)npp, (const PairPrim*)nullptr);
-  hipError_t e = m.make(&p->mem_d);
-  if (e == hipSuccess) e = tmp.make(&tmp_d);
-  p->tasks_d = (Task*)(p->mem_d + ot);
-  p->task_id_d = (int*)(p->mem_d + oi);
-  p->pair_off_d = (int64_t*)(p->mem_d + oo);
-  p->pair_ld_d = (double*)(p->mem_d + ol);
-  p->pp_d = (PairPrim*)(p->mem_d + op);
-  p->pp_pos_d = (int*)(p->mem_d + os);
-  int* const pairs_d = (int*)(tmp_d + xp);
-  PairPrim* const pp_tmp = (PairPrim*)(tmp_d + xt);
+  char* tmp_d = nullptr;  // shell pairs, matrices to lay out, the pair kernel's staging records
+  int* pairs_d = nullptr;
+  XferItem* items_d = nullptr;
+  PairPrim* pp_tmp = nullptr;
+  hipError_t e = hipSuccess;
+  for (bool matrices = !X.items.empty();; matrices = false) {
+    Arena m, tmp;
+    const size_t nx = matrices ? X.items.size() : 0;
+    const size_t ot = m.add((size_t)ntasks, sorted.get()), oi = m.add((size_t)ntasks, sorted_q.get());
+    const size_t oo = m.add(pair_off.size(), pair_off.data());
+    const size_t ox = matrices ? m.add(X.off.size(), X.off.data()) : 0;
+    const size_t ol = m.add(pair_off.size(), (const double*)nullptr);
+    const size_t op = m.add((size_t)npp, (const PairPrim*)nullptr), os = m.add((size_t)npp, (const int*)nullptr);
+    const size_t om = matrices ? m.add((size_t)X.size, (const double*)nullptr) : 0;
+    const size_t xp = tmp.add(pairs.size(), pairs.data()), xi = tmp.add(nx, X.items.data());
+    const size_t xt = tmp.add((size_t)npp, (const PairPrim*)nullptr);
+    e = m.make(&p->mem_d);
+    if (e == hipSuccess) e = tmp.make(&tmp_d);
+    p->tasks_d = (Task*)(p->mem_d + ot);
+    p->task_id_d = (int*)(p->mem_d + oi);
+    p->pair_off_d = (int64_t*)(p->mem_d + oo);
+    p->pair_ld_d = (double*)(p->mem_d + ol);
+    p->pp_d = (PairPrim*)(p->mem_d + op);
+    p->pp_pos_d = (int*)(p->mem_d + os);
+    p->xfer_off_d = matrices ? (int64_t*)(p->mem_d + ox) : nullptr;
+    p->xfer_d = matrices ? (double*)(p->mem_d + om) : nullptr;
+    pairs_d = (int*)(tmp_d + xp);
+    items_d = (XferItem*)(tmp_d + xi);
+    pp_tmp = (PairPrim*)(tmp_d + xt);
+    if (e == hipSuccess || !matrices) break;
+    // no room for the matrices: the generic kernel does without
+    (void)hipGetLastError();
+    dfree(p->mem_d);
+    dfree(tmp_d);
+    p->xfer_size = 0;
+    for (auto* list : {&p->buckets, &p->launches})
+      for (Bucket& bk : *list) off_matrix(p, bk);
+    size_scratch();
+  }
   if (e == hipSuccess)
     e = launch_pairdata(b->vsh_d, b->env_d, nv, pairs_d, (int)(pairs.size() / 2), p->pair_off_d,
                         p->pair_ld_d, pp_tmp, p->pp_d, p->pp_pos_d, nullptr);
-  XferItem* items_d = nullptr;
-  if (e == hipSuccess && !X.items.empty()) {
-    if (dalloc(&items_d, X.items.size()) != hipSuccess || dalloc(&p->xfer_d, (size_t)X.size) != hipSuccess ||
-        dalloc(&p->xfer_off_d, X.off.size()) != hipSuccess) {
-      // no room for the matrices: the generic kernel does without
-      (void)hipGetLastError();
-      dfree(p->xfer_d);
-      dfree(p->xfer_off_d);
-      p->xfer_size = 0;
-      for (auto* list : {&p->buckets, &p->launches})
-        for (Bucket& bk : *list) off_matrix(p, bk);
-      size_scratch();
-    } else {
-      e = to_device(items_d, X.items.data(), X.items.size());
-      if (e == hipSuccess) e = to_device(p->xfer_off_d, X.off.data(), X.off.size());
-      if (e == hipSuccess)
-        e = launch_xfer(b->vsh_d, kind, sph, items_d, (int)X.items.size(), p->xfer_d, nullptr);
-    }
-  }
+  if (e == hipSuccess && p->xfer_d)
+    e = launch_xfer(b->vsh_d, kind, sph, items_d, (int)X.items.size(), X.max_rows, X.max_ks, p->xfer_d, nullptr);
   if (e == hipSuccess) e = hipDeviceSynchronize();
   timer.mark("device upload, pair data");
-  dfree(items_d);
   dfree(tmp_d);
   if (e != hipSuccess) {
     set_err(std::string("mcint_plan_create: ") + hipGetErrorString(e));

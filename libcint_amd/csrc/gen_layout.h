@@ -283,8 +283,9 @@ struct XferView {
   const int64_t* ket;
   int nv;
 };
-hipError_t launch_xfer(const VShell* vsh, int kind, int sph, const XferItem* items, int n, double* m,
-                       hipStream_t stream);
+// max_rows, max_ks: the largest among the items
+hipError_t launch_xfer(const VShell* vsh, int kind, int sph, const XferItem* items, int n, int max_rows, int max_ks,
+                       double* m, hipStream_t stream);
 // The matrix kernel on waves per task (1 or 4; mm_layout(..., waves).waves != 0).
 hipError_t launch_matrix(const BasisView& B, const BucketArgs& A, const XferView& X, int waves,
                          hipStream_t stream);

@@ -611,92 +611,123 @@ __device__ __forceinline__ PairSets pair_sets(int kind, bool ket, int l1, int l2
   return s;
 }
 
-// The matrix that takes a pair's primitive sums (row sets) to its output
-// functions and derivative components: spherical transform of both shells,
-// transfer (a,b| = sum_t C(b,t) (A-B)^(b-t) [a+t|, and the derivative rules of
-// gen_layout.h.  One workgroup per matrix, one lane per output row; laid out
-// as the 16 x 4 tiles of the matrix instruction, lane order, zero padded.
+// One row of a pair's matrix: the output function (ao, bo) and derivative
+// component bc of shells la, lb as a sum over the pair's primitive sums:
+// spherical transform of both shells, transfer (a,b| = sum_t C(b,t)
+// (A-B)^(b-t) [a+t|, and the derivative rules of gen_layout.h.
+// add(set, x, y, z, value).
+template <typename Add>
+__device__ __forceinline__ void xfer_row(int sph, bool one, bool two, int top, int la, int lb, int ao, int bo, int bc,
+                                         const double (*binom)[LMAX + 1], const double (*pw)[LMAX + 1], Add&& add) {
+  const int p = two ? (bc < 3 ? 0 : (bc < 5 ? 1 : 2)) : bc;
+  const int q = two ? (bc < 3 ? bc : (bc < 5 ? bc - 2 : 2)) : 0;
+  const int ra = la * la + ao, rb = lb * lb + bo;
+  const int ia1 = sph ? c2s_sparse.ptr[ra + 1] : ao + 1, ib1 = sph ? c2s_sparse.ptr[rb + 1] : bo + 1;
+  for (int ia = sph ? c2s_sparse.ptr[ra] : ao; ia < ia1; ++ia) {
+    const int ka = sph ? c2s_sparse.k[ia] : ia;
+    int ma = 0;
+    while ((ma + 1) * (ma + 2) / 2 <= ka) ++ma;
+    const int az = ka - ma * (ma + 1) / 2, ay = ma - az, ax = la - ma;
+    const int px = p == 0, py = p == 1, pz = p == 2, qx = q == 0, qy = q == 1, qz = q == 2;
+    const int ap = p == 0 ? ax : (p == 1 ? ay : az), aq = q == 0 ? ax : (q == 1 ? ay : az);
+    for (int ib = sph ? c2s_sparse.ptr[rb] : bo; ib < ib1; ++ib) {
+      const int kb = sph ? c2s_sparse.k[ib] : ib;
+      int mb = 0;
+      while ((mb + 1) * (mb + 2) / 2 <= kb) ++mb;
+      const int bz = kb - mb * (mb + 1) / 2, by = mb - bz, bx = lb - mb;
+      const double cc = sph ? c2s_sparse.v[ia] * c2s_sparse.v[ib] : 1.0;
+      for (int tx = 0; tx <= bx; ++tx)
+        for (int ty = 0; ty <= by; ++ty)
+          for (int tz = 0; tz <= bz; ++tz) {
+            const double w = cc * (binom[bx][tx] * binom[by][ty] * binom[bz][tz]) *
+                             (pw[0][bx - tx] * pw[1][by - ty] * pw[2][bz - tz]);
+            const int x = ax + tx, y = ay + ty, z = az + tz;
+            if (!one && !two) {
+              add(0, x, y, z, w);
+              continue;
+            }
+            if (one) {
+              add(top, x + px, y + py, z + pz, -w);
+              if (ap > 0) add(0, x - px, y - py, z - pz, ap * w);
+              continue;
+            }
+            add(top, x + px + qx, y + py + qy, z + pz + qz, w);
+            if (p == q) {
+              add(top - 1, x, y, z, -(2 * ap + 1) * w);
+              if (ap > 1) add(0, x - 2 * px, y - 2 * py, z - 2 * pz, ap * (ap - 1) * w);
+            } else {
+              if (aq > 0) add(top - 1, x + px - qx, y + py - qy, z + pz - qz, -aq * w);
+              if (ap > 0) add(top - 1, x + qx - px, y + qy - py, z + qz - pz, -ap * w);
+              if (ap > 0 && aq > 0) add(0, x - px - qx, y - py - qy, z - pz - qz, (double)(ap * aq) * w);
+            }
+          }
+    }
+  }
+}
+
+// The matrices of a plan's pairs (blockIdx.x), laid out as the 16 x 4 tiles of
+// the matrix instruction, lane order, zero padded.  A lane sums one row; a
+// workgroup the 2^k rows that fit its LDS, then writes them, and the rows of
+// a matrix are spread over gridDim.y workgroups.  What bounds it: a row is a
+// chain of hundreds to thousands of small additions.  Made in global memory by
+// one workgroup per matrix they took 2.1 ms for 16 (gg| pairs' i-derivatives.
 __global__ void __launch_bounds__(64)
 xfer_kernel(const VShell* __restrict__ vsh, int kind, int sph, const XferItem* __restrict__ items,
-            double* __restrict__ m) {
+            double* __restrict__ m, int lds) {
+  extern __shared__ double acc[];  // lds doubles, [column][row]
+  __shared__ double binom[LMAX + 1][LMAX + 1], pw[3][LMAX + 1];
+  const int tid = threadIdx.x;
   const XferItem it = items[blockIdx.x];
   const bool ket = it.ket, three = kind_three(kind);
   const VShell &a = vsh[it.a], &b = vsh[it.b];
   const int la = a.l, lb = ket && three ? 0 : b.l;
-  const double ab[3] = {a.r[0] - b.r[0], a.r[1] - b.r[1], a.r[2] - b.r[2]};
-  double* const M = m + it.off;
-  for (int64_t i = threadIdx.x; i < (int64_t)it.rows * it.ks * 64; i += 64) M[i] = 0.0;
-  __syncthreads();
+  if (tid <= LMAX)
+    for (int k = 0; k <= tid; ++k) binom[tid][k] = binom_small(tid, k);
+  if (tid < 3) {
+    double v = 1.0;
+    for (int k = 0; k <= lb; ++k) {
+      pw[tid][k] = v;
+      v *= a.r[tid] - b.r[tid];
+    }
+  }
   const PairSets S = pair_sets(kind, ket, la, lb);
   const bool two = !ket && kind == KIND_2E_IPIP1;
   const bool one = !two && (ket ? kind_ket_der(kind) || kind == KIND_2E_IP1IP2
                                 : kind_bra_der(kind) || kind == KIND_2E_IP1IP2);
   const int nA = sph ? 2 * la + 1 : ncart(la), nB = sph ? 2 * lb + 1 : ncart(lb);
   const int n = nA * nB * (two ? 6 : (one ? 3 : 1));
-  for (int row = threadIdx.x; row < n; row += 64) {
-    const int ao = row % nA, bo = (row / nA) % nB, bc = row / (nA * nB);
-    const int p = two ? (bc < 3 ? 0 : (bc < 5 ? 1 : 2)) : bc;
-    const int q = two ? (bc < 3 ? bc : (bc < 5 ? bc - 2 : 2)) : 0;
-    double* const mr = M + (int64_t)(row >> 4) * it.ks * 64 + (row & 15);
-    // column (set r, exponents x y z): k step k / 4, lane group k % 4
-    auto add = [&](int r, int x, int y, int z, double v) {
-      const int k = S.pos[r] + cart_all(x, y, z) - tet_d(S.lo[r]);
-      mr[(k >> 2) * 64 + (k & 3) * 16] += v;
-    };
-    const int ra = la * la + ao, rb = lb * lb + bo;
-    const int ia1 = sph ? c2s_sparse.ptr[ra + 1] : ao + 1, ib1 = sph ? c2s_sparse.ptr[rb + 1] : bo + 1;
-    for (int ia = sph ? c2s_sparse.ptr[ra] : ao; ia < ia1; ++ia) {
-      const int ka = sph ? c2s_sparse.k[ia] : ia;
-      int ma = 0;
-      while ((ma + 1) * (ma + 2) / 2 <= ka) ++ma;
-      const int az = ka - ma * (ma + 1) / 2, ay = ma - az, ax = la - ma;
-      for (int ib = sph ? c2s_sparse.ptr[rb] : bo; ib < ib1; ++ib) {
-        const int kb = sph ? c2s_sparse.k[ib] : ib;
-        int mb = 0;
-        while ((mb + 1) * (mb + 2) / 2 <= kb) ++mb;
-        const int bz = kb - mb * (mb + 1) / 2, by = mb - bz, bx = lb - mb;
-        const double cc = sph ? c2s_sparse.v[ia] * c2s_sparse.v[ib] : 1.0;
-        for (int tx = 0; tx <= bx; ++tx)
-          for (int ty = 0; ty <= by; ++ty)
-            for (int tz = 0; tz <= bz; ++tz) {
-              double w = cc * binom_small(bx, tx) * binom_small(by, ty) * binom_small(bz, tz);
-              for (int j = tx; j < bx; ++j) w *= ab[0];
-              for (int j = ty; j < by; ++j) w *= ab[1];
-              for (int j = tz; j < bz; ++j) w *= ab[2];
-              const int x = ax + tx, y = ay + ty, z = az + tz;
-              if (!one && !two) {
-                add(0, x, y, z, w);
-                continue;
-              }
-              const int px = p == 0, py = p == 1, pz = p == 2;
-              const int ap = p == 0 ? ax : (p == 1 ? ay : az);
-              const int top = S.n - 1;
-              if (one) {
-                add(top, x + px, y + py, z + pz, -w);
-                if (ap > 0) add(0, x - px, y - py, z - pz, ap * w);
-                continue;
-              }
-              const int qx = q == 0, qy = q == 1, qz = q == 2;
-              const int aq = q == 0 ? ax : (q == 1 ? ay : az);
-              add(top, x + px + qx, y + py + qy, z + pz + qz, w);
-              if (p == q) {
-                add(top - 1, x, y, z, -(2 * ap + 1) * w);
-                if (ap > 1) add(0, x - 2 * px, y - 2 * py, z - 2 * pz, ap * (ap - 1) * w);
-              } else {
-                if (aq > 0) add(top - 1, x + px - qx, y + py - qy, z + pz - qz, -aq * w);
-                if (ap > 0) add(top - 1, x + qx - px, y + qy - py, z + qz - pz, -ap * w);
-                if (ap > 0 && aq > 0) add(0, x - px - qx, y - py - qy, z - pz - qz, (double)(ap * aq) * w);
-              }
-            }
-      }
+  const int ncol = it.ks * 4;
+  int rw = 64;
+  while (rw > 1 && rw * ncol > lds) rw >>= 1;
+  double* const M = m + it.off;
+  for (int r0 = blockIdx.y * rw; r0 < it.rows * 16; r0 += gridDim.y * rw) {
+    for (int i = tid; i < rw * ncol; i += 64) acc[i] = 0.0;
+    __syncthreads();
+    const int row = r0 + tid;
+    if (tid < rw && row < n)
+      xfer_row(sph, one, two, S.n - 1, la, lb, row % nA, (row / nA) % nB, row / (nA * nB), binom, pw,
+               [&](int r, int x, int y, int z, double v) {
+                 acc[(S.pos[r] + cart_all(x, y, z) - tet_d(S.lo[r])) * rw + tid] += v;
+               });
+    __syncthreads();
+    // column k: k step k / 4, lane group k % 4
+    for (int i = tid; i < rw * ncol; i += 64) {
+      const int k = i / rw, r = r0 + i % rw;
+      if (r < it.rows * 16) M[((int64_t)(r >> 4) * it.ks + (k >> 2)) * 64 + (k & 3) * 16 + (r & 15)] = acc[i];
     }
+    __syncthreads();
   }
 }
 
-hipError_t launch_xfer(const VShell* vsh, int kind, int sph, const XferItem* items, int n, double* m,
-                       hipStream_t stream) {
+hipError_t launch_xfer(const VShell* vsh, int kind, int sph, const XferItem* items, int n, int max_rows, int max_ks,
+                       double* m, hipStream_t stream) {
   if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(xfer_kernel, dim3((unsigned)n), dim3(64), 0, stream, vsh, kind, sph, items, m);
+  const int lds = std::max(4000, 4 * max_ks);
+  int rw = 64;  // rows at a time of the largest matrix, as in the kernel
+  while (rw > 1 && rw * 4 * max_ks > lds) rw >>= 1;
+  const int split = std::min(64, (max_rows * 16 + rw - 1) / rw);
+  hipLaunchKernelGGL(xfer_kernel, dim3((unsigned)n, (unsigned)split), dim3(64), sizeof(double) * lds,
+                     stream, vsh, kind, sph, items, m, lds);
   return hipGetLastError();
 }
 
