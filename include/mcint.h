@@ -431,10 +431,10 @@ int mcint_schwarz(mcint_basis *b, int nshell, double *q);
  * one; read at launch.
  * MCINT_TUNE_FILL_LANES (default 131072): a class of a plan whose teams put
  * fewer lanes than this to work has them widened (up to one wave per
- * quartet), and runtime classes take one or four waves per quartet by the
- * plan's list.  A block's last bits, not its accuracy, then depend on the
+ * quartet), and runtime and some derivative classes choose between kernels by
+ * the plan's list.  A block's last bits, not its accuracy, then depend on the
  * list it is computed in.  0 keeps the tuned primitive quartets per lane
- * (as for tuning them) and one wave: a tuple's block has the same bits in
+ * (as for tuning them) and one kernel: a tuple's block has the same bits in
  * every list, but for classes that MCINT_TUNE_MATRIX_KIB takes off.
  * MCINT_TUNE_MATRIX_KIB (default 2097152, 2 GiB): bound of the transfer
  * matrices that a plan lays out for its runtime classes; the costliest

@@ -827,6 +827,7 @@ struct mcint_plan {
   mcint_basis* b = nullptr;
   int intor = 0, kind = 0, sph = 1, ncomp = 1;
   int64_t nq = 0, ntasks = 0, out_size = 0;
+  bool by_list = true;     // kernels may be chosen by the list (mcint_tune MCINT_TUNE_FILL_LANES not 0)
   bool grad_refs = false;  // gradient plan: tasks carry a reference atom, no output offset
   std::vector<Bucket> buckets;   // tasks of one class and tuned team
   std::vector<Bucket> launches;  // tasks of one class, lanes per task and kernel
@@ -1082,6 +1083,7 @@ static int plan_create_impl(mcint_plan** out, mcint_basis* b, int intor, const F
   p->ncomp = ncomp;
   p->nq = (int64_t)nq;
   p->grad_refs = grad_refs != nullptr;
+  p->by_list = g_fill_lanes != 0;
 
   // ---- per quartet: validation, block size, canonical order, bucket key --
   // Threads take contiguous quartet ranges; tasks are then placed by a
@@ -1370,7 +1372,7 @@ static int plan_create_impl(mcint_plan** out, mcint_basis* b, int intor, const F
     } else if (bk.mode == 0) {
       const GenLayout G = gen_layout(kind, sph, bk.la, bk.lb, bk.lc, bk.ld, b->omega);
       // one wave where a block must not depend on its list (mm_waves looks at it)
-      bk.mm = g_fill_lanes ? mm_waves(kind, sph, bk.la, bk.lb, bk.lc, bk.ld, b->omega, bk.t1 - bk.t0, np)
+      bk.mm = p->by_list ? mm_waves(kind, sph, bk.la, bk.lb, bk.lc, bk.ld, b->omega, bk.t1 - bk.t0, np)
                            : mm_layout(kind, sph, bk.la, bk.lb, bk.lc, bk.ld, b->omega, 1).waves;
       if (!gen_fits(G)) {
         plan_free(p);
@@ -1680,6 +1682,7 @@ static BucketArgs bucket_args(const mcint_plan* p, const Bucket& bk, double* out
   A.sph = p->sph;
   A.team = bk.lanes;
   A.tune_team = bk.team;
+  A.many = p->by_list && bk.t1 - bk.t0 >= MANY_TASKS;
   A.fp32 = bk.fp32;
   A.t0 = bk.t0;
   A.t1 = bk.t1;

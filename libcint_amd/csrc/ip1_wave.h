@@ -274,6 +274,15 @@ struct Ip1WaveCfg {
   // 426 -> 233 us, (pd|dp) of 36 305 -> 164 us; below, it loses: (dd|ds) of 1
   // 108 -> 270 us, (pp|dp) of 36 178 -> 234 us.
   static constexpr bool OK = C::NF >= 9 && C::NE * C::NF >= 360;
+  // Few columns per lane on a list that fills the chip: the chunk kernels'
+  // lanes have a primitive quartet each.  Lists of 200 000 of 1 and 16 primitive
+  // quartets, chunk and wave kernels: (pd|pp) stored 1.00 / 1.55, 1.71 / 2.68
+  // ms, digested 1.01 / 1.25, 1.75 / 2.41; (dd|pp) stored 2.04 / 2.36, 3.09 /
+  // 3.72, digested 1.79 / 1.65, 2.86 / 3.08; (pd|dp) stored 1.76 / 2.04, 3.02 /
+  // 3.35, digested 1.86 / 1.39, 3.15 / 2.73.  Of 300 to 3000 the wave kernel
+  // takes 1.02 to 2.1 times less in all of them.
+  static constexpr bool MANY_DIGEST = C::NF >= 16;
+  static constexpr bool MANY_STORE = C::NF > 16 || (C::NF == 16 && LA >= LB);
 };
 
 template <int LA, int LB, int LC, int LD>
@@ -511,14 +520,15 @@ __global__ void __launch_bounds__(64) eri_ip1_wave_kernel(BasisView Bv, BucketAr
   if (digest && sl < 6 && cur >= 0) atomicAdd(gbase + 3 * cur + sl % 3, cs);
 }
 
-// Whether buckets of a derivative class with teams of tune_team lanes run
-// the wave kernel: teams of one (up to 128 primitive quartets).  With 216 the
+// Whether a launch of a derivative class runs the wave kernel: teams of one
+// (up to 128 primitive quartets), long lists as above.  With 216 the
 // chunk kernels' lanes all have a primitive quartet of their own: (dp|pp)
 // 420 us against 602, (pp|dp) 746 against 1071.
 template <int LA, int LB, int LC, int LD>
-bool ip1_on_wave(int tune_team, double omega) {
-  if (!Ip1WaveCfg<LA, LB, LC, LD>::OK || g_wave_kernels == 0 || omega < 0) return false;
-  return g_wave_kernels == 2 || tune_team == 1;
+bool ip1_on_wave(const BucketArgs& A, double omega) {
+  using W = Ip1WaveCfg<LA, LB, LC, LD>;
+  if (!W::OK || g_wave_kernels == 0 || omega < 0) return false;
+  return g_wave_kernels == 2 || (A.tune_team == 1 && (!A.many || (A.dm ? W::MANY_DIGEST : W::MANY_STORE)));
 }
 
 template <int LA, int LB, int LC, int LD, int... GRPs>
@@ -528,7 +538,7 @@ hipError_t launch_ip1(const BasisView& B, const BucketArgs& A, hipStream_t strea
   hipError_t e = hipSuccess;
   bool done = false;
   if constexpr (Ip1WaveCfg<LA, LB, LC, LD>::OK) {
-    if (ip1_on_wave<LA, LB, LC, LD>(A.tune_team, B.omega)) {
+    if (ip1_on_wave<LA, LB, LC, LD>(A, B.omega)) {
       constexpr int TPW = Ip1WaveCfg<LA, LB, LC, LD>::TPW;
       const int64_t grp = (n + TPW - 1) / TPW;
       // several groups per wave once the chip is full (16 waves per CU)

@@ -117,6 +117,7 @@ struct BasisView {
 
 // Launch description of one bucket: tasks [t0, t1) share class, kind,
 // team size and path (each task carries its own axis map).
+constexpr int64_t MANY_TASKS = 8192;
 struct BucketArgs {
   const Task* tasks;
   int64_t t0, t1;
@@ -132,6 +133,8 @@ struct BucketArgs {
   int team;              // lanes per task (fast kernels)
   int tune_team;         // team size that selects the tuned kernel of a chunked class
                          // (= team unless the team was widened to fill the chip)
+  int many;              // the launch, of which this may be a slice, holds MANY_TASKS
+                         // (never set where a block must not depend on its list)
   int fp32;              // recurrences and contraction in FP32 (fast kernels)
   int col_major;         // chunked classes: per-task blocks stored [f][e] (wave
                          // kernel) instead of in the chunk order
