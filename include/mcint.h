@@ -417,13 +417,17 @@ int mcint_schwarz(mcint_basis *b, int nshell, double *q);
  * that shares one contracted quartet is the smallest power of two (<= 64)
  * giving at most this many primitive quartets per lane (default 32).
  * MCINT_TUNE_GENERIC_ONLY: value 1 routes every quartet of plans created
- * afterwards to the generic kernel (runtime class, one workgroup per
- * quartet, no register kernels): the plain path that the benchmark times
- * and cross-checks the register kernels against; 0 (default) restores the
- * class-specialised kernels.  MCINT_TUNE_GRAPH_BRANCHES (1..8, default
+ * afterwards to the kernels whose class is known at run time (the matrix
+ * kernel, the generic one where that has no layout or MCINT_TUNE_MATRIX_KIB
+ * takes the class off; one workgroup per quartet, no register kernels): the
+ * plain path that the benchmark times and cross-checks the register kernels
+ * against; 0 (default) restores the class-specialised kernels.
+ * MCINT_TUNE_GRAPH_BRANCHES (1..8, default
  * 4): mcint_plan_execute on a stream captures the plan's buckets into that
  * many concurrent graph branches (buckets balanced by estimated work, one
- * scratch region per branch); takes effect at the next capture.
+ * scratch region per branch); takes effect at the next capture.  Launches that
+ * are not captured (J/K, gradients, host batches) run on as many side streams,
+ * on three at the default of 4.
  * MCINT_TUNE_WAVE_KERNELS (default 1): buckets of the chunked classes run
  * the wave kernel (16-64 lanes per quartet) instead of their
  * component-chunk kernels: 0 never, 1 where measured faster (the tuned

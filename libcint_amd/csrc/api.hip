@@ -695,19 +695,23 @@ constexpr int FILL_LANES = 1 << 17;
 // Tuning state (mcint_tune): primitive quartets per lane that the team
 // size aims at.
 int g_prims_per_lane = 32;
-// 1: every quartet on the generic kernel (mcint_tune MCINT_TUNE_GENERIC_ONLY)
+// 1: every quartet on the runtime-class kernels (mcint_tune MCINT_TUNE_GENERIC_ONLY)
 int g_generic_only = 0;
 // concurrent branches of a captured plan graph (mcint_tune MCINT_TUNE_GRAPH_BRANCHES)
-int g_graph_branches = 4;
+constexpr int GRAPH_BRANCHES = 4;
+int g_graph_branches = GRAPH_BRANCHES;
 constexpr int MAX_GRAPH_BRANCHES = 8;
-// Branches of launches that are not captured (J/K, gradients, host batches).
-// The runtime maps streams onto four hardware queues, the caller's stream
-// among them, so that a fourth side stream queues behind another: J/K of 98
-// shells on 3 / 4 / 6 side streams 16.6 / 17.4 / 16.7 ms, triple zeta 28.6 /
-// 31.8 / 27.9, gradient of 58 shells 12.2 / 13.6 / 12.1 ms.
+// Branches of launches that are not captured (J/K, gradients, host batches):
+// what was asked for, three where that is the default.  The runtime maps
+// streams onto four hardware queues, the caller's stream among them, so that a
+// fourth side stream queues behind another: J/K of 98 shells on 3 / 4 / 6 side
+// streams 16.8 / 17.6 / 16.8 ms, triple zeta 28.6 / 32.0 / 28.4, gradient of 58
+// shells 12.4 / 13.8 / 12.3; three need half the scratch of six.  (A captured
+// graph's branches are scheduled by the graph, not by these streams.)
 constexpr int EAGER_BRANCHES = 3;
 int eager_branches(size_t launches) {
-  return std::max(1, std::min<int>({g_graph_branches, EAGER_BRANCHES, (int)launches}));
+  const int n = g_graph_branches == GRAPH_BRANCHES ? EAGER_BRANCHES : g_graph_branches;
+  return std::max(1, std::min<int>(n, (int)launches));
 }
 // per-class overrides (mcint_tune_class), 0 = the global value; indexed by
 // integral kind and canonical class
