@@ -55,7 +55,9 @@ template <typename T>
 hipError_t dalloc(T** p, size_t n) {
   *p = nullptr;
   if (n == 0) return hipSuccess;
-  return hipMalloc((void**)p, n * sizeof(T));
+  const hipError_t e = hipMalloc((void**)p, n * sizeof(T));
+  if (e != hipSuccess) (void)hipGetLastError();  // e says it; the next launch check must not
+  return e;
 }
 
 template <typename T>
@@ -1493,7 +1495,6 @@ static int plan_create_impl(mcint_plan** out, mcint_basis* b, int intor, const F
     pp_tmp = (PairPrim*)(tmp_d + xt);
     if (e == hipSuccess || !matrices) break;
     // no room for the matrices: the generic kernel does without
-    (void)hipGetLastError();
     dfree(p->mem_d);
     dfree(tmp_d);
     p->xfer_size = 0;
@@ -1945,12 +1946,17 @@ extern "C" int mcint_plan_execute_jk(mcint_plan* p, const double* dm_dev, int na
   if (const int st = ensure_scratch(p, nbr)) return st;
   const int64_t nn = (int64_t)nao * nao;
   const int64_t stride = (2 * nn + 15) & ~int64_t(15);  // whole cache lines
-  const int slots = JK_SLOTS * stride <= JK_SLOT_DOUBLES ? JK_SLOTS : 1;
+  int slots = JK_SLOTS * stride <= JK_SLOT_DOUBLES ? JK_SLOTS : 1;
   if (p->jk_n < slots * stride) {
     if (p->jk_d) HIPCHK(hipDeviceSynchronize());
     dfree(p->jk_d);
     p->jk_n = 0;
-    HIPCHK(dalloc(&p->jk_d, (size_t)(slots * stride)));
+    hipError_t e = dalloc(&p->jk_d, (size_t)(slots * stride));
+    if (e != hipSuccess && slots > 1) {
+      slots = 1;  // no room for the copies
+      e = dalloc(&p->jk_d, (size_t)stride);
+    }
+    HIPCHK(e);
     p->jk_n = slots * stride;
   }
   double* Jp = vj_dev ? p->jk_d : nullptr;
@@ -2376,9 +2382,8 @@ int mcint::stages_live() { return Stage::live; }
 // unless a scratch region for each would be large.
 static int plan_run(mcint_plan* p, double* out, FINT* not0, hipStream_t stream) {
   const int nbr = eager_branches(p->launches.size());
-  if (nbr <= 1 || p->scratch_size * nbr > GEN_SCRATCH_DOUBLES / 8)
-    return mcint_plan_execute_direct(p, out, not0, stream);
-  if (const int st = ensure_scratch(p, nbr)) return st;
+  if (nbr <= 1 || p->scratch_size * nbr > GEN_SCRATCH_DOUBLES / 8 || ensure_scratch(p, nbr) != MCINT_OK)
+    return mcint_plan_execute_direct(p, out, not0, stream);  // one region, if at all
   return launch_branched(p, stream, nbr, [&](const Bucket& bk, hipStream_t s, const ScratchView& S) {
     return bucket_launch(p, bk, out, not0, s, S);
   });
