@@ -1635,15 +1635,35 @@ extern "C" int mcint_gradient_list(const mcint_basis* b, FINT* shls, FINT* refs,
   return MCINT_OK;
 }
 
-extern "C" int mcint_plan_create_gradient(mcint_plan** out, mcint_basis* b, const FINT* shls,
-                                          const FINT* refs, size_t nq, const uint8_t* fp32_flags) {
+static int gradient_plan_impl(mcint_plan** out, mcint_basis* b, const FINT* shls, const FINT* refs, size_t nq,
+                              const uint8_t* fp32_flags, bool upload) {
   if (!refs && nq) {
     set_err("mcint_plan_create_gradient: null argument");
     return MCINT_ERR_ARG;
   }
   static const FINT none = -1;
-  return plan_create_impl(out, b, MCINT_INT2E_IP1_SPH, shls, nq, nullptr, fp32_flags, nullptr, true,
+  return plan_create_impl(out, b, MCINT_INT2E_IP1_SPH, shls, nq, nullptr, fp32_flags, nullptr, upload,
                           refs ? refs : &none);
+}
+
+extern "C" int mcint_plan_create_gradient(mcint_plan** out, mcint_basis* b, const FINT* shls,
+                                          const FINT* refs, size_t nq, const uint8_t* fp32_flags) {
+  return gradient_plan_impl(out, b, shls, refs, nq, fp32_flags, true);
+}
+
+int mcint::gradient_plan_host_only(mcint_basis* b, const FINT* shls, const FINT* refs, size_t nq,
+                                   const uint8_t* fp32_flags, int64_t* stats) {
+  mcint_plan* p = nullptr;
+  const int st = gradient_plan_impl(&p, b, shls, refs, nq, fp32_flags, false);
+  if (st != MCINT_OK) return st;
+  mcint_plan_stats(p, stats);
+  plan_free(p);
+  return MCINT_OK;
+}
+
+int mcint::basis_create_host_only(mcint_basis** b, const FINT* atm, FINT natm, const FINT* bas, FINT nbas,
+                                  const double* env) {
+  return basis_create_impl(b, atm, natm, bas, nbas, env, false);
 }
 
 extern "C" int64_t mcint_plan_fp32_tasks(const mcint_plan* p) { return p ? p->stats_fp32 : 0; }

@@ -38,6 +38,15 @@ int plan_build_host_only(const FINT* atm, FINT natm, const FINT* bas, FINT nbas,
 int plan_matrices_host_only(const FINT* atm, FINT natm, const FINT* bas, FINT nbas, const double* env,
                             int intor, const FINT* shls, size_t nq, int64_t* n);
 
+// The host tables of a basis alone (no HIP call), for mcint_gradient_list and
+// the host stage of plans; freed by mcint_basis_destroy.  For tests.
+int basis_create_host_only(mcint_basis** b, const FINT* atm, FINT natm, const FINT* bas, FINT nbas,
+                           const double* env);
+// The host stage of mcint_plan_create_gradient (no HIP call): the statistics
+// of mcint_plan_stats.  For tests.
+int gradient_plan_host_only(mcint_basis* b, const FINT* shls, const FINT* refs, size_t nq,
+                            const uint8_t* fp32_flags, int64_t* stats);
+
 // Sets the calling thread's mcint_last_error() text.
 void set_error(const char* msg);
 
