@@ -131,7 +131,7 @@ def sampled_check(db, B, plan, quart, out, per_bucket=2, seed=7) -> dict:
     gp.close()
     err = np.abs(got - ref)
     return {"quartets": int(idx.size), "buckets": len(plan.buckets()),
-            "reference": "matrix kernel on the same quartets",
+            "reference": "runtime-class kernels (matrix, generic) on the same quartets",
             "max_abs_err": float(err.max()),
             "max_rel_err": float((err / np.maximum(np.abs(ref), 1e-300)).max()),
             "within_1e-12_abs_1e-10_rel": bool(np.all(err <= 1e-12 + 1e-10 * np.abs(ref)))}
@@ -261,8 +261,8 @@ def gradient_section(reps: int = 3) -> dict:
                                                    / (t_plain + t_jk32 + t_grad32),
             "speedup_mixed_vs_fp64_batched": (t_plain + t_jk + t_grad) / (t_plain + t_jk32 + t_grad32),
             "plain_fp64_generic_max_abs_diff_jk_grad": gen_err,
-            "definition": "plain FP64 GPU path = every quartet on the matrix kernel (one "
-                          "workgroup per quartet, runtime class, FP64); batched mixed = class "
+            "definition": "plain FP64 GPU path = every quartet on the runtime-"
+                          "class kernels (matrix, generic; FP64); batched mixed = class "
                           "buckets on the register kernels in concurrent graph branches with "
                           "the FP32 tier for Schwarz x max|D|^2 < 1e-7",
         },

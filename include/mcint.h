@@ -327,12 +327,12 @@ int64_t mcint_noalloc_scratch_doubles(void);
 void mcint_plan_destroy(mcint_plan *p);
 
 /* Plan statistics: n[0] tasks, n[1] buckets, n[2] tasks on fast kernels,
- * n[3] tasks on the generic kernel, n[4] primitive quartets before
+ * n[3] tasks of runtime classes (matrix or generic kernel), n[4] primitive quartets before
  * screening, n[5] output doubles. */
 int mcint_plan_stats(const mcint_plan *p, int64_t *n);
 
 /* Buckets of a plan (one kernel launch each).  info receives: la, lb, lc,
- * ld (canonical class), perm, team lanes, kernel path (0 generic, 1 single
+ * ld (canonical class), perm, team lanes, kernel path (0 runtime class, 1 single
  * register kernel, 2 chunked), task count. */
 int mcint_plan_nbuckets(const mcint_plan *p);
 int mcint_plan_bucket_info(const mcint_plan *p, int bucket, int64_t *info);
@@ -374,7 +374,8 @@ int mcint_plan_create_gradient(mcint_plan **p, mcint_basis *b, const FINT *shls,
  *   vj[p,q] = sum_rs (pq|rs) D[r,s],   vk[p,r] = sum_qs (pq|rs) D[q,s]
  * (overwritten; either nullable).  dm_dev: nao x nao spherical density
  * (row-major, symmetric).  No ERI buffer: device memory is the plan's
- * scratch and two nao x nao matrices.  Plain and long-range operators;
+ * scratch and eight copies of two nao x nao matrices (one copy where eight
+ * exceed 256 MiB).  Plain and long-range operators;
  * mixed-precision plans digest their FP32 blocks too.  Asynchronous on
  * hip_stream.  (The integral-side layer libcint leaves to its callers,
  * PySCF's _vhf.) */

@@ -1002,9 +1002,8 @@ struct Matrices {
 };
 
 // The matrices of the plan's matrix launches, the costliest launch first;
-// one whose pairs no longer fit the bound goes to the generic kernel (2.7
-// times slower: 29.4 against 10.9 ms for the second derivatives of 20
-// shells), and only it.
+// one whose pairs no longer fit the bound goes to the generic kernel (second
+// derivatives of 20 shells 25.1 ms, 10.7 on the matrix kernel), and only it.
 static void admit_matrices(mcint_plan* p, const Task* tasks, Matrices& X) {
   const int kind = p->kind, nv = p->b->nv;
   const int64_t nn = (int64_t)nv * nv, bound = (int64_t)g_matrix_kib * 128;
@@ -1135,8 +1134,7 @@ static int plan_create_impl(mcint_plan** out, mcint_basis* b, int intor, const F
       tuple_class(kind, Q, la, lb, lc, ld, perm);
       const int64_t nprimq = (int64_t)Q.np[0] * Q.np[1] * Q.np[2] * (naxes == 4 ? Q.np[3] : 1);
       nprim_sum += nprimq;
-      // the short-range derivative integrals run on the generic kernel;
-      // everything else has register kernels
+      // the short-range i-derivatives run on the runtime-class kernels
       const int mode =
           reg_ok ? mode_tab[((la * (LMAX + 1) + lb) * (LMAX + 1) + lc) * (LMAX + 1) + ld] : 0;
       const int ppl_c = g_class_ppl[kind][class_index(la, lb, lc, ld)];

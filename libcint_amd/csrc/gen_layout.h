@@ -157,7 +157,8 @@ inline GenLayout gen_layout(int kind, int sph, int la, int lb, int lc, int ld, d
   const int fixed = ntb + ntk + (10 + ncode + ntb + ntk + g.ncb + g.ncd + 4 + 1) / 2;
   // a batch of primitive quartets: enough (primitive, direction, root)
   // recurrences for the lanes, at most 16 KB of tables
-  // (second derivatives of 20 shells: 29.4 ms; 8 KB 31.9 ms, 4 KB 46 ms)
+  // (second derivatives of 20 shells, when this was chosen: 29.4 ms; 8 KB
+  // 31.9 ms, 4 KB 46 ms)
   g.PB = 1;
   while (g.PB < 16 && g.PB * 3 * g.nrt < GEN_LANES && (g.PB + 1) * PV <= 2048) ++g.PB;
   const int walk = g.PB * PV;
@@ -211,7 +212,7 @@ inline GenLayout mm_layout(int kind, int sph, int la, int lb, int lc, int ld, do
   // A batch: two (primitive, direction, root) recurrences per lane, so that
   // its barriers are shared by more primitive quartets, in tables that leave
   // the LDS to several workgroups.  Second derivatives of 20 shells / three-
-  // centre derivatives of 186 shells: 10.9 / 4.95 ms; one recurrence per lane
+  // centre derivatives of 186 shells, when this was chosen: 10.9 / 4.95 ms; one recurrence per lane
   // 11.3 / 5.1; four 10.8 / 5.2; tables of 24 and 16 KB (four waves, one)
   // 11.2 / 4.9, of 32 and 16 KB 10.8 / 5.1.
   const int VT = 3 * g.nrt * (g.E + 1) * (g.F + 1);

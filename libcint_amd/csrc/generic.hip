@@ -1,8 +1,8 @@
 // Generic kernel: any class and kind, one 64-lane workgroup per contracted
 // quartet, class known at run time.  It serves what has neither a register
 // kernel nor a plan's transfer matrices (matrix.hip): single calls on an
-// optimizer's device state, classes whose sums exceed the LDS, plans whose
-// matrices would exceed their bound.
+// optimizer's device state, classes whose sums exceed the LDS or leave a CU too
+// few waves, whose matrices outweigh their walk or exceed the plan's bound.
 //
 // The walk takes 64 candidate primitive quartets at a time (one per lane, in
 // libcint's order and with its tests), compacts the survivors, and for a
@@ -18,7 +18,7 @@
 // What bounds it: latency (waves wait 0.6 of their cycles, VALU issue 0.18,
 // a quarter of it FP64) at the index arithmetic and LDS reads of runtime
 // classes, and few lanes in use for small classes.  Measured on all of
-// int2e_ipip1 + int2e_ip1ip2 of 20 shells: 29.4 ms, 101 ms with the block in
+// int2e_ipip1 + int2e_ip1ip2 of 20 shells: 25.1 ms, 101 ms with the block in
 // global memory, one primitive quartet at a time and binomials and powers
 // recomputed for each transfer term.
 #include <algorithm>

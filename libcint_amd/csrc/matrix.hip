@@ -20,10 +20,9 @@
 // per batch) where tasks hold hundreds of primitive quartets, the set-up per
 // task where they hold one.  Measured against the generic kernel, whose
 // passes go term by term and whose tasks have one wave:
-//   int2e_ipip1 + int2e_ip1ip2 of 20 shells (168 000 quartets): 29.4 -> 10.9 ms
-//   ((pp|pp), 756 tasks of 330 primitive quartets: 4.2 -> 1.1 ms;
-//   (dd|dd), 160 tasks of one: 0.62 -> 0.05 ms)
-//   int3c2e_ip1 + int3c2e_ip2 of 186 shells: 5.53 -> 4.95 ms
+//   int2e_ipip1 + int2e_ip1ip2 of 20 shells (168 000 quartets): 25.1 -> 10.7 ms
+//   int3c2e_ip1 + int3c2e_ip2 of 186 shells: 5.25 -> 4.83 ms
+// Where the generic kernel is the better one: mm_waves (gen_layout.h).
 #include <algorithm>
 
 #include "gen_device.h"

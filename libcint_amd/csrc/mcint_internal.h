@@ -141,7 +141,7 @@ struct BucketArgs {
   // gradient digest (i-derivative plans): instead of storing the block,
   // contract it with the density and add to grad[atom of shell i][x]
   const double* dm;      // nao x nao density, row-major (nullable: store mode)
-  double* grad;          // nslot blocks of grad_stride (= 3 natm) accumulators
+  double* grad;          // nslot copies of the 3 natm accumulators
   int nao;
   // accumulator copies of the gradient and of J', K': block b adds to copy
   // b % nslot, slot_stride doubles apart
